@@ -127,10 +127,19 @@ int max_lds_bytes() {
   return v;
 }
 
+int num_cus() {
+  int dev = 0, v = 0;
+  if (hipGetDevice(&dev) != hipSuccess) return 256;
+  if (hipDeviceGetAttribute(&v, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || v < 1) return 256;
+  return v;
+}
+
 int sampler_launch(int mode, const hipns_launch_t* L, const hipns::SampleArgs& A0, int R, int max_chains, int maxD,
                    int dps, int max_slices, hipStream_t s) {
   int lpc = hipns::sampler_lpc(L->family, L->lanes_per_chain, dps, maxD);
   hipns::SampleArgs A = A0;
+  int waves = L->waves_per_block, groups = L->waves_per_block;
+  bool spread = false;  // regression rows spread over the most wavefronts of few workgroups
   if (L->family == HIPNS_FAM_LINREG) {
     if (L->lr_terms == 5)
       return fail(HIPNS_EINVAL, "lr_terms 5 (the refinement form) is for hipns_log_likelihood; sampling takes 1, 3 or 4");
@@ -144,8 +153,27 @@ int sampler_launch(int mode, const hipns_launch_t* L, const hipns::SampleArgs& A
     A.lr_npad = lr.npad;
     A.lr_panels = lr.panels;
     A.lr_terms = lr.terms;
+    // A launch whose workgroups cannot occupy every CU leaves most of the chip idle while each of its
+    // workgroups walks all data rows: it takes the fewest chain groups per workgroup that still fit one
+    // workgroup per CU, and the most wavefronts to share the rows.  A launch of more workgroups keeps the
+    // requested groups, one per wavefront, so that the workgroups of a CU overlap.  4096 x 16, 16 runs of
+    // 512 chains (64 workgroups of four groups, or 256 of one): 17.9 -> 6.5 us per chain step, 1 382 -> 515
+    // ms per batch; a 65536 x 128 shell of 2048 chains (32 workgroups, or 128): 318 -> 194 ms.
+    const int cw = HIPNS_WAVE / lpc;
+    const int64_t per_run = (max_chains + cw - 1) / cw;
+    for (int g = 1; g <= L->waves_per_block; ++g) {
+      if (R * ((per_run + g - 1) / g) <= num_cus()) {
+        groups = g;
+        waves = hipns::lr_max_waves(hipns::sampler_nj(maxD, lpc));
+        if (waves < g) waves = g;
+        spread = true;
+        break;
+      }
+    }
   }
-  A.alpha_off = (int32_t)hipns::sampler_lds_floats(L->family, dps, maxD, L->gmm_K, lpc, L->waves_per_block);
+  A.lr_groups = groups;
+  A.alpha_off =
+      (int32_t)hipns::sampler_lds_floats(L->family, dps, maxD, L->gmm_K, lpc, groups, L->lr_ndata);
   const size_t base_f = (size_t)A.alpha_off + (size_t)max_slices;
   size_t lds = base_f * sizeof(float);
   if ((int)lds > max_lds_bytes())
@@ -165,6 +193,13 @@ int sampler_launch(int mode, const hipns_launch_t* L, const hipns::SampleArgs& A
     ring = 0;
   }
   A.dir_ring = ring;
+  if (spread) {
+    const size_t off = (lds / sizeof(float) + 3) / 4 * 4, end = (off + (size_t)L->lr_ndata) * sizeof(float);
+    if ((int64_t)end <= max_lds_bytes()) {
+      A.lr_r0_off = (int32_t)off;
+      lds = end;
+    }
+  }
   if (mode == hipns::MODE_GSLICE) {
     // the gradient's scratch at the same offset: [grad_rows][64 / lpc + 1] floats per wavefront
     lds = ((size_t)A.ring_off + (size_t)hipns::grad_rows(nj, lpc) * (HIPNS_WAVE / lpc + 1) * L->waves_per_block) *
@@ -175,6 +210,7 @@ int sampler_launch(int mode, const hipns_launch_t* L, const hipns::SampleArgs& A
   }
   hipns_launch_t L2 = *L;
   L2.lanes_per_chain = lpc;
+  L2.waves_per_block = waves;
   hipError_t e;
   switch (mode) {
     case hipns::MODE_SLICE: e = hipns::launch_sampler_slice(A, R, max_chains, L2, maxD, lds, s); break;
@@ -552,7 +588,8 @@ int hipns_log_likelihood(const float* U_dev, int64_t B, double* logL_dev, const 
   const int D = runs_host[0].D;
   if (D < 1 || D > bufs->dps) return fail(HIPNS_EINVAL, "D outside [1, dps]");
   int lpc = hipns::sampler_lpc(launch->family, launch->lanes_per_chain, bufs->dps, D);
-  size_t lds = hipns::sampler_lds_floats(launch->family, bufs->dps, D, launch->gmm_K, lpc, launch->waves_per_block) *
+  size_t lds = hipns::sampler_lds_floats(launch->family, bufs->dps, D, launch->gmm_K, lpc, launch->waves_per_block,
+                                         launch->lr_ndata) *
                sizeof(float);
   if ((int)lds > max_lds_bytes()) return fail(HIPNS_ERANGE, "parameters exceed LDS");
   hipns_launch_t L2 = *launch;
@@ -583,7 +620,7 @@ int hipns_log_likelihood_grad(const float* U_dev, int64_t B, double* logL_dev, f
   if (D < 1 || D > bufs->dps) return fail(HIPNS_EINVAL, "D outside [1, dps]");
   const int lpc = hipns::sampler_lpc(launch->family, launch->lanes_per_chain, bufs->dps, D);
   const size_t base_f =
-      hipns::sampler_lds_floats(launch->family, bufs->dps, D, launch->gmm_K, lpc, launch->waves_per_block);
+      hipns::sampler_lds_floats(launch->family, bufs->dps, D, launch->gmm_K, lpc, launch->waves_per_block, 0);
   const int gscr_off = (int)((base_f + 3) / 4 * 4);
   const int nj = hipns::sampler_nj(D, lpc);
   const size_t lds =
@@ -614,7 +651,7 @@ int hipns_linreg_stats(const float* U_dev, int64_t B, double* logL_dev, double* 
   if (D < 1 || D > bufs->dps) return fail(HIPNS_EINVAL, "D outside [1, dps]");
   const int lpc = bufs->dps > 64 ? 4 : launch->lanes_per_chain;
   if ((rc = check_panels(launch, D, lpc))) return rc;
-  const size_t lds = hipns::sampler_lds_floats(HIPNS_FAM_LINREG, bufs->dps, D, 1, lpc, 1) * sizeof(float);
+  const size_t lds = hipns::sampler_lds_floats(HIPNS_FAM_LINREG, bufs->dps, D, 1, lpc, 1, launch->lr_ndata, 2) * sizeof(float);
   hipError_t e = hipns::launch_linreg_stats(U_dev, B, logL_dev, rss_dev, yr_dev, runs_dev, *bufs, lpc, D, lds,
                                             as_stream(stream), linreg_view(bufs, launch));
   if (e != hipSuccess) return hip_fail(e, "linreg stats launch");

@@ -31,6 +31,8 @@ struct SampleArgs {
   int32_t lr_npad;
   int32_t lr_panels;
   int32_t lr_terms;
+  int32_t lr_groups;  // chain groups per workgroup (the other wavefronts only take rows)
+  int32_t lr_r0_off;  // LDS float offset of r0 (0: read from global memory)
   int32_t ring_off;   // LDS float offset of the direction rings (16-byte aligned)
   // injected-draw mode
   int32_t inj_buf;
@@ -55,9 +57,11 @@ struct LinRegLds {
   float* s;            // [dps]
   float* w0;           // [dps] centre of the residual GEMM
   double inv2s2;       // 1 / (2 sigma^2), held as FP64 so that logL is smooth in sigma
-  void* bops;          // [G][NG][3][64] B operands (8 bf16 each) published by every wavefront
-  double* partial;     // [2][G][G][CW] per-wavefront partial sums (|r|^2, then y^T r)
+  void* bops;          // [G][NG][3][64] B operands (8 bf16 each) published by every chain group
+  double* partial;     // [2][G][row blocks][CW] partial sums (|r|^2, then y^T r)
   const float* r0;     // [npad] r0 = y - X w0 (computed in FP64, zero on padding rows)
+  float* r0l;          // r0 in LDS where `staged`
+  bool staged;
   const uint16_t* xh;  // [panels][npad][16] bf16 hi part of the column-scaled X
   const uint16_t* xl;  // [panels][npad][16] bf16 lo part (X - hi)
   const float* y;      // [npad] targets (zero on padding rows), read by the adjoint statistics only
@@ -101,12 +105,22 @@ __host__ __device__ constexpr int grad_rows(int nj, int lpc) {
   return ((nj * lpc + 64 / lpc - 1) / (64 / lpc)) * (64 / lpc);
 }
 
-// floats of dynamic LDS one sampler block needs (layout of load_params in ns_sampler_impl.h)
-inline size_t sampler_lds_floats(int fam, int dps, int D, int K, int lpc, int G = 1) {
+// Regression: the most wavefronts of a workgroup (chain groups and row helpers; the instances of more than
+// 8 slots need more than the 256 VGPRs that two wavefronts per SIMD leave each), and the fixed blocks that
+// the data rows are summed in, whatever the number of wavefronts that share them.  A block boundary costs a
+// cross-lane FP64 sum per group, so short data take 8 (one per wavefront of a full workgroup); from 1024
+// tiles on, 32 blocks (16 of the twice as wide ones at 2 lanes per chain: the same LDS) of at least 32
+// tiles.
+__host__ __device__ constexpr int lr_max_waves(int nj) { return nj <= 8 ? 8 : 4; }
+__host__ __device__ inline int lr_row_blocks(int tiles, int lpc) { return tiles < 1024 ? 8 : (lpc == 2 ? 16 : 32); }
+
+// floats of dynamic LDS one sampler block needs (layout of load_params in ns_sampler_impl.h); npad: the
+// regression family's padded data rows, sums: row sums kept per point (2 for the adjoint statistics)
+inline size_t sampler_lds_floats(int fam, int dps, int D, int K, int lpc, int G, int npad, int sums = 1) {
   if (fam == HIPNS_FAM_LINREG) {
     const size_t NG = (size_t)sampler_nj(D, lpc) / 8;
     const size_t CW = (size_t)(64 / lpc);
-    return (size_t)4 * dps + 4 + (size_t)G * NG * 3 * 64 * 4 + (size_t)2 * G * G * CW * 2;
+    return (size_t)4 * dps + 4 + (size_t)G * NG * 3 * 64 * 4 + (size_t)sums * G * lr_row_blocks((int)(npad / CW), lpc) * CW * 2;
   }
   if (fam == HIPNS_FAM_MVN) {
     // W^T holds a (zero) row for every dimension slot of the instance, so the kernel reads all NJ slots

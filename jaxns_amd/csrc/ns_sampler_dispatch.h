@@ -12,8 +12,9 @@ namespace hipns {
 template <int LPC, int NJ, int FAM, int MODE>
 inline hipError_t launch_one(const SampleArgs& A, int R, int max_chains, int wpb, size_t lds_bytes, hipStream_t s) {
   constexpr int CW = HIPNS_WAVE / LPC;
+  const int per_block = FAM == HIPNS_FAM_LINREG ? A.lr_groups : wpb;  // chain groups
   int groups = (max_chains + CW - 1) / CW;
-  int bx = (groups + wpb - 1) / wpb;
+  int bx = (groups + per_block - 1) / per_block;
   if (bx < 1) bx = 1;
   dim3 grid(bx, R), block(wpb * HIPNS_WAVE);
   hipLaunchKernelGGL((k_sample<LPC, NJ, FAM, MODE>), grid, block, lds_bytes, s, A);

@@ -14,6 +14,8 @@
 // nested_samplers/common/uniform_sample.py:12-61 (initial live points),
 // samplers/bases.py:63-74 + internals/random.py:34-84 (seed choice).
 #pragma once
+#include <type_traits>
+
 #include "hipns_dev.h"
 #include "ns_sampler.h"
 
@@ -111,16 +113,18 @@ __device__ __forceinline__ double chain_sum_d(double v) {
 
 // Gaussian linear regression: r = r0 - X (w - w0) with w = p + s (.) q(u); logL = c - |r|^2 / (2 sigma^2).
 // The MFMA chain of a tile starts from C = r0 with the weight operands negated, so it ends on r.
-// The G wavefronts of a workgroup each own one group of CW chains.  Every step they publish the
-// B operands of their chains (w - w0 split into bf16 parts) in LDS, then each wavefront takes 1/G of
-// the data-row tiles and multiplies every row tile it loads against all G groups' operands, so X is
-// read once per step per workgroup instead of once per chain group.  Each product is BF16x3
+// The first G of a workgroup's W wavefronts each own one group of CW chains.  Every step they publish
+// the B operands of their chains (w - w0 split into bf16 parts) in LDS, then each of the W wavefronts
+// takes its share of the data-row tiles and multiplies every row tile it loads against all G groups'
+// operands, so X is read once per step per workgroup instead of once per chain group.  The rows are cut
+// into lr_row_blocks fixed blocks, a wavefront takes whole blocks, and the blocks' sums meet in block
+// order, so a point's value depends on the data alone and not on G, W or the batch.  Each product is BF16x3
 // (hi.hi + hi.lo + lo.hi, FP32 accumulate; terms == 4 adds hi times the third bf16 part of w - w0,
 // which removes the error of the 16-bit weight split that every row shares): LPC=2 uses
 // v_mfma_f32_32x32x16_bf16 over 32-row tiles, LPC=4 v_mfma_f32_16x16x32_bf16 over 16-row tiles.
 // X is stored in 16-column panels ([panel][row][16] bf16) so both layouts read dense rows.  Squares
-// of a tile are summed in FP32 and accumulated in FP64; the G partial sums of a group meet in LDS
-// in a fixed order.  All G wavefronts must call this together (two workgroup barriers).
+// of a tile are summed in FP32 and accumulated in FP64.  All W wavefronts must call this together (two
+// workgroup barriers).
 constexpr int LR_MAX_G = 4;
 
 template <int LPC>
@@ -194,16 +198,21 @@ __device__ __forceinline__ typename LrAcc<LPC>::type lr_mfma(const bf16x8_t& a, 
 
 // The BF16 residual tiles [t0, t1) of one wavefront against the B operands of GG chain groups (GG
 // known at compile time, so the groups' MFMA chains are interleaved and nothing branches per group).
-// The tile loop has wavefront-uniform bounds; at LPC=4 the tiles are double-buffered (the next tile's
-// X panels and r0 load while this one multiplies).  With few (group, k-group) pairs the step's B
-// operands are held in registers for all tiles; otherwise they are read from LDS per tile.
-template <int LPC, int NJ, int GG, bool STATS>
+// The tile loop has wavefront-uniform bounds.  With few (group, k-group) pairs the step's B operands are
+// held in registers for all tiles; otherwise they are read from LDS per tile.  X panels (and r0) of the
+// next tiles load while this one multiplies: one tile ahead at LPC=4; none ahead at LPC=2, where the
+// second buffer (24 VGPRs) would drop the kernel to one wavefront per SIMD, which costs more than the
+// exposed load latency (4096 x 16, 128 runs: 17.1 ms with it, 14.6 without).
+// R0L (r0 staged in LDS): launches of at most one workgroup per CU, where each SIMD holds two
+// wavefronts at most and the latency of a tile's loads (about 3x its arithmetic) is what bounds the
+// loop.  Without r0 a tile is 8 VGPRs per k-group, so four tiles load ahead (two with more k-groups).
+template <int LPC, int NJ, int GG, bool STATS, bool R0L>
 __device__ __forceinline__ void lr_bf16_tiles(const LinRegLds& P, const bf16x8_t* Bs, int t0, int t1, bool t4,
                                               double (&ss)[LR_MAX_G], double (&sy)[LR_MAX_G]) {
   constexpr int CW = HIPNS_WAVE / LPC;
   constexpr int NG = NJ / 8;
   constexpr int NR = (LPC == 2) ? 16 : 4;
-  constexpr bool BREG = LPC == 4 && GG * NG <= 4;
+  constexpr bool BREG = (LPC == 4 || R0L) && GG * NG <= (LPC == 4 ? 4 : 2);
   typedef typename LrAcc<LPC>::type Acc;
   const int l = lane_id();
   const int m = l % CW;
@@ -220,25 +229,28 @@ __device__ __forceinline__ void lr_bf16_tiles(const LinRegLds& P, const bf16x8_t
       }
   }
   auto tile_row = [&](int tl, int i) { return (LPC == 2) ? tl * 32 + 8 * (i >> 2) + 4 * h + (i & 3) : tl * 16 + 4 * h + i; };
-  auto load = [&](int tl, bf16x8_t (&xh)[NG], bf16x8_t (&xl)[NG], float (&rv)[NR]) {
+  auto load = [&](int tl, bf16x8_t (&xh)[NG], bf16x8_t (&xl)[NG]) {
     const int row = tl * CW + m;
 #pragma unroll
     for (int gg = 0; gg < NG; ++gg) {
       xh[gg] = __builtin_bit_cast(bf16x8_t, *(const uint4*)lr_panel_ptr<LPC>(P.xh, P.npad, gg, row, h));
       xl[gg] = __builtin_bit_cast(bf16x8_t, *(const uint4*)lr_panel_ptr<LPC>(P.xl, P.npad, gg, row, h));
     }
-    // the lane's rows of the tile come in aligned runs of four (tile_row): r0 in 16-byte loads
+  };
+  // the lane's rows of the tile come in aligned runs of four (tile_row): r0 in 16-byte loads
+  const float* r0 = R0L ? P.r0l : P.r0;
+  auto load_r0 = [&](int tl, float (&rv)[NR]) {
     if constexpr (LPC == 2) {
 #pragma unroll
       for (int q = 0; q < 4; ++q) {
-        const float4 v = *(const float4*)(P.r0 + tl * 32 + 8 * q + 4 * h);
+        const float4 v = *(const float4*)(r0 + tl * 32 + 8 * q + 4 * h);
         rv[4 * q] = v.x;
         rv[4 * q + 1] = v.y;
         rv[4 * q + 2] = v.z;
         rv[4 * q + 3] = v.w;
       }
     } else {
-      const float4 v = *(const float4*)(P.r0 + tl * 16 + 4 * h);
+      const float4 v = *(const float4*)(r0 + tl * 16 + 4 * h);
       rv[0] = v.x;
       rv[1] = v.y;
       rv[2] = v.z;
@@ -299,25 +311,49 @@ __device__ __forceinline__ void lr_bf16_tiles(const LinRegLds& P, const bf16x8_t
       }
     }
   };
-  bf16x8_t xh0[NG], xl0[NG];
-  float r00[NR];
-  if constexpr (LPC == 4) {
-    // double-buffered: the next tile's X panels and r0 load while this one multiplies
-    bf16x8_t xh1[NG], xl1[NG];
-    float r01[NR];
-    if (t0 < t1) load(t0, xh0, xl0, r00);
+  if constexpr (R0L) {
+    constexpr int DEPTH = NG == 1 ? 4 : 2;
+    bf16x8_t xh[DEPTH][NG], xl[DEPTH][NG];
+#pragma unroll
+    for (int i = 0; i < DEPTH; ++i)
+      if (t0 + i < t1) load(t0 + i, xh[i], xl[i]);
+    for (int tl = t0; tl < t1; tl += DEPTH) {
+#pragma unroll
+      for (int i = 0; i < DEPTH; ++i) {
+        if (tl + i < t1) {
+          float rv[NR];
+          load_r0(tl + i, rv);
+          compute(tl + i, xh[i], xl[i], rv);
+          if (tl + DEPTH + i < t1) load(tl + DEPTH + i, xh[i], xl[i]);
+        }
+      }
+    }
+  } else if constexpr (LPC == 4) {
+    bf16x8_t xh0[NG], xl0[NG], xh1[NG], xl1[NG];
+    float r00[NR], r01[NR];
+    if (t0 < t1) {
+      load(t0, xh0, xl0);
+      load_r0(t0, r00);
+    }
     for (int tl = t0; tl < t1; tl += 2) {
-      if (tl + 1 < t1) load(tl + 1, xh1, xl1, r01);
+      if (tl + 1 < t1) {
+        load(tl + 1, xh1, xl1);
+        load_r0(tl + 1, r01);
+      }
       compute(tl, xh0, xl0, r00);
       if (tl + 1 >= t1) break;
-      if (tl + 2 < t1) load(tl + 2, xh0, xl0, r00);
+      if (tl + 2 < t1) {
+        load(tl + 2, xh0, xl0);
+        load_r0(tl + 2, r00);
+      }
       compute(tl + 1, xh1, xl1, r01);
     }
   } else {
-    // LPC=2: the second buffer (24 VGPRs) would drop the kernel to one wavefront per SIMD, which
-    // costs more than the exposed load latency (4096 x 16, 128 runs: 17.1 ms with it, 14.6 without)
+    bf16x8_t xh0[NG], xl0[NG];
+    float r00[NR];
     for (int tl = t0; tl < t1; ++tl) {
-      load(tl, xh0, xl0, r00);
+      load(tl, xh0, xl0);
+      load_r0(tl, r00);
       compute(tl, xh0, xl0, r00);
     }
   }
@@ -328,7 +364,7 @@ __device__ __forceinline__ void lr_bf16_tiles(const LinRegLds& P, const bf16x8_t
 // (256 VGPRs against 214 at 8 slots and LPC=2), so there terms 5 is rejected by the host.
 template <int LPC, int NJ, bool STATS = false, bool F64T = false>
 __device__ __forceinline__ double lik_linreg(const float (&up)[NJ], int nj, int D, const LinRegLds& P, uint32_t tfm,
-                                             int g, int G, double log_const, double* rss = nullptr,
+                                             int g, int G, int W, double log_const, double* rss = nullptr,
                                              double* yr = nullptr) {
   constexpr int CW = HIPNS_WAVE / LPC;
   constexpr int NG = NJ / 8;  // k-groups of 8 owned dims
@@ -337,163 +373,177 @@ __device__ __forceinline__ double lik_linreg(const float (&up)[NJ], int nj, int 
   const int h = l / CW;
   const bool t4 = P.terms == 4;
   const bool fp32 = P.terms == 1 || (F64T && P.terms == 5);
-  float dwv[NJ], qv[NJ];
-  if (F64T && P.terms == 5) {
-    // refinement: w - w0 from the FP64 transform and FP64 parameters, rounded once to FP32 (the FP32
-    // ndtri's ~1e-7 relative error would otherwise shift w by far more than the posterior width of
-    // strongly determined weights)
-    const double* p64 = P.f64;
-    const double* s64 = P.f64 + P.dps;
-    const double* w64 = P.f64 + 2 * P.dps;
-#pragma unroll
-    for (int j = 0; j < NJ; ++j) {
-      const int d = owned_dim<LPC>(h, j);
-      float dw = 0.0f;
-      if (j < nj && d < D) {
-        const double u = (double)up[j];
-        const double q = ((tfm >> j) & 1u) ? ndtri_f64(u) : u;
-        dw = (float)(fma(s64[d], q, p64[d]) - w64[d]);
-      }
-      dwv[j] = dw;
-    }
-  } else {
-    prior_q<NJ>(up, qv, tfm);
-#pragma unroll
-    for (int j = 0; j < NJ; ++j) {
-      const int d = owned_dim<LPC>(h, j);
-      float dw = 0.0f;
-      if (j < nj && d < D) dw = fmaf(P.s[d], qv[j], P.p[d]) - P.w0[d];
-      dwv[j] = dw;
-    }
-  }
-  // publish this wavefront's B operands, negated so that the MFMA chain started from C = r0 yields
-  // r = r0 - X (w - w0): BF16 forms [G][NG][3][64] vectors of 8 bf16, plain FP32 [G][NJ][64] floats
   bf16x8_t* Bs = (bf16x8_t*)P.bops;
   float* Bf = (float*)P.bops;
-  if (fp32) {
+  if (g < G) {
+    float dwv[NJ], qv[NJ];
+    if (F64T && P.terms == 5) {
+      // refinement: w - w0 from the FP64 transform and FP64 parameters, rounded once to FP32 (the FP32
+      // ndtri's ~1e-7 relative error would otherwise shift w by far more than the posterior width of
+      // strongly determined weights)
+      const double* p64 = P.f64;
+      const double* s64 = P.f64 + P.dps;
+      const double* w64 = P.f64 + 2 * P.dps;
 #pragma unroll
-    for (int j = 0; j < NJ; ++j) Bf[(g * NJ + j) * HIPNS_WAVE + l] = -dwv[j];
-  } else {
-#pragma unroll
-    for (int gg = 0; gg < NG; ++gg) {
-      bf16x8_t bh, bl, bt;
-#pragma unroll
-      for (int i = 0; i < 8; ++i) {
-        const float dw = dwv[gg * 8 + i];
-        const __bf16 hi = (__bf16)dw;
-        const float rem = dw - (float)hi;
-        const __bf16 lo = (__bf16)rem;
-        bh[i] = -hi;
-        bl[i] = -lo;
-        bt[i] = -(__bf16)(rem - (float)lo);
+      for (int j = 0; j < NJ; ++j) {
+        const int d = owned_dim<LPC>(h, j);
+        float dw = 0.0f;
+        if (j < nj && d < D) {
+          const double u = (double)up[j];
+          const double q = ((tfm >> j) & 1u) ? ndtri_f64(u) : u;
+          dw = (float)(fma(s64[d], q, p64[d]) - w64[d]);
+        }
+        dwv[j] = dw;
       }
-      Bs[((g * NG + gg) * 3 + 0) * HIPNS_WAVE + l] = bh;
-      Bs[((g * NG + gg) * 3 + 1) * HIPNS_WAVE + l] = bl;
-      Bs[((g * NG + gg) * 3 + 2) * HIPNS_WAVE + l] = bt;
+    } else {
+      prior_q<NJ>(up, qv, tfm);
+#pragma unroll
+      for (int j = 0; j < NJ; ++j) {
+        const int d = owned_dim<LPC>(h, j);
+        float dw = 0.0f;
+        if (j < nj && d < D) dw = fmaf(P.s[d], qv[j], P.p[d]) - P.w0[d];
+        dwv[j] = dw;
+      }
+    }
+    // publish this wavefront's B operands, negated so that the MFMA chain started from C = r0 yields
+    // r = r0 - X (w - w0): BF16 forms [G][NG][3][64] vectors of 8 bf16, plain FP32 [G][NJ][64] floats
+    if (fp32) {
+#pragma unroll
+      for (int j = 0; j < NJ; ++j) Bf[(g * NJ + j) * HIPNS_WAVE + l] = -dwv[j];
+    } else {
+#pragma unroll
+      for (int gg = 0; gg < NG; ++gg) {
+        bf16x8_t bh, bl, bt;
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+          const float dw = dwv[gg * 8 + i];
+          const __bf16 hi = (__bf16)dw;
+          const float rem = dw - (float)hi;
+          const __bf16 lo = (__bf16)rem;
+          bh[i] = -hi;
+          bl[i] = -lo;
+          bt[i] = -(__bf16)(rem - (float)lo);
+        }
+        Bs[((g * NG + gg) * 3 + 0) * HIPNS_WAVE + l] = bh;
+        Bs[((g * NG + gg) * 3 + 1) * HIPNS_WAVE + l] = bl;
+        Bs[((g * NG + gg) * 3 + 2) * HIPNS_WAVE + l] = bt;
+      }
     }
   }
   __syncthreads();
   const int tiles = P.npad / CW;
-  const int t0 = (int)(((long long)tiles * g) / G), t1 = (int)(((long long)tiles * (g + 1)) / G);
-  double ss[LR_MAX_G], sy[LR_MAX_G];
-#pragma unroll
-  for (int q = 0; q < LR_MAX_G; ++q) {
-    ss[q] = 0.0;
-    sy[q] = 0.0;
-  }
+  const int NB = lr_row_blocks(tiles, LPC);
   constexpr int NR = (LPC == 2) ? 16 : 4;  // accumulator rows per lane
   // rows of tile tl held by this lane (the MFMA output layout)
   auto tile_row = [&](int tl, int i) { return (LPC == 2) ? tl * 32 + 8 * (i >> 2) + 4 * h + (i & 3) : tl * 16 + 4 * h + i; };
-  if (fp32) {
-    // plain FP32 form: v_mfma_f32_32x32x2_f32 (LPC=2) / v_mfma_f32_16x16x4_f32 (LPC=4), one MFMA per
-    // owned dimension slot, X read in FP32 from its own panels
-    for (int tl = t0; tl < t1; ++tl) {
-      const int row = tl * CW + m;
-      float xa[NJ];
+  // this wavefront's row blocks, each summed by itself (wavefront-uniform ranges: scalar loop control)
+  const int b0 = __builtin_amdgcn_readfirstlane(NB * g / W), b1 = __builtin_amdgcn_readfirstlane(NB * (g + 1) / W);
+  for (int blk = b0; blk < b1; ++blk) {
+    const int t0 = (int)(((long long)tiles * blk) / NB), t1 = (int)(((long long)tiles * (blk + 1)) / NB);
+    double ss[LR_MAX_G], sy[LR_MAX_G];
 #pragma unroll
-      for (int gg = 0; gg < NG; ++gg) {
-        const float* xp = (LPC == 2) ? P.xf + ((int64_t)gg * P.npad + row) * 16 + 8 * h
-                                     : P.xf + ((int64_t)(2 * gg + (h >> 1)) * P.npad + row) * 16 + 8 * (h & 1);
-        const float4 v0 = *(const float4*)xp, v1 = *(const float4*)(xp + 4);
-        xa[gg * 8 + 0] = v0.x;
-        xa[gg * 8 + 1] = v0.y;
-        xa[gg * 8 + 2] = v0.z;
-        xa[gg * 8 + 3] = v0.w;
-        xa[gg * 8 + 4] = v1.x;
-        xa[gg * 8 + 5] = v1.y;
-        xa[gg * 8 + 6] = v1.z;
-        xa[gg * 8 + 7] = v1.w;
-      }
-      float rv[NR], yv[NR];
+    for (int q = 0; q < LR_MAX_G; ++q) {
+      ss[q] = 0.0;
+      sy[q] = 0.0;
+    }
+    if (fp32) {
+      // plain FP32 form: v_mfma_f32_32x32x2_f32 (LPC=2) / v_mfma_f32_16x16x4_f32 (LPC=4), one MFMA per
+      // owned dimension slot, X read in FP32 from its own panels
+      for (int tl = t0; tl < t1; ++tl) {
+        const int row = tl * CW + m;
+        float xa[NJ];
 #pragma unroll
-      for (int i = 0; i < NR; ++i) {
-        rv[i] = P.r0[tile_row(tl, i)];
-        if (STATS) yv[i] = P.y[tile_row(tl, i)];
-      }
+        for (int gg = 0; gg < NG; ++gg) {
+          const float* xp = (LPC == 2) ? P.xf + ((int64_t)gg * P.npad + row) * 16 + 8 * h
+                                       : P.xf + ((int64_t)(2 * gg + (h >> 1)) * P.npad + row) * 16 + 8 * (h & 1);
+          const float4 v0 = *(const float4*)xp, v1 = *(const float4*)(xp + 4);
+          xa[gg * 8 + 0] = v0.x;
+          xa[gg * 8 + 1] = v0.y;
+          xa[gg * 8 + 2] = v0.z;
+          xa[gg * 8 + 3] = v0.w;
+          xa[gg * 8 + 4] = v1.x;
+          xa[gg * 8 + 5] = v1.y;
+          xa[gg * 8 + 6] = v1.z;
+          xa[gg * 8 + 7] = v1.w;
+        }
+        float rv[NR], yv[NR];
 #pragma unroll
-      for (int q = 0; q < LR_MAX_G; ++q) {
-        if (q < G) {
-          const float* B = Bf + q * NJ * HIPNS_WAVE + l;
-          float part = 0.0f, ypart = 0.0f;
-          if constexpr (LPC == 2) {
-            f32x16 acc;
+        for (int i = 0; i < NR; ++i) {
+          rv[i] = P.r0[tile_row(tl, i)];
+          if (STATS) yv[i] = P.y[tile_row(tl, i)];
+        }
 #pragma unroll
-            for (int i = 0; i < 16; ++i) acc[i] = rv[i];
+        for (int q = 0; q < LR_MAX_G; ++q) {
+          if (q < G) {
+            const float* B = Bf + q * NJ * HIPNS_WAVE + l;
+            float part = 0.0f, ypart = 0.0f;
+            if constexpr (LPC == 2) {
+              f32x16 acc;
 #pragma unroll
-            for (int j = 0; j < NJ; ++j)
-              acc = __builtin_amdgcn_mfma_f32_32x32x2f32(xa[j], B[j * HIPNS_WAVE], acc, 0, 0, 0);
+              for (int i = 0; i < 16; ++i) acc[i] = rv[i];
 #pragma unroll
-            for (int i = 0; i < 16; ++i) {
-              part = fmaf(acc[i], acc[i], part);
-              if (STATS) ypart = fmaf(yv[i], acc[i], ypart);
+              for (int j = 0; j < NJ; ++j)
+                acc = __builtin_amdgcn_mfma_f32_32x32x2f32(xa[j], B[j * HIPNS_WAVE], acc, 0, 0, 0);
+#pragma unroll
+              for (int i = 0; i < 16; ++i) {
+                part = fmaf(acc[i], acc[i], part);
+                if (STATS) ypart = fmaf(yv[i], acc[i], ypart);
+              }
+            } else {
+              f32x4 acc;
+#pragma unroll
+              for (int i = 0; i < 4; ++i) acc[i] = rv[i];
+#pragma unroll
+              for (int j = 0; j < NJ; ++j)
+                acc = __builtin_amdgcn_mfma_f32_16x16x4f32(xa[j], B[j * HIPNS_WAVE], acc, 0, 0, 0);
+#pragma unroll
+              for (int i = 0; i < 4; ++i) {
+                part = fmaf(acc[i], acc[i], part);
+                if (STATS) ypart = fmaf(yv[i], acc[i], ypart);
+              }
             }
-          } else {
-            f32x4 acc;
-#pragma unroll
-            for (int i = 0; i < 4; ++i) acc[i] = rv[i];
-#pragma unroll
-            for (int j = 0; j < NJ; ++j)
-              acc = __builtin_amdgcn_mfma_f32_16x16x4f32(xa[j], B[j * HIPNS_WAVE], acc, 0, 0, 0);
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-              part = fmaf(acc[i], acc[i], part);
-              if (STATS) ypart = fmaf(yv[i], acc[i], ypart);
-            }
+            ss[q] += (double)part;
+            if (STATS) sy[q] += (double)ypart;
           }
-          ss[q] += (double)part;
-          if (STATS) sy[q] += (double)ypart;
         }
       }
+    } else {
+      auto run_tiles = [&](auto staged) {
+        constexpr bool R0L = decltype(staged)::value;
+        if (G == 1)
+          lr_bf16_tiles<LPC, NJ, 1, STATS, R0L>(P, Bs, t0, t1, t4, ss, sy);
+        else if (G == 2)
+          lr_bf16_tiles<LPC, NJ, 2, STATS, R0L>(P, Bs, t0, t1, t4, ss, sy);
+        else if (G == 4)
+          lr_bf16_tiles<LPC, NJ, 4, STATS, R0L>(P, Bs, t0, t1, t4, ss, sy);
+        else
+          lr_bf16_tiles<LPC, NJ, 3, STATS, R0L>(P, Bs, t0, t1, t4, ss, sy);
+      };
+      if (!STATS && !F64T && P.staged)
+        run_tiles(std::integral_constant<bool, !STATS && !F64T>());
+      else
+        run_tiles(std::false_type());
     }
-  } else {
-    // wavefront-uniform tile range (scalar loop control)
-    const int u0 = __builtin_amdgcn_readfirstlane(t0), u1 = __builtin_amdgcn_readfirstlane(t1);
-    if (G == 4)
-      lr_bf16_tiles<LPC, NJ, 4, STATS>(P, Bs, u0, u1, t4, ss, sy);
-    else if (G == 2)
-      lr_bf16_tiles<LPC, NJ, 2, STATS>(P, Bs, u0, u1, t4, ss, sy);
-    else if (G == 1)
-      lr_bf16_tiles<LPC, NJ, 1, STATS>(P, Bs, u0, u1, t4, ss, sy);
-    else
-      lr_bf16_tiles<LPC, NJ, 3, STATS>(P, Bs, u0, u1, t4, ss, sy);
-  }
-  // partial sums of every group from this wavefront's rows -> LDS [group][wavefront][chain]
+    // partial sums of every group from this row block -> LDS [group][row block][chain]
 #pragma unroll
-  for (int q = 0; q < LR_MAX_G; ++q) {
-    if (q < G) {
-      const double v = chain_sum_d<LPC>(ss[q]);
-      const double vy = STATS ? chain_sum_d<LPC>(sy[q]) : 0.0;
-      if (h == 0) {
-        P.partial[(q * G + g) * CW + m] = v;
-        if (STATS) P.partial[(G * G + q * G + g) * CW + m] = vy;
+    for (int q = 0; q < LR_MAX_G; ++q) {
+      if (q < G) {
+        const double v = chain_sum_d<LPC>(ss[q]);
+        const double vy = STATS ? chain_sum_d<LPC>(sy[q]) : 0.0;
+        if (h == 0) {
+          P.partial[(q * NB + blk) * CW + m] = v;
+          if (STATS) P.partial[((G + q) * NB + blk) * CW + m] = vy;
+        }
       }
     }
   }
   __syncthreads();
   double tot = 0.0, toty = 0.0;
-  for (int k = 0; k < G; ++k) {
-    tot += P.partial[(g * G + k) * CW + m];
-    if (STATS) toty += P.partial[(G * G + g * G + k) * CW + m];
+  if (g < G) {
+    for (int k = 0; k < NB; ++k) {
+      tot += P.partial[(g * NB + k) * CW + m];
+      if (STATS) toty += P.partial[((G + g) * NB + k) * CW + m];
+    }
   }
   if constexpr (STATS) {
     *rss = tot;
@@ -966,7 +1016,7 @@ __device__ __forceinline__ void uniform_point(float (&up)[NJ], int chain, uint32
 }
 
 template <int LPC, int NJ, int FAM, int MODE>
-__global__ void __launch_bounds__(256) k_sample(SampleArgs A) {
+__global__ void __launch_bounds__(FAM == HIPNS_FAM_LINREG ? HIPNS_WAVE * lr_max_waves(NJ) : 256) k_sample(SampleArgs A) {
   constexpr int CW = HIPNS_WAVE / LPC;
   // the regression family multiplies the data rows against every chain group of the workgroup
   // cooperatively, so its wavefronts step together (workgroup-uniform loop)
@@ -989,13 +1039,15 @@ __global__ void __launch_bounds__(256) k_sample(SampleArgs A) {
   if (MODE != MODE_INJ && st->done) return;  // uniform across the block
   const int wpb = blockDim.x / HIPNS_WAVE;
   const int wave = threadIdx.x / HIPNS_WAVE;
-  const int G = COOP ? wpb : 1;
+  // chain groups of the workgroup; the regression family's further wavefronts take a share of the rows only
+  const int G = COOP ? A.lr_groups : wpb;
+  const bool chain_wave = !COOP || wave < G;
   const int l = lane_id();
   const int c = l % CW;
   const int h = l / CW;
   const int nchains = (MODE == MODE_INIT) ? run.N : ((MODE == MODE_INJ) ? A.inj_C : run.shell);
-  const int chain0 = (blockIdx.x * wpb + wave) * CW;
-  if (blockIdx.x * wpb * CW >= nchains) return;  // whole block idle
+  const int chain0 = (blockIdx.x * G + wave) * CW;
+  if (blockIdx.x * G * CW >= nchains) return;  // whole block idle
   const int dps = A.B.dps;
   const int D = run.D;
   const int DPr = ((D + 8 * LPC - 1) / (8 * LPC)) * (8 * LPC);
@@ -1004,9 +1056,15 @@ __global__ void __launch_bounds__(256) k_sample(SampleArgs A) {
   MvnLds mv;
   GmmLds gm;
   LinRegLds lr;
-  load_params(FAM, A.B.params + run.param_off, dps, D, A.gmm_K, lds, mv, gm, LPC, &lr, G, NJ / 8);
+  load_params(FAM, A.B.params + run.param_off, dps, D, A.gmm_K, lds, mv, gm, LPC, &lr, COOP ? G : 1, NJ / 8);
   if (COOP) {
     lr.r0 = A.lr_r0;
+    lr.r0l = lds + A.lr_r0_off;
+    lr.staged = A.lr_r0_off > 0;
+    if (lr.staged) {
+      // in place before the first step's barriers
+      for (int i = threadIdx.x; i < A.lr_npad; i += blockDim.x) lr.r0l[i] = A.lr_r0[i];
+    }
     lr.xh = A.lr_xh;
     lr.xl = A.lr_xl;
     lr.xf = A.lr_xf;
@@ -1018,7 +1076,7 @@ __global__ void __launch_bounds__(256) k_sample(SampleArgs A) {
   const uint32_t tfm = transform_mask<LPC, NJ>(FAM == HIPNS_FAM_MVN ? mv.tf : gm.tf, h, nj);
 
   const int chain = chain0 + c;
-  bool alive = chain < nchains;
+  bool alive = chain_wave && chain < nchains;
   const int64_t iter = (MODE == MODE_INIT) ? 0xFFFFFFFFll : ((MODE == MODE_INJ) ? 0 : st->iteration);
   const uint32_t k0 = run.seed_lo, k1 = run.seed_hi;
   const uint32_t it32 = (uint32_t)iter;
@@ -1141,7 +1199,7 @@ __global__ void __launch_bounds__(256) k_sample(SampleArgs A) {
   // word to the others.
   for (int w = 0; COOP ? __syncthreads_or(alive) : __any(alive); ++w) {
     uint32_t pickw = 0u;
-    if (DRAWN) {
+    if (DRAWN && chain_wave) {
       if ((w & (4 * LPC - 1)) == 0)
         pickblk = philox4x32((uint32_t)chain, it32, (uint32_t)((w >> 2) + h), RNG_PICK, k0, k1);
       const int kw = w & 3;
@@ -1204,7 +1262,7 @@ __global__ void __launch_bounds__(256) k_sample(SampleArgs A) {
     } else if constexpr (FAM == HIPNS_FAM_GMM) {
       L = lik_gmm<LPC, NJ>(up, nj, D, gm, tfm);
     } else {
-      L = lik_linreg<LPC, NJ>(up, nj, D, lr, tfm, wave, G, run.log_const);
+      L = lik_linreg<LPC, NJ>(up, nj, D, lr, tfm, wave, G, wpb, run.log_const);
     }
 
     if (alive) {

@@ -40,7 +40,7 @@ __global__ void __launch_bounds__(256) k_loglik(const float* U, int64_t B, doubl
   else if constexpr (FAM == HIPNS_FAM_GMM)
     L = lik_gmm<LPC, NJ>(up, nj, D, gm, tfm);
   else
-    L = lik_linreg<LPC, NJ, false, true>(up, nj, D, lr, tfm, wave, wpb, run.log_const);
+    L = lik_linreg<LPC, NJ, false, true>(up, nj, D, lr, tfm, wave, wpb, wpb, run.log_const);
   if (ok && h == 0) out[row] = L;
 }
 
@@ -182,7 +182,7 @@ __global__ void __launch_bounds__(64) k_linreg_stats(const float* U, int64_t B, 
   }
   const uint32_t tfm = transform_mask<LPC, NJ>(lr.tf, h, nj);
   double ss = 0.0, sy = 0.0;
-  const double L = lik_linreg<LPC, NJ, true>(up, nj, D, lr, tfm, 0, 1, run.log_const, &ss, &sy);
+  const double L = lik_linreg<LPC, NJ, true>(up, nj, D, lr, tfm, 0, 1, 1, run.log_const, &ss, &sy);
   if (ok && h == 0) {
     logL[row] = L;
     rss[row] = ss;

@@ -801,3 +801,27 @@ def test_linreg_precision_at_scale():
             f"(mean logL {ref64[Q].mean():.4g}); against the device's FP32 q prior {prod[P].max():.2e} "
             f"posterior {prod[Q].max():.2e}")
         assert tot[P].max() < tol_prior and tot[Q].max() < tol_post
+
+
+@pytest.mark.parametrize("rows,D,lpc", [(37, 5, 2), (4096, 16, 2), (300, 40, 4), (33000, 9, 2), (16500, 20, 4)])
+def test_regression_runs_do_not_depend_on_row_split(rows, D, lpc):
+    """A small launch shares the data rows among more wavefronts and fewer chain groups per workgroup than a
+    full one (300 runs: more workgroups than compute units).  Every point's value is summed in the same row
+    blocks either way, so a run's shells are the same bit for bit alone, among 8 runs and among 300."""
+    from jaxns_amd.engine import DeviceBatch, RunSpec
+    say(f"regression row split {rows}x{D} lpc={lpc}")
+    model, _, _ = linreg_problem(rows, D, seed=rows, sigma=0.4, tau=1.0)
+
+    def shells(R, wpb):
+        specs = [RunSpec(model=model, num_live_points=70, num_slices=D, max_samples=700, seed=s) for s in range(R)]
+        b = DeviceBatch(specs, lanes_per_chain=lpc, waves_per_block=wpb)
+        b.init_state()
+        for _ in range(3):
+            b.collect_shell(dict(max_samples=700.0))
+        st = b.states()[0]
+        return [x[:70].cpu().numpy() for x in (b.live_U[st.buf], b.live_logL[st.buf], b.live_evals[st.buf])]
+
+    ref = shells(300, 1)
+    for R, wpb in ((1, 1), (1, 4), (8, 2)):
+        for x, y in zip(ref, shells(R, wpb)):
+            assert np.array_equal(x, y), (R, wpb)
