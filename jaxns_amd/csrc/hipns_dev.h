@@ -309,62 +309,177 @@ __device__ __forceinline__ float ndtri_f32(float u) {
 }
 
 // ---------------------------------------------------------------------------
-// FP64 log-space arithmetic.  lae(a, b) = log(e^a + e^b) with the jnp.logaddexp
-// convention for equal infinities (returns a + b).
+// Non-negative FP64 numbers of any magnitude: m 2^e, the exponent a whole-valued double.  The evidence
+// recurrence multiplies and adds quantities far outside the range of a double (likelihoods of e^-1e10,
+// volumes of e^-1000).  Held as logarithms every sum is an exp and a log1p (about 75 FP64 instructions);
+// held like this it is two shifts and an add.
+// Zero has exponent -inf (so it never sets the scale of a sum); +inf and NaN live in m.
 // ---------------------------------------------------------------------------
-__device__ __forceinline__ double lae(double a, double b) {
-  double m = fmax(a, b);
-  double d = a - b;
-  if (__builtin_isnan(d)) return a + b;
-  return m + log1p(exp(-fabs(d)));
+struct Sc {
+  double m, e;
+};
+
+__device__ __forceinline__ Sc sc_zero() { return {0.0, -__builtin_inf()}; }
+
+__device__ __forceinline__ Sc sc_mul(const Sc& x, const Sc& y) { return {x.m * y.m, x.e + y.e}; }
+__device__ __forceinline__ Sc sc_scale(const Sc& x, double c) { return {x.m * c, x.e}; }
+
+// both mantissas shifted to the larger exponent (the conversion saturates, and a shift that far is zero;
+// two zeros have a NaN difference, which converts to 0)
+__device__ __forceinline__ Sc sc_add(const Sc& x, const Sc& y) {
+#pragma clang fp contract(off)
+  const double e = fmax(x.e, y.e);
+  return {__builtin_amdgcn_ldexp(x.m, (int)(x.e - e)) + __builtin_amdgcn_ldexp(y.m, (int)(y.e - e)), e};
+}
+
+// m in [1/2, 1)
+__device__ __forceinline__ Sc sc_norm(const Sc& x) {
+  return {__builtin_amdgcn_frexp_mant(x.m), x.e + (double)__builtin_amdgcn_frexp_exp(x.m)};
+}
+
+// e^L.  L = k ln 2 + r with k whole and |r| <= ln(2) / 2, e^r by its Taylor series (the first term left out
+// is below 2^-53).  Beyond 2^52 a double no longer separates L from its neighbours by less than one, and r
+// only has to stay bounded.
+__device__ __forceinline__ Sc sc_exp(double L) {
+  constexpr double LOG2E = 1.4426950408889634074, LN2_HI = 0.69314718055994530942, LN2_LO = 2.3190468138462996e-17;
+  const double k = rint(L * LOG2E);
+  double r = fma(-k, LN2_LO, fma(-k, LN2_HI, L));
+  r = fmin(fmax(r, -0.35), 0.35);
+  double p = 1.0 / 6227020800.0;
+  p = fma(p, r, 1.0 / 479001600.0);
+  p = fma(p, r, 1.0 / 39916800.0);
+  p = fma(p, r, 1.0 / 3628800.0);
+  p = fma(p, r, 1.0 / 362880.0);
+  p = fma(p, r, 1.0 / 40320.0);
+  p = fma(p, r, 1.0 / 5040.0);
+  p = fma(p, r, 1.0 / 720.0);
+  p = fma(p, r, 1.0 / 120.0);
+  p = fma(p, r, 1.0 / 24.0);
+  p = fma(p, r, 1.0 / 6.0);
+  p = fma(p, r, 0.5);
+  p = fma(p, r, 1.0);
+  p = fma(p, r, 1.0);
+  // -inf, +inf and NaN
+  if (!(fabs(L) < __builtin_inf())) return L < 0.0 ? sc_zero() : Sc{L, 0.0};
+  return {p, k};
+}
+
+// ln(m 2^e) = ln f + k ln 2 with f in [sqrt(1/2), sqrt(2)), ln f = 2 artanh((f - 1) / (f + 1)) by its power
+// series (|s| < 0.172: the first term left out is below 2^-54 of the sum).  About two thirds of the
+// instructions of the library's log; m is never negative here.
+__device__ __forceinline__ double sc_log(const Sc& x) {
+  const double f0 = __builtin_amdgcn_frexp_mant(x.m);
+  const bool low = f0 < 0.70710678118654752440;
+  const double f = low ? f0 + f0 : f0;
+  const double k = x.e + (double)(__builtin_amdgcn_frexp_exp(x.m) - (low ? 1 : 0));
+  const double num = f - 1.0, den = f + 1.0;
+  double y = __builtin_amdgcn_rcp(den);
+  y = fma(fma(-den, y, 1.0), y, y);
+  y = fma(fma(-den, y, 1.0), y, y);
+  double s = num * y;
+  s = fma(fma(-den, s, num), y, s);
+  const double t = s * s;
+  double p = 2.0 / 21.0;
+  p = fma(p, t, 2.0 / 19.0);
+  p = fma(p, t, 2.0 / 17.0);
+  p = fma(p, t, 2.0 / 15.0);
+  p = fma(p, t, 2.0 / 13.0);
+  p = fma(p, t, 2.0 / 11.0);
+  p = fma(p, t, 2.0 / 9.0);
+  p = fma(p, t, 2.0 / 7.0);
+  p = fma(p, t, 2.0 / 5.0);
+  p = fma(p, t, 2.0 / 3.0);
+  const double lf = fma(s * t, p, s + s);
+  // (zero has k = -inf)
+  return x.m == __builtin_inf() ? x.m : fma(k, 0.69314718055994530942, lf);
+}
+
+// The same with an unevaluated low part, for the long products of the recurrence: X is a product of up to
+// millions of n / (n + 1), and the rounding of a factor that repeats would add up.
+struct Scd {
+  double m, lo, e;
+};
+
+__device__ __forceinline__ Scd scd_zero() { return {0.0, 0.0, -__builtin_inf()}; }
+__device__ __forceinline__ Sc sc_of(const Scd& x) { return {x.m, x.e}; }
+
+// x (t + tl), mantissa not renormalised
+__device__ __forceinline__ Scd scd_scale(const Scd& x, double t, double tl) {
+#pragma clang fp contract(off)
+  const double p = x.m * t;
+  return {p, fma(x.m, t, -p) + fma(x.m, tl, x.lo * t), x.e};
+}
+// low part below half an ulp of the high part, m in [1/2, 1)
+__device__ __forceinline__ Scd scd_norm(const Scd& x) {
+#pragma clang fp contract(off)
+  const double s = x.m + x.lo;
+  const double lo = x.lo - (s - x.m);
+  const int k = __builtin_amdgcn_frexp_exp(s);
+  return {__builtin_amdgcn_frexp_mant(s), __builtin_amdgcn_ldexp(lo, -k), x.e + (double)k};
+}
+__device__ __forceinline__ Scd scd_mul(const Scd& x, const Scd& y) {
+  Scd r = scd_scale(x, y.m, y.lo);
+  r.e += y.e;
+  return scd_norm(r);
 }
 
 // ---------------------------------------------------------------------------
 // Evidence recurrence as composable maps.
 //
 // One _update_evidence_calc_op step (internals/shrinkage_statistics.py:43-94)
-// acts on S = (X, X2, Z, ZX, Z2, dZ2) (all >= 0, kept as logs) linearly:
+// acts on (X, X2, Z, ZX, Z2, dZ2) (all >= 0) as
 //   X'  = T X                 X2' = T2 X2
 //   Z'  = Z  + (t m) X        ZX' = T ZX + (tT m) X2
 //   Z2' = Z2 + (2 t m) ZX + (t2 m^2) X2
 //   dZ2'= dZ2 + (t2 m^2) X2
 // with T=n/(n+1), t=1/(n+1), T2=n/(n+2), t2=2/((n+1)(n+2)), tT=n/((n+1)(n+2)),
-// m = (L_prev + L)/2.  Maps of the form
-//   X'=aX, X2'=bX2, Z'=Z+gX, ZX'=aZX+eX2, Z2'=Z2+zZX+hX2, dZ2'=dZ2+thX2
-// are closed under composition, so the scan over samples is a prefix scan
-// of 7-coefficient maps in log space.
+// m = (L_prev + L)/2.  With Q = X2 / X and Y = ZX / X, w = t m X (the step's dZ) and
+// y = m Q / (n+2) it is
+//   X' = T X,  Q' = (n+1)/(n+2) Q,  Z' = Z + w,  Y' = Y + y,  Z2' = Z2 + 2 w Y',  dZ2' = dZ2 + 2 w y:
+// two products and four sums, and nothing decays but X and Q.  A sequence of steps is a map
+//   X'=aX, Q'=bQ, Z'=Z+gX, Y'=Y+cQ, Z2'=Z2+2gXY+hXQ, dZ2'=dZ2+kXQ,
+// closed under composition, so the scan over samples is a prefix scan of 6-coefficient maps.  The
+// coefficients of a map are also the state that it takes (1, 1, 0, 0, 0, 0) to, so a sequence of steps
+// composes by stepping that state.
 // ---------------------------------------------------------------------------
-struct EvMap {
-  double a, b, g, e, z, h, th;
-};
-
 struct EvState {
-  double L, X, X2, Z, ZX, Z2, dZ, dZ2;
+  Scd X, Q;
+  Sc Z, Y, Z2, dZ2;
+};
+struct EvMap {
+  Scd a, b;
+  Sc g, c, h, k;
 };
 
 __device__ __forceinline__ EvMap evmap_identity() {
-  const double ninf = -__builtin_inf();
-  return {0.0, 0.0, ninf, ninf, ninf, ninf, ninf};
+  return {{1.0, 0.0, 0.0}, {1.0, 0.0, 0.0}, sc_zero(), sc_zero(), sc_zero(), sc_zero()};
+}
+__device__ __forceinline__ EvState evstate_initial() {
+  return {{1.0, 0.0, 0.0}, {1.0, 0.0, 0.0}, sc_zero(), sc_zero(), sc_zero(), sc_zero()};
+}
+__device__ __forceinline__ EvState evstate_of(const EvMap& f) { return {f.a, f.b, f.g, f.c, f.h, f.k}; }
+// with every mantissa back in [1/2, 1)
+__device__ __forceinline__ EvMap evmap_of(const EvState& s) {
+  return {scd_norm(s.X), scd_norm(s.Q), sc_norm(s.Z), sc_norm(s.Y), sc_norm(s.Z2), sc_norm(s.dZ2)};
 }
 
-// the single-step map of sample (n, logL) preceded by log-likelihood Lprev; the
-// per-factor expressions follow shrinkage_statistics.py:47-72.
-// the coefficients of one step that depend on the live-point count n alone (T, T2, t, t2, tT)
+// the coefficients of one step that depend on the live-point count n alone.  A count with no logarithm
+// gives NaN, as in the reference.
 struct EvCoef {
-  double n, T, T2, t, t2, tT;
+  double n, T, Tl, R, Rl, t, i2;  // T and R = (n+1)/(n+2) with their low parts, t = 1/(n+1), i2 = 1/(n+2)
 };
 __device__ __forceinline__ EvCoef evcoef(double n) {
-  const double LOG2 = 0.69314718055994530942;
-  const double log_n = log(n);
-  const double log_n1 = log(n + 1.0);
-  const double log_n2 = log(n + 2.0);
+  const double n1 = n + 1.0, n2 = n + 2.0;
+  const double i1 = 1.0 / n1, i2 = 1.0 / n2;
+  const bool whole = n < __builtin_inf();
   EvCoef c;
   c.n = n;
-  c.T = -lae(0.0, -log_n);
-  c.t = -log_n1;
-  c.T2 = -lae(0.0, LOG2 - log_n);
-  c.t2 = LOG2 - log_n1 - log_n2;
-  c.tT = c.T - log_n2;
+  c.T = n < 0.0 ? __builtin_nan("") : (n < 1.0 ? n * i1 : 1.0 - i1);
+  c.Tl = whole ? fma(-c.T, n1, n) * i1 : 0.0;
+  c.R = 1.0 - i2;
+  c.Rl = whole ? fma(-c.R, n2, n1) * i2 : 0.0;
+  c.t = n1 < 0.0 ? __builtin_nan("") : i1;
+  c.i2 = n2 < 0.0 ? __builtin_nan("") : i2;
   return c;
 }
 // the coefficients of n, formed again only when n differs from the cached step's (runs of equal n
@@ -376,98 +491,67 @@ __device__ __forceinline__ const EvCoef& evcoef_cached(EvCoef& c, double n) {
 __device__ __forceinline__ EvCoef evcoef_empty() {
   EvCoef c;
   c.n = __builtin_nan("");
-  c.T = c.T2 = c.t = c.t2 = c.tT = 0.0;
+  c.T = c.Tl = c.R = c.Rl = c.t = c.i2 = 0.0;
   return c;
 }
 
-__device__ __forceinline__ EvMap evmap_step_c(const EvCoef& c, double Lprev, double L, double* log_tm) {
-  const double LOG2 = 0.69314718055994530942;
-  double midL = -LOG2 + lae(L, Lprev);
-  EvMap m;
-  m.a = c.T;
-  m.b = c.T2;
-  m.g = c.t + midL;
-  m.e = c.tT + midL;
-  m.z = LOG2 + c.t + midL;
-  m.h = c.t2 + 2.0 * midL;
-  m.th = m.h;
-  *log_tm = m.g;
-  return m;
-}
+// m = (L_prev + L) / 2 of a step
+__device__ __forceinline__ Sc ev_mid(const Sc& Lprev, const Sc& L) { return sc_scale(sc_add(L, Lprev), 0.5); }
 
-__device__ __forceinline__ EvMap evmap_step(double n, double Lprev, double L, double* log_tm) {
-  return evmap_step_c(evcoef(n), Lprev, L, log_tm);
+// one step of the recurrence; returns dZ = t m X
+__device__ __forceinline__ Sc ev_step(EvState& s, const EvCoef& c, const Sc& mid) {
+  Sc w = {c.t * mid.m * s.X.m, mid.e + s.X.e};
+  Sc y = {c.i2 * mid.m * s.Q.m, mid.e + s.Q.e};
+  if (c.t == 0.0) w = y = sc_zero();  // an infinite count
+  const Sc w2 = sc_scale(w, 2.0);
+  s.Z = sc_add(s.Z, w);
+  s.Y = sc_add(s.Y, y);
+  s.Z2 = sc_add(s.Z2, sc_mul(w2, s.Y));
+  s.dZ2 = sc_add(s.dZ2, sc_mul(w2, y));
+  s.X = scd_scale(s.X, c.T, c.Tl);
+  s.Q = scd_scale(s.Q, c.R, c.Rl);
+  // counts below one shrink X by more than half a step: not left to the end of the caller's run of steps
+  if (c.T < 0.5) s.X = c.T == 0.0 ? scd_zero() : scd_norm(s.X);
+  return w;
 }
 
 // f then g
 __device__ __forceinline__ EvMap evmap_then(const EvMap& f, const EvMap& g) {
   EvMap r;
-  r.a = g.a + f.a;
-  r.b = g.b + f.b;
-  r.g = lae(f.g, g.g + f.a);
-  r.e = lae(g.a + f.e, g.e + f.b);
-  r.z = lae(f.z, g.z + f.a);
-  r.h = lae(lae(f.h, g.z + f.e), g.h + f.b);
-  r.th = lae(f.th, g.th + f.b);
+  const Sc fa = sc_of(f.a), fb = sc_of(f.b);
+  const Sc ga = sc_mul(g.g, fa), fab = sc_mul(fa, fb);
+  r.a = scd_mul(f.a, g.a);
+  r.b = scd_mul(f.b, g.b);
+  r.g = sc_norm(sc_add(f.g, ga));
+  r.c = sc_norm(sc_add(f.c, sc_mul(g.c, fb)));
+  r.h = sc_norm(sc_add(sc_add(f.h, sc_scale(sc_mul(ga, f.c), 2.0)), sc_mul(g.h, fab)));
+  r.k = sc_norm(sc_add(f.k, sc_mul(g.k, fab)));
   return r;
 }
 
 __device__ __forceinline__ EvState evmap_apply(const EvMap& f, const EvState& s) {
-  EvState o;
-  o.L = s.L;
-  o.X = f.a + s.X;
-  o.X2 = f.b + s.X2;
-  o.Z = lae(s.Z, f.g + s.X);
-  o.ZX = lae(f.a + s.ZX, f.e + s.X2);
-  o.Z2 = lae(lae(s.Z2, f.z + s.ZX), f.h + s.X2);
-  o.dZ = s.dZ;
-  o.dZ2 = lae(s.dZ2, f.th + s.X2);
-  return o;
+  return evstate_of(evmap_then({s.X, s.Q, s.Z, s.Y, s.Z2, s.dZ2}, f));
 }
 
-// one sequential recurrence step (the reference op itself); returns the new state
-__device__ __forceinline__ EvState ev_step_c(const EvState& s, const EvCoef& c, double L) {
-  double log_tm;
-  EvMap f = evmap_step_c(c, s.L, L, &log_tm);
-  EvState o = evmap_apply(f, s);
-  o.L = L;
-  o.dZ = log_tm + s.X;
-  return o;
-}
-__device__ __forceinline__ EvState ev_step(const EvState& s, double n, double L) {
-  double log_tm;
-  EvMap f = evmap_step(n, s.L, L, &log_tm);
-  EvState o = evmap_apply(f, s);
-  o.L = L;
-  o.dZ = log_tm + s.X;
-  return o;
-}
+// the fields of EvidenceCalculation that a state stands for
+__device__ __forceinline__ Sc ev_X2(const EvState& s) { return sc_mul(sc_of(s.X), sc_of(s.Q)); }
+__device__ __forceinline__ Sc ev_ZX(const EvState& s) { return sc_mul(sc_of(s.X), s.Y); }
 
-__device__ __forceinline__ EvState evstate_from(const double* s8) {
-  return {s8[0], s8[1], s8[2], s8[3], s8[4], s8[5], s8[6], s8[7]};
+__device__ __forceinline__ Sc sc_shfl_down(const Sc& x, int o) { return {__shfl_down(x.m, o, 64), __shfl_down(x.e, o, 64)}; }
+__device__ __forceinline__ Sc sc_shfl_up(const Sc& x, int o) { return {__shfl_up(x.m, o, 64), __shfl_up(x.e, o, 64)}; }
+__device__ __forceinline__ Scd sc_shfl_down(const Scd& x, int o) {
+  return {__shfl_down(x.m, o, 64), __shfl_down(x.lo, o, 64), __shfl_down(x.e, o, 64)};
 }
-__device__ __forceinline__ void evstate_to(const EvState& s, double* s8) {
-  s8[0] = s.L;
-  s8[1] = s.X;
-  s8[2] = s.X2;
-  s8[3] = s.Z;
-  s8[4] = s.ZX;
-  s8[5] = s.Z2;
-  s8[6] = s.dZ;
-  s8[7] = s.dZ2;
-}
-
-__device__ __forceinline__ EvMap shfl_xor_map(const EvMap& m, int o) {
-  return {__shfl_xor(m.a, o, 64), __shfl_xor(m.b, o, 64), __shfl_xor(m.g, o, 64), __shfl_xor(m.e, o, 64),
-          __shfl_xor(m.z, o, 64), __shfl_xor(m.h, o, 64), __shfl_xor(m.th, o, 64)};
+__device__ __forceinline__ Scd sc_shfl_up(const Scd& x, int o) {
+  return {__shfl_up(x.m, o, 64), __shfl_up(x.lo, o, 64), __shfl_up(x.e, o, 64)};
 }
 __device__ __forceinline__ EvMap shfl_down_map(const EvMap& m, int o) {
-  return {__shfl_down(m.a, o, 64), __shfl_down(m.b, o, 64), __shfl_down(m.g, o, 64), __shfl_down(m.e, o, 64),
-          __shfl_down(m.z, o, 64), __shfl_down(m.h, o, 64), __shfl_down(m.th, o, 64)};
+  return {sc_shfl_down(m.a, o), sc_shfl_down(m.b, o), sc_shfl_down(m.g, o),
+          sc_shfl_down(m.c, o), sc_shfl_down(m.h, o), sc_shfl_down(m.k, o)};
 }
 __device__ __forceinline__ EvMap shfl_up_map(const EvMap& m, int o) {
-  return {__shfl_up(m.a, o, 64), __shfl_up(m.b, o, 64), __shfl_up(m.g, o, 64), __shfl_up(m.e, o, 64),
-          __shfl_up(m.z, o, 64), __shfl_up(m.h, o, 64), __shfl_up(m.th, o, 64)};
+  return {sc_shfl_up(m.a, o), sc_shfl_up(m.b, o), sc_shfl_up(m.g, o),
+          sc_shfl_up(m.c, o), sc_shfl_up(m.h, o), sc_shfl_up(m.k, o)};
 }
 
 // linear_to_log_stats (internals/stats.py:55-74)

@@ -11,7 +11,7 @@ namespace hipns {
 
 // ===========================================================================
 // Evidence scan: compute_evidence_stats (internals/shrinkage_statistics.py:131-157)
-// as a reduce-then-scan over 7-coefficient log-space maps, in three launches
+// as a reduce-then-scan over 6-coefficient maps, in three launches
 // (grid.y = segment, so one set of launches serves every run of a batch):
 //   1. k_ev_reduce: each 256-thread block reduces a tile of 256*ITEMS
 //      consecutive samples (each thread composes its ITEMS step maps, then an
@@ -19,13 +19,18 @@ namespace hipns {
 //      every thread's exclusive prefix within the tile;
 //   2. k_ev_scan_tiles: one block per segment scans the tile aggregates
 //      (exclusive, in place);
-//   3. k_ev_apply: each thread applies its prefix to the initial state and
-//      steps through its samples, forming each step map again.
+//   3. k_ev_apply_all: each thread applies its prefix to the initial state and
+//      steps through its samples; k_ev_last does so for the last sample alone
+//      where nothing else is wanted.
 // The grouping of the compositions depends only on the sample count, so a
 // segment's results do not depend on the other segments or on timing.
+// Bound by FP64 VALU.  With the maps held as logarithms every sum in a composition was an exp and a
+// log1p; as scaled numbers (Sc, hipns_dev.h) 2 M samples take 31 us to reduce (192 before), 15 to scan the
+// tiles (83) and 83 to write all statistics (140); 1024 runs of 5 000 samples reduce in 0.31 ms (2.49).
 // ===========================================================================
 constexpr int EV_THREADS = 256;
-constexpr int EV_ITEMS = 8;
+constexpr int EV_ITEMS = 16;
+constexpr int EV_STEP = 8;  // samples of a thread whose loads issue together
 constexpr int EV_TILE = EV_THREADS * EV_ITEMS;
 constexpr int EV_SCAN_THREADS = 1024;
 
@@ -79,6 +84,17 @@ struct EvSegBatch {
   }
 };
 
+// a thread's prefix within its tile, as it is stored (a tile's product has no use for a low part)
+struct EvPrefix {
+  Sc a, b, g, c, h, k;
+};
+__device__ __forceinline__ EvPrefix evprefix_of(const EvMap& f) {
+  return {sc_of(f.a), sc_of(f.b), f.g, f.c, f.h, f.k};
+}
+__device__ __forceinline__ EvMap evmap_of(const EvPrefix& f) {
+  return {{f.a.m, 0.0, f.a.e}, {f.b.m, 0.0, f.b.e}, f.g, f.c, f.h, f.k};
+}
+
 // ordered inclusive scan of one map per lane across the wavefront
 __device__ __forceinline__ EvMap wave_incl_scan(EvMap x) {
   const int l = lane_id();
@@ -91,7 +107,7 @@ __device__ __forceinline__ EvMap wave_incl_scan(EvMap x) {
 }
 
 template <class Seg>
-__global__ void __launch_bounds__(EV_THREADS) k_ev_reduce(Seg seg, int64_t T, EvMap* tile_agg, EvMap* thr_excl) {
+__global__ void __launch_bounds__(EV_THREADS) k_ev_reduce(Seg seg, int64_t T, EvMap* tile_agg, EvPrefix* thr_excl) {
   __shared__ EvMap wave_aggs[EV_THREADS / 64];
   const int r = blockIdx.y;
   const int64_t M = seg.len(r), stop = seg.stop_at(r);
@@ -100,17 +116,29 @@ __global__ void __launch_bounds__(EV_THREADS) k_ev_reduce(Seg seg, int64_t T, Ev
   const auto src = seg.src(r);
   const int tid = threadIdx.x, l = lane_id(), w = tid / 64;
   const int64_t base = tile * EV_TILE + (int64_t)tid * EV_ITEMS;
-  const double ninf = -__builtin_inf();
-  EvMap m = evmap_identity();
+  const int64_t end = stop < M ? stop : M;
+  EvState st = evstate_initial();
   EvCoef cc = evcoef_empty();
-  for (int k = 0; k < EV_ITEMS; ++k) {
-    const int64_t i = base + k;
-    if (i < M && i < stop) {
-      double lt;
-      const double Lp = i == 0 ? ninf : src.L(i - 1);
-      m = evmap_then(m, evmap_step_c(evcoef_cached(cc, src.N(i)), Lp, src.L(i), &lt));
+  Sc prev = (base > 0 && base < end) ? sc_exp(src.L(base - 1)) : sc_zero();
+  for (int k0 = 0; k0 < EV_ITEMS; k0 += EV_STEP) {
+    double L[EV_STEP], n[EV_STEP];
+    // all loads first (clamped in-bounds index, so they issue together)
+#pragma unroll
+    for (int k = 0; k < EV_STEP; ++k) {
+      const int64_t i = base + k0 + k < M ? base + k0 + k : M - 1;
+      L[k] = src.L(i);
+      n[k] = src.N(i);
+    }
+#pragma unroll
+    for (int k = 0; k < EV_STEP; ++k) {
+      if (base + k0 + k < end) {
+        const Sc cur = sc_exp(L[k]);
+        ev_step(st, evcoef_cached(cc, n[k]), ev_mid(prev, cur));
+        prev = cur;
+      }
     }
   }
+  const EvMap m = evmap_of(st);
   const EvMap incl = wave_incl_scan(m);
   if (l == 63) wave_aggs[w] = incl;
   __syncthreads();
@@ -118,7 +146,7 @@ __global__ void __launch_bounds__(EV_THREADS) k_ev_reduce(Seg seg, int64_t T, Ev
   for (int i = 0; i < w; ++i) wave_prefix = evmap_then(wave_prefix, wave_aggs[i]);
   EvMap lane_excl = shfl_up_map(incl, 1);
   if (l == 0) lane_excl = evmap_identity();
-  thr_excl[((int64_t)r * T + tile) * EV_THREADS + tid] = evmap_then(wave_prefix, lane_excl);
+  thr_excl[((int64_t)r * T + tile) * EV_THREADS + tid] = evprefix_of(evmap_then(wave_prefix, lane_excl));
   if (tid == 0) {
     EvMap agg = evmap_identity();
     for (int i = 0; i < EV_THREADS / 64; ++i) agg = evmap_then(agg, wave_aggs[i]);
@@ -168,77 +196,131 @@ __global__ void __launch_bounds__(EV_SCAN_THREADS) k_ev_scan_tiles(Seg seg, int6
   }
 }
 
-__device__ __forceinline__ void write_fin8(double* fin8, const EvState& o) {
-  fin8[0] = o.L;
-  fin8[1] = o.X;
-  fin8[2] = o.X2;
-  fin8[3] = o.Z;
-  fin8[4] = o.ZX;
-  fin8[5] = o.Z2;
-  fin8[6] = o.dZ;
-  fin8[7] = o.dZ2;
+__device__ __forceinline__ void write_fin8_initial(double* fin8) {
+  const double ninf = -__builtin_inf();
+  const double v[8] = {ninf, 0.0, 0.0, ninf, ninf, ninf, ninf, ninf};
+  for (int i = 0; i < 8; ++i) fin8[i] = v[i];
 }
 
-// per8 (PER8, flat segment only): [8][M] field-major; fin: 8 doubles per segment (may be NULL)
-template <bool PER8, class Seg>
-__global__ void __launch_bounds__(EV_THREADS) k_ev_apply(Seg seg, int64_t T, const EvMap* tile_excl,
-                                                         const EvMap* thr_excl, double* per8, double* fin) {
-  __shared__ double s_stage[PER8 ? EV_TILE : 1];
-  const int r = blockIdx.y;
-  const int64_t M = seg.len(r), stop = seg.stop_at(r);
-  const int64_t tile = blockIdx.x;
-  const int tid = threadIdx.x, l = lane_id(), w = tid / 64;
+__device__ __forceinline__ void ev_fields(double (&o)[8], double L, const EvState& s, const Sc& dZ) {
+  o[0] = L;
+  o[1] = sc_log(sc_of(s.X));
+  o[2] = sc_log(ev_X2(s));
+  o[3] = sc_log(s.Z);
+  o[4] = sc_log(ev_ZX(s));
+  o[5] = sc_log(s.Z2);
+  o[6] = sc_log(dZ);
+  o[7] = sc_log(s.dZ2);
+}
+
+// steps s through the samples [i0, i1) (uniform bounds are not needed); prev is L of the sample before i0
+template <class Src>
+__device__ __forceinline__ void ev_walk(EvState& s, Sc& prev, EvCoef& cc, const Src& src, int64_t i0, int64_t i1) {
+#pragma unroll 1
+  for (int64_t i = i0; i < i1; ++i) {
+    const Sc cur = sc_exp(src.L(i));
+    ev_step(s, evcoef_cached(cc, src.N(i)), ev_mid(prev, cur));
+    prev = cur;
+  }
+}
+
+// per8: [8][M] field-major; fin8: the last sample's (may be NULL).  One wavefront per block, 8 samples per
+// lane, so that the wavefront's 512 samples leave through LDS as whole 128-byte lines: with 16 per lane
+// and part of them staged at a time, lines left the L2 in pieces (2 M samples: 105 us with runs of 4
+// samples, 83 us with runs of 8).  A prefix covers 16 samples: the odd lane of a pair first walks the
+// even lane's.  Bound by FP64 VALU (seven logarithms per sample) at one wavefront per SIMD (LDS).
+constexpr int EV_OUT = EV_ITEMS / 2;
+__global__ void __launch_bounds__(64) k_ev_apply_all(EvSegFlat seg, const EvMap* tile_excl, const EvPrefix* thr_excl,
+                                                     double* per8, double* fin8) {
+  constexpr int PITCH = EV_OUT + 1;
+  __shared__ double stage[8][64 * PITCH];
+  const int64_t M = seg.M, stop = seg.stop;
+  const int l = threadIdx.x;
   const double ninf = -__builtin_inf();
-  const EvState s_init = {ninf, 0.0, 0.0, ninf, ninf, ninf, ninf, ninf};
-  double* fin8 = fin ? fin + 8 * (int64_t)r : nullptr;
-  if (M == 0) {
-    if (fin8 && tile == 0 && tid == 0) write_fin8(fin8, s_init);
+  const int64_t wbase = (int64_t)blockIdx.x * 64 * EV_OUT;
+  const auto src = seg.src(0);
+  const int64_t base = wbase + (int64_t)l * EV_OUT, pair = base - (base % EV_ITEMS);
+  const int64_t end = stop < M ? stop : M;
+  // the wavefront's L and n, read as whole lines into the places that fields 0 and 7 go to later
+  double* sL = stage[0];
+  double* sn = stage[7];
+#pragma unroll
+  for (int q = 0; q < EV_OUT; ++q) {
+    const int j = q * 64 + l, at = (j / EV_OUT) * PITCH + j % EV_OUT;
+    const int64_t i = wbase + j < M ? wbase + j : M - 1;
+    sL[at] = src.L(i);
+    sn[at] = src.N(i);
+  }
+  __syncthreads();
+  EvState s = evstate_initial();
+  Sc prev = sc_zero();
+  EvCoef cc = evcoef_empty();
+  if (base < end) {
+    s = evstate_of(evmap_then(tile_excl[wbase / EV_TILE], evmap_of(thr_excl[pair / EV_ITEMS])));
+    const int even = l & ~1;
+    if (pair > 0) prev = sc_exp(even > 0 ? sL[(even - 1) * PITCH + EV_OUT - 1] : src.L(wbase - 1));
+    if (l & 1) {
+#pragma unroll 1
+      for (int k = 0; k < EV_OUT; ++k) {
+        const Sc cur = sc_exp(sL[even * PITCH + k]);
+        ev_step(s, evcoef_cached(cc, sn[even * PITCH + k]), ev_mid(prev, cur));
+        prev = cur;
+      }
+      s = evstate_of(evmap_of(s));  // the mantissas back to [1/2, 1)
+    }
+  }
+  __syncthreads();
+#pragma unroll 1
+  for (int k = 0; k < EV_OUT; ++k) {
+    const int64_t i = base + k;
+    double o[8] = {ninf, 0.0, 0.0, ninf, ninf, ninf, ninf, ninf};
+    if (i < end) {
+      const double L = sL[l * PITCH + k];
+      const Sc cur = sc_exp(L);
+      const Sc dZ = ev_step(s, evcoef_cached(cc, sn[l * PITCH + k]), ev_mid(prev, cur));
+      prev = cur;
+      ev_fields(o, L, s, dZ);
+      if (fin8 && i == end - 1)
+        for (int f = 0; f < 8; ++f) fin8[f] = o[f];
+    }
+#pragma unroll
+    for (int f = 0; f < 8; ++f) stage[f][l * PITCH + k] = o[f];
+  }
+  __syncthreads();
+#pragma unroll
+  for (int f = 0; f < 8; ++f)
+#pragma unroll
+    for (int q = 0; q < EV_OUT; ++q) {
+      const int j = q * 64 + l;
+      if (wbase + j < M) per8[(int64_t)f * M + wbase + j] = stage[f][(j / EV_OUT) * PITCH + j % EV_OUT];
+    }
+}
+
+// the last sample's statistics alone: one thread per segment steps its run of samples
+template <class Seg>
+__global__ void __launch_bounds__(64) k_ev_last(Seg seg, int R, int64_t T, const EvMap* tile_excl,
+                                                const EvPrefix* thr_excl, double* fin) {
+  const int r = blockIdx.x * blockDim.x + threadIdx.x;
+  if (r >= R) return;
+  double* fin8 = fin + 8 * (int64_t)r;
+  const int64_t M = seg.len(r), stop = seg.stop_at(r);
+  const int64_t end = stop < M ? stop : M;
+  if (end < 1) {
+    write_fin8_initial(fin8);
     return;
   }
-  if (tile * EV_TILE >= M) return;  // block-uniform
   const auto src = seg.src(r);
-  const int64_t base = tile * EV_TILE + (int64_t)tid * EV_ITEMS;
-  const EvMap pre = evmap_then(tile_excl[(int64_t)r * T + tile], thr_excl[((int64_t)r * T + tile) * EV_THREADS + tid]);
-  EvState s = evmap_apply(pre, s_init);
-  s.L = (base == 0) ? ninf : (base - 1 < stop ? src.L(base - 1) : ninf);
-  s.dZ = ninf;
-  const int64_t last = (stop < M ? stop : M) - 1;
-  EvState out[PER8 ? EV_ITEMS : 1];
+  const int64_t t = (end - 1) / EV_ITEMS, base = t * EV_ITEMS, tile = t / EV_THREADS;
+  EvState s = evstate_of(
+      evmap_then(tile_excl[(int64_t)r * T + tile], evmap_of(thr_excl[(int64_t)r * T * EV_THREADS + t])));
+  Sc prev = base > 0 ? sc_exp(src.L(base - 1)) : sc_zero();
   EvCoef cc = evcoef_empty();
-#pragma unroll
-  for (int k = 0; k < EV_ITEMS; ++k) {
-    const int64_t i = base + k;
-    EvState o = s_init;
-    if (i < M && i < stop) {
-      o = ev_step_c(s, evcoef_cached(cc, src.N(i)), src.L(i));
-      s = o;
-    }
-    if constexpr (PER8) out[k] = o;
-    if (fin8 && i == last) write_fin8(fin8, o);
-  }
-  if constexpr (PER8) {
-    // field by field through a per-wavefront LDS stage, so that each store writes 64 consecutive
-    // samples (the thread's own samples are consecutive, 8 doubles apart between lanes)
-    double* stage = s_stage + w * 64 * EV_ITEMS;
-    const int64_t wbase = tile * EV_TILE + (int64_t)w * 64 * EV_ITEMS;
-#pragma unroll
-    for (int f = 0; f < 8; ++f) {
-#pragma unroll
-      for (int k = 0; k < EV_ITEMS; ++k) {
-        const EvState& o = out[k];
-        const double v = f == 0 ? o.L : f == 1 ? o.X : f == 2 ? o.X2 : f == 3 ? o.Z : f == 4 ? o.ZX
-                       : f == 5 ? o.Z2 : f == 6 ? o.dZ : o.dZ2;
-        stage[l * EV_ITEMS + k] = v;
-      }
-      __syncthreads();
-#pragma unroll
-      for (int k = 0; k < EV_ITEMS; ++k) {
-        const int64_t i = wbase + k * 64 + l;
-        if (i < M) per8[(int64_t)f * M + i] = stage[k * 64 + l];
-      }
-      __syncthreads();
-    }
-  }
+  ev_walk(s, prev, cc, src, base, end - 1);
+  const Sc cur = sc_exp(src.L(end - 1));
+  const Sc dZ = ev_step(s, evcoef_cached(cc, src.N(end - 1)), ev_mid(prev, cur));
+  double o[8];
+  ev_fields(o, src.L(end - 1), evstate_of(evmap_of(s)), dZ);
+  for (int f = 0; f < 8; ++f) fin8[f] = o[f];
 }
 
 // workspace of the scan of R segments of at most Mmax samples: tile aggregates / prefixes, then the
@@ -246,28 +328,30 @@ __global__ void __launch_bounds__(EV_THREADS) k_ev_apply(Seg seg, int64_t T, con
 static int64_t ev_tiles(int64_t Mmax) { return Mmax > 0 ? (Mmax + EV_TILE - 1) / EV_TILE : 1; }
 static size_t ev_ws_bytes(int R, int64_t Mmax) {
   const int64_t T = ev_tiles(Mmax);
-  return (size_t)R * T * sizeof(EvMap) * (1 + EV_THREADS) + 256;
+  return (size_t)R * T * (sizeof(EvMap) + sizeof(EvPrefix) * EV_THREADS) + 256;
 }
 
 template <class Seg>
 static void ev_launch(const Seg& seg, int R, int64_t Mmax, void* ws, double* per8, double* fin, hipStream_t s) {
   const int64_t T = ev_tiles(Mmax);
   EvMap* tile_agg = (EvMap*)ws;
-  EvMap* thr_excl = tile_agg + (size_t)R * T;
+  EvPrefix* thr_excl = (EvPrefix*)(tile_agg + (size_t)R * T);
   const dim3 grid((unsigned)T, (unsigned)R);
   hipLaunchKernelGGL(k_ev_reduce<Seg>, grid, dim3(EV_THREADS), 0, s, seg, T, tile_agg, thr_excl);
   hipLaunchKernelGGL(k_ev_scan_tiles<Seg>, dim3(1, (unsigned)R), dim3(EV_SCAN_THREADS), 0, s, seg, T, tile_agg);
-  if (per8)
-    hipLaunchKernelGGL((k_ev_apply<true, Seg>), grid, dim3(EV_THREADS), 0, s, seg, T, tile_agg, thr_excl, per8, fin);
-  else
-    hipLaunchKernelGGL((k_ev_apply<false, Seg>), grid, dim3(EV_THREADS), 0, s, seg, T, tile_agg, thr_excl, per8, fin);
+  if constexpr (std::is_same<Seg, EvSegFlat>::value) {
+    if (per8) {
+      hipLaunchKernelGGL(k_ev_apply_all, dim3((unsigned)((seg.M + 64 * EV_OUT - 1) / (64 * EV_OUT))), dim3(64), 0, s,
+                         seg, tile_agg, thr_excl, per8, fin);
+      return;
+    }
+  }
+  if (fin)
+    hipLaunchKernelGGL(k_ev_last<Seg>, dim3((unsigned)((R + 63) / 64)), dim3(64), 0, s, seg, R, T, tile_agg, thr_excl,
+                       fin);
 }
 
-__global__ void k_fin_init(double* fin8) {
-  const double ninf = -__builtin_inf();
-  double v[8] = {ninf, 0.0, 0.0, ninf, ninf, ninf, ninf, ninf};
-  for (int i = 0; i < 8; ++i) fin8[i] = v[i];
-}
+__global__ void k_fin_init(double* fin8) { write_fin8_initial(fin8); }
 
 size_t evidence_scan_ws(int64_t M) { return ev_ws_bytes(1, M); }
 
@@ -297,7 +381,7 @@ void* g_scratch_dev[HIPNS_MAX_DEVICES] = {};
 
 size_t evidence_scan_static_max() {
   // the largest M whose workspace fits the array
-  const size_t per_tile = sizeof(EvMap) * (1 + EV_THREADS);
+  const size_t per_tile = sizeof(EvMap) + sizeof(EvPrefix) * EV_THREADS;
   return (size_t)((HIPNS_SCAN_SCRATCH_BYTES - 256) / per_tile) * EV_TILE;
 }
 

@@ -155,6 +155,40 @@ def test_evidence_scan_vs_oracle(M, stop):
         np.testing.assert_allclose(a[fa], b[fb], rtol=1e-9, atol=1e-9)
 
 
+@pytest.mark.parametrize("kind", ["plain", "unsorted", "wide", "empty head", "nothing left"])
+@pytest.mark.parametrize("M", [1, 15, 16, 17, 511, 512, 513, 4095, 4096, 4097, 12289])
+def test_evidence_scan_edges_and_ranges(M, kind):
+    """Sizes at the edges of a thread's 16 samples, a wavefront's 512 and a tile's 4096, and inputs far outside
+    the range of a double: log L over twelve decades, log L = -inf, and a live-point count of 0 (X and ZX
+    become zero).  Each of M steps rounds at most 8 times on either side: 1.1e-11 absolute at M = 12289; the
+    oracle's logarithms round relative to their size, M ulps at most (2.7e-12)."""
+    torch = _torch()
+    rng = np.random.default_rng(M)
+    say(f"evidence_scan {kind} M={M}")
+    logL = np.sort(rng.normal(size=M) * 40.0)
+    n = rng.integers(1, 400, size=M).astype(np.float64)
+    if kind == "unsorted":
+        logL = rng.normal(size=M) * 400.0
+    elif kind == "wide":
+        logL = np.sort(-10.0 ** rng.uniform(-3, 9, size=M))
+    elif kind == "empty head":
+        logL[:M // 3 + 1] = -np.inf
+    elif kind == "nothing left":
+        n[2 * M // 3] = 0.0
+    fin_o, per_o = O.compute_evidence_stats(logL, n)
+    L, N = torch.from_numpy(logL).cuda(), torch.from_numpy(n).cuda()
+    per = torch.empty((8, M), dtype=torch.float64, device="cuda")
+    fin = [torch.empty(8, dtype=torch.float64, device="cuda") for _ in range(2)]
+    ws = torch.empty(lib().hipns_evidence_scan_workspace_size(M), dtype=torch.uint8, device="cuda")
+    check(lib().hipns_evidence_scan(ptr(L), ptr(N), M, -1, ptr(per), ptr(fin[0]), ptr(ws), ws.numel(), _stream()))
+    check(lib().hipns_evidence_scan(ptr(L), ptr(N), M, -1, None, ptr(fin[1]), ptr(ws), ws.numel(), _stream()))
+    for a, b in ((per.cpu().numpy().T, per_o), (fin[0].cpu().numpy(), fin_o), (fin[1].cpu().numpy(), fin_o)):
+        fa = np.isfinite(a)
+        assert np.array_equal(fa, np.isfinite(b))
+        assert np.array_equal(a[~fa], b[~fa])
+        np.testing.assert_allclose(a[fa], b[fa], rtol=2.7e-12, atol=1.1e-11)
+
+
 def test_evidence_scan_closed_form_large():
     """3 000 000 samples (1465 tiles of 2048, so the tile scan composes two tiles per thread) against
     the closed forms of a constant likelihood L = 1 with n = N throughout: log X_i = i log(N/(N+1)),
