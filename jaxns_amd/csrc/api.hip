@@ -173,24 +173,31 @@ int sampler_launch(int mode, const hipns_launch_t* L, const hipns::SampleArgs& A
   }
   A.lr_groups = groups;
   A.alpha_off =
-      (int32_t)hipns::sampler_lds_floats(L->family, dps, maxD, L->gmm_K, lpc, groups, L->lr_ndata);
+      (int32_t)hipns::sampler_lds_floats(L->family, dps, maxD, L->gmm_K, lpc, groups, L->lr_ndata, 1,
+                                         mode == hipns::MODE_GSLICE);
   const size_t base_f = (size_t)A.alpha_off + (size_t)max_slices;
   size_t lds = base_f * sizeof(float);
   if ((int)lds > max_lds_bytes())
     return fail(HIPNS_ERANGE, "model parameters need %zu B of LDS, device allows %d", lds, max_lds_bytes());
-  // direction rings after the alpha table (16-byte aligned): depth 3 for the 8-slot instances, 2 with one
-  // wavefront per block (where the per-block parameters repeat per wavefront and LDS would cap residency)
-  // and for 16 slots; none when the block's LDS would exceed the device limit
+  // direction rings after the alpha table (16-byte aligned), as deep as the LDS of a CU allows with the
+  // workgroups resident that the launch brings it; none where even DIR_RING_MIN slots exceed the limit
   const int nj = hipns::sampler_nj(maxD, lpc);
-  int ring = hipns::dir_ring_max(mode, L->family, nj);
-  if (ring > 2 && L->waves_per_block < 2) ring = 2;
+  int ring = 0;
   A.ring_off = (int32_t)((base_f + 3) / 4 * 4);
-  const size_t ring_lds =
-      ((size_t)A.ring_off + (size_t)ring * HIPNS_WAVE * nj * L->waves_per_block) * sizeof(float);
-  if (ring > 0 && (int)ring_lds <= max_lds_bytes()) {
-    lds = ring_lds;
-  } else {
-    ring = 0;
+  if (hipns::has_dir_ring(mode, L->family, nj)) {
+    const int wpb = L->waves_per_block, cw = HIPNS_WAVE / lpc;
+    const int64_t blocks = (int64_t)R * ((max_chains + cw * wpb - 1) / (cw * wpb));
+    const int64_t most = (nj <= 8 ? 16 : 8) / wpb;  // by registers
+    int64_t per_cu = (blocks + num_cus() - 1) / num_cus();
+    if (per_cu > most) per_cu = most < 1 ? 1 : most;
+    const size_t slot = (size_t)HIPNS_WAVE * nj * wpb * sizeof(float), fixed = (size_t)A.ring_off * sizeof(float);
+    // (a tenth less than the LDS: four workgroups of 37.6 KiB did not stay resident in 160 KiB)
+    const size_t budget = (size_t)max_lds_bytes() * 9 / 10 / per_cu;
+    ring = budget > fixed ? (int)((budget - fixed) / slot) : 0;
+    if (ring > hipns::DIR_RING_MAX) ring = hipns::DIR_RING_MAX;
+    if (ring < hipns::DIR_RING_MIN) ring = hipns::DIR_RING_MIN;
+    if (fixed + ring * slot > (size_t)max_lds_bytes()) ring = 0;
+    if (ring > 0) lds = fixed + ring * slot;
   }
   A.dir_ring = ring;
   if (spread) {
@@ -620,7 +627,7 @@ int hipns_log_likelihood_grad(const float* U_dev, int64_t B, double* logL_dev, f
   if (D < 1 || D > bufs->dps) return fail(HIPNS_EINVAL, "D outside [1, dps]");
   const int lpc = hipns::sampler_lpc(launch->family, launch->lanes_per_chain, bufs->dps, D);
   const size_t base_f =
-      hipns::sampler_lds_floats(launch->family, bufs->dps, D, launch->gmm_K, lpc, launch->waves_per_block, 0);
+      hipns::sampler_lds_floats(launch->family, bufs->dps, D, launch->gmm_K, lpc, launch->waves_per_block, 0, 1, true);
   const int gscr_off = (int)((base_f + 3) / 4 * 4);
   const int nj = hipns::sampler_nj(D, lpc);
   const size_t lds =

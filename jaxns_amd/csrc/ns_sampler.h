@@ -105,6 +105,13 @@ __host__ __device__ constexpr int grad_rows(int nj, int lpc) {
   return ((nj * lpc + 64 / lpc - 1) / (64 / lpc)) * (64 / lpc);
 }
 
+// rows of W^T in LDS: one (zero beyond the model) for every dimension slot of the instance, which reads all
+// of them; the gradient's product reads whole blocks of output rows
+__host__ __device__ constexpr int mvn_rows(int nj, int lpc, bool grad) { return grad ? grad_rows(nj, lpc) : nj * lpc; }
+
+// component rows of the mixture kernels' instances: 4, 6 or 8
+__host__ __device__ constexpr int gmm_rows(int K) { return K <= 4 ? 4 : (K <= 6 ? 6 : HIPNS_MAX_GMM_K); }
+
 // Regression: the most wavefronts of a workgroup (chain groups and row helpers; the instances of more than
 // 8 slots need more than the 256 VGPRs that two wavefronts per SIMD leave each), and the fixed blocks that
 // the data rows are summed in, whatever the number of wavefronts that share them.  A block boundary costs a
@@ -116,34 +123,36 @@ __host__ __device__ inline int lr_row_blocks(int tiles, int lpc) { return tiles 
 
 // floats of dynamic LDS one sampler block needs (layout of load_params in ns_sampler_impl.h); npad: the
 // regression family's padded data rows, sums: row sums kept per point (2 for the adjoint statistics)
-inline size_t sampler_lds_floats(int fam, int dps, int D, int K, int lpc, int G, int npad, int sums = 1) {
+inline size_t sampler_lds_floats(int fam, int dps, int D, int K, int lpc, int G, int npad, int sums = 1,
+                                 bool grad = false) {
   if (fam == HIPNS_FAM_LINREG) {
     const size_t NG = (size_t)sampler_nj(D, lpc) / 8;
     const size_t CW = (size_t)(64 / lpc);
     return (size_t)4 * dps + 4 + (size_t)G * NG * 3 * 64 * 4 + (size_t)sums * G * lr_row_blocks((int)(npad / CW), lpc) * CW * 2;
   }
   if (fam == HIPNS_FAM_MVN) {
-    // W^T holds a (zero) row for every dimension slot of the instance, so the kernel reads all NJ slots
     const int nj = sampler_nj(D, lpc);
-    const int rows = dps > nj * lpc ? dps : nj * lpc;
-    return (size_t)2 * dps + (size_t)rows * mvn_row_stride(nj, lpc);
+    return (size_t)2 * dps + (size_t)mvn_rows(nj, lpc, grad) * mvn_row_stride(nj, lpc);
   }
-  return (size_t)(3 + K) * dps + 2 * K;
+  return (size_t)(3 + gmm_rows(K)) * dps + 2 * gmm_rows(K);
 }
 
-// Depth of the per-chain ring of slice directions drawn ahead by an instance (0: none).  Every
-// wavefront step in which some chain of the wavefront begins a slice runs the direction draw for all
-// of its lanes, and ~43 % of chain steps begin one, so nearly every step paid for a draw.  With a ring
-// the draw runs only when a chain about to begin a slice has no direction left, and then tops up every
-// chain of the wavefront by one, so a pass serves several chains' later slices (0.96 -> ~0.6 passes per
-// step at depth 3 for 16 chains).  One ring slot is 64 lanes x nj floats per wavefront.  The regression
-// family (whose step is its data-row GEMM) and the 8-slot mixture instance (at 128 VGPRs, where the
-// ring's registers would cost a wavefront per SIMD) keep the draw at the slice start.
-__host__ __device__ constexpr int dir_ring_max(int mode, int fam, int nj) {
-  return (mode != MODE_SLICE || fam == HIPNS_FAM_LINREG || (fam == HIPNS_FAM_GMM && nj <= 8))
-             ? 0
-             : (nj <= 8 ? 3 : (nj <= 16 ? 2 : 0));
+// Whether an instance keeps a per-chain ring of slice directions drawn ahead.  Every wavefront step in
+// which some chain of the wavefront begins a slice runs the direction draw for all of its lanes, and
+// ~43 % of chain steps begin one, so nearly every step paid for a draw.  With a ring the draw runs only
+// when a chain about to begin a slice has no direction left, and then tops up every chain of the
+// wavefront by one, so a pass serves several chains' later slices.  One ring slot is 64 lanes x nj floats
+// per wavefront.  The regression family (whose step is its data-row GEMM) keeps the draw at the slice
+// start, and so do the 32-slot instances (8 KiB a slot).  Mixture, 64 runs of D <= 64 at 8 lanes per
+// chain: 799 ms per batch without a ring, 689 with one of depth 2.
+__host__ __device__ constexpr bool has_dir_ring(int mode, int fam, int nj) {
+  return mode == MODE_SLICE && fam != HIPNS_FAM_LINREG && nj <= 16;
 }
+// The ring's depth: draws per step fall from 0.69 at depth 2 over 0.59 at 3 to 0.47 at 8 (16 chains, 0.43
+// begins per chain step; a simulation of the slice lengths), so the ring takes the LDS that the launch
+// leaves free: a launch that fills the chip keeps its wavefronts resident (4 per SIMD at 8 slots, 2 at
+// 16; depth 3 or 2), a small one goes to 8.
+constexpr int DIR_RING_MIN = 2, DIR_RING_MAX = 8;
 
 hipError_t launch_ext_step(const hipns_run_desc_t* runs, hipns_run_state_t* states, const hipns_buffers_t& B,
                            const hipns_ext_state_t& E, int mode, int w, int max_steps, int R, int max_chains, int lpc,

@@ -9,16 +9,29 @@ namespace hipns {
 // ---------------------------------------------------------------------------
 // host-side dispatch over the template grid
 // ---------------------------------------------------------------------------
-template <int LPC, int NJ, int FAM, int MODE>
-inline hipError_t launch_one(const SampleArgs& A, int R, int max_chains, int wpb, size_t lds_bytes, hipStream_t s) {
+template <int LPC, int NJ, int FAM, int MODE, int KT>
+inline hipError_t launch_rows(const SampleArgs& A, int R, int max_chains, int wpb, size_t lds_bytes, hipStream_t s) {
   constexpr int CW = HIPNS_WAVE / LPC;
   const int per_block = FAM == HIPNS_FAM_LINREG ? A.lr_groups : wpb;  // chain groups
   int groups = (max_chains + CW - 1) / CW;
   int bx = (groups + per_block - 1) / per_block;
   if (bx < 1) bx = 1;
   dim3 grid(bx, R), block(wpb * HIPNS_WAVE);
-  hipLaunchKernelGGL((k_sample<LPC, NJ, FAM, MODE>), grid, block, lds_bytes, s, A);
+  hipLaunchKernelGGL((k_sample<LPC, NJ, FAM, MODE, KT>), grid, block, lds_bytes, s, A);
   return hipGetLastError();
+}
+
+template <int LPC, int NJ, int FAM, int MODE>
+inline hipError_t launch_one(const SampleArgs& A, int R, int max_chains, int wpb, size_t lds_bytes, hipStream_t s) {
+  if constexpr (FAM == HIPNS_FAM_GMM) {
+    switch (gmm_rows(A.gmm_K)) {
+      case 4: return launch_rows<LPC, NJ, FAM, MODE, 4>(A, R, max_chains, wpb, lds_bytes, s);
+      case 6: return launch_rows<LPC, NJ, FAM, MODE, 6>(A, R, max_chains, wpb, lds_bytes, s);
+      default: return launch_rows<LPC, NJ, FAM, MODE, HIPNS_MAX_GMM_K>(A, R, max_chains, wpb, lds_bytes, s);
+    }
+  } else {
+    return launch_rows<LPC, NJ, FAM, MODE, 1>(A, R, max_chains, wpb, lds_bytes, s);
+  }
 }
 
 // register slots per lane: the smallest instance whose NJ * LPC covers the widest run (D rounded up

@@ -77,10 +77,9 @@ struct GmmLds {
   float* tf;     // [DP]
   float* p;      // [DP]
   float* q;      // [DP]
-  float* mean;   // [K][DP]
-  float* inv2s2; // [K]
-  float* logc;   // [K]
-  int K;
+  float* mean;   // [gmm_rows(K)][DP]
+  float* inv2s2; // [gmm_rows(K)]
+  float* logc;   // [gmm_rows(K)], -inf past K
   int dps;
 };
 
@@ -574,14 +573,17 @@ __device__ __forceinline__ double lik_mvn(const float (&up)[NJ], int nj, int D, 
   const int m = l % CW;
   const int h = l / CW;
   float z[NJ];
-  prior_q<NJ>(up, z, tfm);
+  prior_q<NJ>(up, z, tfm);  // finite on padding slots (u = 1/2), which meet zeros of W
+  if constexpr (LPC == 4 && NJ == 8) {
+    // not needed, but this instance's schedule is the better one with the masks (D=32, 1024 runs: 12.42
+    // against 12.24 G evaluations/s), the others' without (D=10: 19.2 against 18.7; D=20: 8.9 against 8.6)
 #pragma unroll
-  for (int j = 0; j < NJ; ++j)
-    if (!(j < nj && owned_dim<LPC>(h, j) < D)) z[j] = 0.0f;
+    for (int j = 0; j < NJ; ++j)
+      if (!(j < nj && owned_dim<LPC>(h, j) < D)) z[j] = 0.0f;
+  }
   // A operands W[row][owned dim] at compile-time offsets from the lane's base (row m of block mb, owned
   // dim 8h); the accumulator of each block starts from this lane's output rows of b.  W^T has a row for
-  // every slot of the instance (zero beyond the model), and z is zero on slots beyond D, so all NJ
-  // slots are multiplied unconditionally.
+  // every slot of the instance (zero beyond the model), so all NJ slots are multiplied unconditionally.
   constexpr int RS = mvn_row_stride(NJ, LPC);
   constexpr int MBI = (NJ * LPC + CW - 1) / CW;
   const float* wt = P.WT + 8 * h * RS + m;
@@ -687,20 +689,23 @@ __device__ __forceinline__ double lik_mvn(const float (&up)[NJ], int nj, int D, 
 // GRAD: when some lane of the wavefront asks (want), also g = d logL / du of the owned slots:
 // d logL / dx_d = sum_k w_k (-2 inv2s2_k (x_d - m_kd)) with w_k the components' softmax weights, and
 // dx_d / du_d = q_d dq/du (x = p + q (.) q(u))
-template <int LPC, int NJ, bool GRAD = false>
+// KT: component rows in LDS (gmm_rows), those past K of weight zero.  Their number is known at compile time:
+// a test per component is a branch, and a wavefront alone on its SIMD pays each one in full (D=4, K=4, one
+// run of 60 chains: 2.27 -> 1.55 us a step with the tests and the padding masks gone and a direction ring).
+template <int LPC, int NJ, int KT, bool GRAD = false>
 __device__ __forceinline__ double lik_gmm(const float (&up)[NJ], int nj, int D, const GmmLds& P, uint32_t tfm,
                                           float* g = nullptr, bool want = false) {
   constexpr int CW = HIPNS_WAVE / LPC;
   const int h = lane_id() / CW;
-  float part[HIPNS_MAX_GMM_K];
+  float part[KT];
 #pragma unroll
-  for (int k = 0; k < HIPNS_MAX_GMM_K; ++k) part[k] = 0.0f;
+  for (int k = 0; k < KT; ++k) part[k] = 0.0f;
   float qv[NJ];
   prior_q<NJ>(up, qv, tfm);
   // Slots 4i..4i+3 of a lane are four consecutive dimensions (owned_dim), so the prior scale, offset and
   // component means come in 16-byte LDS reads, all issued before the arithmetic that waits on them.
-  // The reads cover the run's padding dimensions (below the row stride, so inside the LDS block);
-  // those slots contribute nothing.
+  // The reads cover the run's padding dimensions (below the row stride, so inside the LDS block), which
+  // hold zeros: x and the means are zero there.
   float xv[NJ];
 #pragma unroll
   for (int j = 0; j < NJ; j += 4) {
@@ -718,20 +723,22 @@ __device__ __forceinline__ double lik_gmm(const float (&up)[NJ], int nj, int D, 
   for (int j = 0; j < NJ; j += 4) {
     if (j < nj) {
       const int d0 = owned_dim<LPC>(h, j);
-      // every component's four means of these slots, read before any is used (components past K
-      // read component K - 1 again, a valid row, and are not used)
-      float4 m[HIPNS_MAX_GMM_K];
+      // four components' means of these slots at a time, read before any is used
 #pragma unroll
-      for (int k = 0; k < HIPNS_MAX_GMM_K; ++k)
-        m[k] = *reinterpret_cast<const float4*>(P.mean + (k < P.K ? k : P.K - 1) * P.dps + d0);
+      for (int k0 = 0; k0 < KT; k0 += 4) {
+        constexpr int KC = KT < 4 ? KT : 4;
+        float4 m[KC];
 #pragma unroll
-      for (int k = 0; k < HIPNS_MAX_GMM_K; ++k) {
-        if (k < P.K) {
+        for (int k = 0; k < KC; ++k)
+          if (k0 + k < KT) m[k] = *reinterpret_cast<const float4*>(P.mean + (k0 + k) * P.dps + d0);
+#pragma unroll
+        for (int k = 0; k < KC; ++k) {
+          if (k0 + k >= KT) break;
           const float mv[4] = {m[k].x, m[k].y, m[k].z, m[k].w};
 #pragma unroll
           for (int i = 0; i < 4; ++i) {
-            const float r = d0 + i < D ? xv[j + i] - mv[i] : 0.0f;  // padding slots contribute nothing
-            part[k] = fmaf(r, r, part[k]);
+            const float r = xv[j + i] - mv[i];
+            part[k0 + k] = fmaf(r, r, part[k0 + k]);
           }
         }
       }
@@ -742,31 +749,27 @@ __device__ __forceinline__ double lik_gmm(const float (&up)[NJ], int nj, int D, 
   // a peak keep distinct values), the correction (>= 0, <= log K) in FP32 with the hardware exp2 / log2
   float mx = -__builtin_inff(), ss_top = 0.0f, i_top = 0.0f, c_top = 0.0f;
 #pragma unroll
-  for (int k = 0; k < HIPNS_MAX_GMM_K; ++k) {
-    if (k < P.K) {
-      const float ss = chain_sum<LPC>(part[k]);
-      part[k] = fmaf(-ss, P.inv2s2[k], P.logc[k]);  // component log-density, FP32
-      if (!(part[k] <= mx)) {  // first maximum (a NaN component is taken, and propagates)
-        mx = part[k];
-        ss_top = ss;
-        i_top = P.inv2s2[k];
-        c_top = P.logc[k];
-      }
+  for (int k = 0; k < KT; ++k) {
+    const float ss = chain_sum<LPC>(part[k]);
+    part[k] = fmaf(-ss, P.inv2s2[k], P.logc[k]);  // component log-density, FP32
+    if (!(part[k] <= mx)) {  // first maximum (a NaN component is taken, and propagates)
+      mx = part[k];
+      ss_top = ss;
+      i_top = P.inv2s2[k];
+      c_top = P.logc[k];
     }
   }
   float sum = 0.0f;
 #pragma unroll
-  for (int k = 0; k < HIPNS_MAX_GMM_K; ++k)
-    if (k < P.K) sum += __builtin_amdgcn_exp2f((part[k] - mx) * 1.44269504088896341f);
+  for (int k = 0; k < KT; ++k)
+    sum += __builtin_amdgcn_exp2f((part[k] - mx) * 1.44269504088896341f);
   if constexpr (GRAD) {
     if (__any(want)) {
-      float wk[HIPNS_MAX_GMM_K];
+      float wk[KT];
       const float inv_sum = 1.0f / sum;
 #pragma unroll
-      for (int k = 0; k < HIPNS_MAX_GMM_K; ++k)
-        wk[k] = k < P.K ? -2.0f * P.inv2s2[k] * __builtin_amdgcn_exp2f((part[k] - mx) * 1.44269504088896341f) *
-                              inv_sum
-                        : 0.0f;
+      for (int k = 0; k < KT; ++k)
+        wk[k] = -2.0f * P.inv2s2[k] * __builtin_amdgcn_exp2f((part[k] - mx) * 1.44269504088896341f) * inv_sum;
 #pragma unroll
       for (int j = 0; j < NJ; ++j) {
         const int d = owned_dim<LPC>(h, j);
@@ -775,8 +778,8 @@ __device__ __forceinline__ double lik_gmm(const float (&up)[NJ], int nj, int D, 
         if (in) {
           const float x = xv[j];
 #pragma unroll
-          for (int k = 0; k < HIPNS_MAX_GMM_K; ++k)
-            if (k < P.K) dx = fmaf(wk[k], x - P.mean[k * P.dps + d], dx);
+          for (int k = 0; k < KT; ++k)
+            dx = fmaf(wk[k], x - P.mean[k * P.dps + d], dx);
         }
         g[j] = in ? dx * P.q[d] * dq_du(qv[j], (tfm >> j) & 1u) : 0.0f;
       }
@@ -804,7 +807,8 @@ __device__ __forceinline__ uint32_t transform_mask(const float* tf, int h, int n
 
 // dynamic LDS layout of one block (one run per block)
 __device__ __forceinline__ void load_params(int fam, const float* prm, int dps, int D, int K, float* lds, MvnLds& mv,
-                                            GmmLds& gm, int LPCv, LinRegLds* lr = nullptr, int G = 1, int NG = 1) {
+                                            GmmLds& gm, int LPCv, LinRegLds* lr = nullptr, int G = 1, int NG = 1,
+                                            bool grad = false) {
   const int tid = threadIdx.x;
   const int nt = blockDim.x;
   if (fam == HIPNS_FAM_LINREG) {
@@ -831,26 +835,32 @@ __device__ __forceinline__ void load_params(int fam, const float* prm, int dps, 
     mv.b = lds + dps;
     mv.WT = lds + 2 * dps;
     mv.RS = RS;
+    // padding dimensions hold zeros, whatever the caller's block has there
     for (int i = tid; i < dps; i += nt) {
-      mv.tf[i] = prm[i];
+      mv.tf[i] = i < D ? prm[i] : 0.0f;
+      mv.b[i] = i < D ? prm[dps + i] : 0.0f;
     }
-    for (int i = tid; i < dps; i += nt) mv.b[i] = prm[dps + i];
     const float* W = prm + 2 * dps;
-    const int rows = dps > 8 * NG * LPCv ? dps : 8 * NG * LPCv;
+    const int rows = mvn_rows(8 * NG, LPCv, grad);
     for (int i = tid; i < rows * RS; i += nt) {
       int d = i / RS, m = i % RS;
-      mv.WT[i] = (d < dps && m < dps && m < RS - 1) ? W[m * dps + d] : 0.0f;
+      mv.WT[i] = (d < D && m < D && m < RS - 1) ? W[m * dps + d] : 0.0f;
     }
   } else {
     gm.tf = lds;
     gm.p = lds + dps;
     gm.q = lds + 2 * dps;
     gm.mean = lds + 3 * dps;
-    gm.inv2s2 = lds + 3 * dps + K * dps;
-    gm.logc = gm.inv2s2 + K;
-    gm.K = K;
+    const int KT = gmm_rows(K);
+    gm.inv2s2 = lds + 3 * dps + KT * dps;
+    gm.logc = gm.inv2s2 + KT;
     gm.dps = dps;
-    for (int i = tid; i < (3 + K) * dps + 2 * K; i += nt) lds[i] = prm[i];
+    // padding dimensions and the rows past K hold zeros (log weight -inf)
+    for (int i = tid; i < (3 + KT) * dps; i += nt) lds[i] = (i < (3 + K) * dps && i % dps < D) ? prm[i] : 0.0f;
+    for (int k = tid; k < KT; k += nt) {
+      gm.inv2s2[k] = k < K ? prm[(3 + K) * dps + k] : 0.0f;
+      gm.logc[k] = k < K ? prm[(3 + K) * dps + K + k] : -__builtin_inff();
+    }
   }
   __syncthreads();
 }
@@ -1015,8 +1025,12 @@ __device__ __forceinline__ void uniform_point(float (&up)[NJ], int chain, uint32
   }
 }
 
-template <int LPC, int NJ, int FAM, int MODE>
-__global__ void __launch_bounds__(FAM == HIPNS_FAM_LINREG ? HIPNS_WAVE * lr_max_waves(NJ) : 256) k_sample(SampleArgs A) {
+// (the 8-slot mixture instances of up to six components fit the 128 VGPRs of four wavefronts per SIMD; that
+// of eight would spill 32 of them there, 9.2 against 9.6 G evaluations/s at D=32, K=8, 512 runs)
+template <int LPC, int NJ, int FAM, int MODE, int KT>
+__global__ void __launch_bounds__(FAM == HIPNS_FAM_LINREG ? HIPNS_WAVE * lr_max_waves(NJ) : 256,
+                                  FAM == HIPNS_FAM_GMM && NJ == 8 && KT <= 6 && MODE != MODE_GSLICE ? 4 : 1)
+    k_sample(SampleArgs A) {
   constexpr int CW = HIPNS_WAVE / LPC;
   // the regression family multiplies the data rows against every chain group of the workgroup
   // cooperatively, so its wavefronts step together (workgroup-uniform loop)
@@ -1051,12 +1065,14 @@ __global__ void __launch_bounds__(FAM == HIPNS_FAM_LINREG ? HIPNS_WAVE * lr_max_
   const int dps = A.B.dps;
   const int D = run.D;
   const int DPr = ((D + 8 * LPC - 1) / (8 * LPC)) * (8 * LPC);
-  const int nj = DPr / LPC;
+  // (a run has at least 8 slots per lane; not folded where lik_mvn keeps its masks)
+  const int nj = (NJ == 8 && !(FAM == HIPNS_FAM_MVN && LPC == 4)) ? 8 : DPr / LPC;
 
   MvnLds mv;
   GmmLds gm;
   LinRegLds lr;
-  load_params(FAM, A.B.params + run.param_off, dps, D, A.gmm_K, lds, mv, gm, LPC, &lr, COOP ? G : 1, NJ / 8);
+  load_params(FAM, A.B.params + run.param_off, dps, D, A.gmm_K, lds, mv, gm, LPC, &lr, COOP ? G : 1, NJ / 8,
+              MODE == MODE_GSLICE);
   if (COOP) {
     lr.r0 = A.lr_r0;
     lr.r0l = lds + A.lr_r0_off;
@@ -1128,11 +1144,11 @@ __global__ void __launch_bounds__(FAM == HIPNS_FAM_LINREG ? HIPNS_WAVE * lr_max_
   // ---- ring of slice directions drawn ahead (MODE_SLICE): slot b of this wavefront holds, for every
   // lane, the nj owned components of one direction, as nj / 4 float4 rows of 64 lanes.  A chain's ring
   // holds the directions of its slices [s, gen) (gen - s <= ring), in slot (slice index mod ring).
-  constexpr int RB = dir_ring_max(MODE, FAM, NJ);
+  constexpr bool RB = has_dir_ring(MODE, FAM, NJ);
   constexpr int RSLOT = (NJ / 4) * HIPNS_WAVE;  // float4s of one ring slot
-  const int ring = RB > 0 ? A.dir_ring : 0;
+  const int ring = RB ? A.dir_ring : 0;
   float4* ring_base = nullptr;
-  if (RB > 0) ring_base = (float4*)(lds + A.ring_off) + (size_t)wave * ring * RSLOT + l;
+  if (RB) ring_base = (float4*)(lds + A.ring_off) + (size_t)wave * ring * RSLOT + l;
   int gen = 0, gslot = 0;  // next slice to draw and its slot
   // gradient slice chains: the wavefront's LDS scratch for d logL / dU, and the state of the gradient step
   float* gscr = GG ? lds + A.ring_off + (size_t)wave * grad_rows(NJ, LPC) * (CW + 1) : nullptr;
@@ -1147,7 +1163,7 @@ __global__ void __launch_bounds__(FAM == HIPNS_FAM_LINREG ? HIPNS_WAVE * lr_max_
     alpha = alpha_tab[si];
     if (GG && dir_ready) {
       dir_ready = false;  // the direction of the gradient step (reflected, or the unit gradient)
-    } else if (RB > 0 && ring > 0) {
+    } else if (RB && ring > 0) {
       // slice si = s is in the ring (gen > s), gen - s slots behind the next free one
       int rslot = gslot - (gen - si);
       if (rslot < 0) rslot += ring;
@@ -1206,7 +1222,7 @@ __global__ void __launch_bounds__(FAM == HIPNS_FAM_LINREG ? HIPNS_WAVE * lr_max_
       const uint32_t own = kw == 0 ? pickblk.x : (kw == 1 ? pickblk.y : (kw == 2 ? pickblk.z : pickblk.w));
       pickw = part_broadcast<LPC>(own, (w >> 2) & (LPC - 1));
     }
-    if (RB > 0 && ring > 0) {
+    if (RB && ring > 0) {
       // a chain about to begin slice s with an empty ring: one draw for every live chain whose ring has
       // room (the same Philox counters as a draw at the slice start, so the directions are unchanged)
       if (__any(alive && need_begin && gen == s)) {
@@ -1256,11 +1272,11 @@ __global__ void __launch_bounds__(FAM == HIPNS_FAM_LINREG ? HIPNS_WAVE * lr_max_
       if constexpr (FAM == HIPNS_FAM_MVN)
         L = lik_mvn<LPC, NJ, true>(up, nj, D, dps, mv, run.log_const, tfm, gscr, gv, alive && need_grad);
       else
-        L = lik_gmm<LPC, NJ, true>(up, nj, D, gm, tfm, gv, alive && need_grad);
+        L = lik_gmm<LPC, NJ, KT, true>(up, nj, D, gm, tfm, gv, alive && need_grad);
     } else if constexpr (FAM == HIPNS_FAM_MVN) {
       L = lik_mvn<LPC, NJ>(up, nj, D, dps, mv, run.log_const, tfm);
     } else if constexpr (FAM == HIPNS_FAM_GMM) {
-      L = lik_gmm<LPC, NJ>(up, nj, D, gm, tfm);
+      L = lik_gmm<LPC, NJ, KT>(up, nj, D, gm, tfm);
     } else {
       L = lik_linreg<LPC, NJ>(up, nj, D, lr, tfm, wave, G, wpb, run.log_const);
     }

@@ -7,7 +7,7 @@ namespace hipns {
 // batched likelihood (Model.forward over a batch) through the same device code:
 // row i of U plays the role of chain i of a single wavefront tile.
 // ---------------------------------------------------------------------------
-template <int LPC, int NJ, int FAM>
+template <int LPC, int NJ, int FAM, int KT>
 __global__ void __launch_bounds__(256) k_loglik(const float* U, int64_t B, double* out, const hipns_run_desc_t* runs,
                                                 hipns_buffers_t Bf, int K, LinRegLds lrd) {
   constexpr int CW = HIPNS_WAVE / LPC;
@@ -16,7 +16,7 @@ __global__ void __launch_bounds__(256) k_loglik(const float* U, int64_t B, doubl
   const int dps = Bf.dps;
   const int D = run.D;
   const int DPr = ((D + 8 * LPC - 1) / (8 * LPC)) * (8 * LPC);
-  const int nj = DPr / LPC;
+  const int nj = NJ == 8 ? 8 : DPr / LPC;
   MvnLds mv;
   GmmLds gm;
   LinRegLds lr = lrd;
@@ -38,7 +38,7 @@ __global__ void __launch_bounds__(256) k_loglik(const float* U, int64_t B, doubl
   if constexpr (FAM == HIPNS_FAM_MVN)
     L = lik_mvn<LPC, NJ>(up, nj, D, dps, mv, run.log_const, tfm);
   else if constexpr (FAM == HIPNS_FAM_GMM)
-    L = lik_gmm<LPC, NJ>(up, nj, D, gm, tfm);
+    L = lik_gmm<LPC, NJ, KT>(up, nj, D, gm, tfm);
   else
     L = lik_linreg<LPC, NJ, false, true>(up, nj, D, lr, tfm, wave, wpb, wpb, run.log_const);
   if (ok && h == 0) out[row] = L;
@@ -46,7 +46,7 @@ __global__ void __launch_bounds__(256) k_loglik(const float* U, int64_t B, doubl
 
 // the same with d logL / dU (MVN and mixture families), the device form the gradient-guided chains
 // use: grad[row * dps + d] for d < D; the wavefront's gradient scratch follows the parameters in LDS
-template <int LPC, int NJ, int FAM>
+template <int LPC, int NJ, int FAM, int KT>
 __global__ void __launch_bounds__(256) k_loglik_grad(const float* U, int64_t B, double* out, float* grad,
                                                      const hipns_run_desc_t* runs, hipns_buffers_t Bf, int K,
                                                      int gscr_off) {
@@ -56,12 +56,12 @@ __global__ void __launch_bounds__(256) k_loglik_grad(const float* U, int64_t B, 
   const int dps = Bf.dps;
   const int D = run.D;
   const int DPr = ((D + 8 * LPC - 1) / (8 * LPC)) * (8 * LPC);
-  const int nj = DPr / LPC;
+  const int nj = NJ == 8 ? 8 : DPr / LPC;
   MvnLds mv;
   GmmLds gm;
   LinRegLds lr{};
   const int wpb = blockDim.x / HIPNS_WAVE;
-  load_params(FAM, Bf.params + run.param_off, dps, D, K, lds, mv, gm, LPC, &lr, wpb, NJ / 8);
+  load_params(FAM, Bf.params + run.param_off, dps, D, K, lds, mv, gm, LPC, &lr, wpb, NJ / 8, true);
   const int wave = threadIdx.x / HIPNS_WAVE;
   const int l = lane_id();
   const int c = l % CW, h = l / CW;
@@ -79,7 +79,7 @@ __global__ void __launch_bounds__(256) k_loglik_grad(const float* U, int64_t B, 
     float* gscr = lds + gscr_off + (size_t)wave * grad_rows(NJ, LPC) * (CW + 1);
     L = lik_mvn<LPC, NJ, true>(up, nj, D, dps, mv, run.log_const, tfm, gscr, g, true);
   } else {
-    L = lik_gmm<LPC, NJ, true>(up, nj, D, gm, tfm, g, true);
+    L = lik_gmm<LPC, NJ, KT, true>(up, nj, D, gm, tfm, g, true);
   }
   if (ok) {
     if (h == 0) out[row] = L;
@@ -98,7 +98,18 @@ static hipError_t launch_loglik_grad_one(const float* U, int64_t B, double* out,
   constexpr int CW = HIPNS_WAVE / LPC;
   int64_t groups = (B + CW - 1) / CW;
   dim3 grid((unsigned)((groups + wpb - 1) / wpb)), block(wpb * HIPNS_WAVE);
-  hipLaunchKernelGGL((k_loglik_grad<LPC, NJ, FAM>), grid, block, lds, s, U, B, out, grad, runs, Bf, K, gscr_off);
+  if constexpr (FAM == HIPNS_FAM_GMM) {
+    const int rows = gmm_rows(K);
+    if (rows == 4)
+      hipLaunchKernelGGL((k_loglik_grad<LPC, NJ, FAM, 4>), grid, block, lds, s, U, B, out, grad, runs, Bf, K, gscr_off);
+    else if (rows == 6)
+      hipLaunchKernelGGL((k_loglik_grad<LPC, NJ, FAM, 6>), grid, block, lds, s, U, B, out, grad, runs, Bf, K, gscr_off);
+    else
+      hipLaunchKernelGGL((k_loglik_grad<LPC, NJ, FAM, HIPNS_MAX_GMM_K>), grid, block, lds, s, U, B, out, grad, runs, Bf, K,
+                         gscr_off);
+  } else {
+    hipLaunchKernelGGL((k_loglik_grad<LPC, NJ, FAM, 1>), grid, block, lds, s, U, B, out, grad, runs, Bf, K, gscr_off);
+  }
   return hipGetLastError();
 }
 
@@ -129,7 +140,17 @@ static hipError_t launch_loglik_one(const float* U, int64_t B, double* out, cons
   constexpr int CW = HIPNS_WAVE / LPC;
   int64_t groups = (B + CW - 1) / CW;
   dim3 grid((unsigned)((groups + wpb - 1) / wpb)), block(wpb * HIPNS_WAVE);
-  hipLaunchKernelGGL((k_loglik<LPC, NJ, FAM>), grid, block, lds, s, U, B, out, runs, Bf, K, lr);
+  if constexpr (FAM == HIPNS_FAM_GMM) {
+    const int rows = gmm_rows(K);
+    if (rows == 4)
+      hipLaunchKernelGGL((k_loglik<LPC, NJ, FAM, 4>), grid, block, lds, s, U, B, out, runs, Bf, K, lr);
+    else if (rows == 6)
+      hipLaunchKernelGGL((k_loglik<LPC, NJ, FAM, 6>), grid, block, lds, s, U, B, out, runs, Bf, K, lr);
+    else
+      hipLaunchKernelGGL((k_loglik<LPC, NJ, FAM, HIPNS_MAX_GMM_K>), grid, block, lds, s, U, B, out, runs, Bf, K, lr);
+  } else {
+    hipLaunchKernelGGL((k_loglik<LPC, NJ, FAM, 1>), grid, block, lds, s, U, B, out, runs, Bf, K, lr);
+  }
   return hipGetLastError();
 }
 
@@ -165,7 +186,7 @@ __global__ void __launch_bounds__(64) k_linreg_stats(const float* U, int64_t B, 
   const int dps = Bf.dps;
   const int D = run.D;
   const int DPr = ((D + 8 * LPC - 1) / (8 * LPC)) * (8 * LPC);
-  const int nj = DPr / LPC;
+  const int nj = NJ == 8 ? 8 : DPr / LPC;
   MvnLds mv;
   GmmLds gm;
   LinRegLds lr = lrd;

@@ -859,3 +859,64 @@ def test_regression_runs_do_not_depend_on_row_split(rows, D, lpc):
     for R, wpb in ((1, 1), (1, 4), (8, 2)):
         for x, y in zip(ref, shells(R, wpb)):
             assert np.array_equal(x, y), (R, wpb)
+
+
+@pytest.mark.parametrize("fam,D,lpc", [("mvn", 10, 2), ("mvn", 33, 4), ("gmm", 5, 4), ("gmm", 21, 8)])
+def test_runs_do_not_depend_on_direction_ring(fam, D, lpc):
+    """The ring of slice directions drawn ahead is as deep as a launch's free LDS allows (8 for one run, 2 or
+    3 among 3000): directions are drawn from the same counters at any depth, so a run's shells are the same
+    bit for bit."""
+    from jaxns_amd.engine import DeviceBatch, RunSpec
+    say(f"direction ring {fam} D={D} lpc={lpc}")
+    model = (mvn_problem(D, seed=D) if fam == "mvn" else gmm_problem(D, seed=D))[0]
+
+    def shells(R, wpb):
+        specs = [RunSpec(model=model, num_live_points=70, num_slices=2 * D, max_samples=700, seed=s) for s in range(R)]
+        b = DeviceBatch(specs, lanes_per_chain=lpc, waves_per_block=wpb)
+        b.init_state()
+        for _ in range(3):
+            b.collect_shell(dict(max_samples=700.0))
+        st = b.states()[0]
+        return [x[:70].cpu().numpy() for x in (b.live_U[st.buf], b.live_logL[st.buf], b.live_evals[st.buf])]
+
+    ref = shells(3000, 1)
+    for R, wpb in ((1, 1), (1, 4), (300, 2)):
+        for x, y in zip(ref, shells(R, wpb)):
+            assert np.array_equal(x, y), (R, wpb)
+
+
+@pytest.mark.parametrize("K", [1, 3, 4, 5, 6, 7, 8])
+@pytest.mark.parametrize("D,lpc", [(3, 2), (30, 4), (50, 8)])
+def test_mixture_component_rows(K, D, lpc):
+    """Mixture kernels have 4, 6 or 8 component rows, those past K of weight zero: the batched likelihood and
+    its gradient against FP64 (1e-5 relative; every gradient component within 2e-5 of its row's largest),
+    and a sampled shell's log L against the FP64 likelihood of its points."""
+    torch = _torch()
+    from jaxns_amd.engine import DeviceBatch, RunSpec
+    say(f"mixture rows K={K} D={D} lpc={lpc}")
+    model, _, means, sig = gmm_problem(D, seed=10 * K + D, K=K)
+    b = DeviceBatch([RunSpec(model=model, num_live_points=64, num_slices=2 * D, max_samples=640, seed=1)],
+                    lanes_per_chain=lpc, waves_per_block=2)
+    rng = np.random.default_rng(K)
+    B = 197
+    U = np.full((B, b.dps), 0.5, np.float32)
+    U[:, :D] = ((means[rng.integers(0, K, B)] + rng.normal(size=(B, D))).clip(-9.9, 9.9) + 10.0) / 20.0
+    Ud = torch.from_numpy(U).cuda()
+    L = [torch.empty(B, dtype=torch.float64, device="cuda") for _ in range(2)]
+    g = torch.zeros((B, b.dps), dtype=torch.float32, device="cuda")
+    args = (ptr(b.runs_dev), b.runs_host, C.byref(b.bufs), C.byref(b.launch), _stream())
+    check(lib().hipns_log_likelihood(ptr(Ud), B, ptr(L[0]), *args))
+    check(lib().hipns_log_likelihood_grad(ptr(Ud), B, ptr(L[1]), ptr(g), *args))
+    u = torch.from_numpy(U[:, :D].astype(np.float64)).requires_grad_(True)
+    ref = model.log_likelihood.torch_log_prob(-10.0 + 20.0 * u)
+    gref, = torch.autograd.grad(ref.sum(), u)
+    ref, gref = ref.detach().numpy(), gref.numpy()
+    for x in L:
+        assert np.max(np.abs(x.cpu().numpy() - ref) / np.maximum(1.0, np.abs(ref))) < 1e-5
+    err = np.abs(g.cpu().numpy()[:, :D] - gref) / np.max(np.abs(gref), axis=1, keepdims=True)
+    assert err.max() < 2e-5, err.max()
+    b.init_state()
+    b.collect_shell(dict(max_samples=640.0))
+    new_U, new_L = b.new_U[:32, :D].cpu().numpy(), b.new_logL[:32].cpu().numpy()
+    f = model.forward_numpy(new_U.astype(np.float64))
+    assert np.max(np.abs(new_L - f) / np.maximum(1.0, np.abs(f))) < 1e-5
