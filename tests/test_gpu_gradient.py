@@ -262,3 +262,39 @@ def test_gradient_slice_whole_runs():
         assert np.all(diff[ph] == 0) and np.all(diff[init] == 0) and np.all(diff[slice_samples] == ns)
         say(f"  run {r}: {m} samples, best log L {c.log_L[:m].max():.4f}, peak {peak:.4f}")
         assert c.log_L[:m].max() > peak - 0.5
+
+
+@pytest.mark.parametrize("fam,D,lpc,wpb", [("mvn", 7, 2, 1), ("mvn", 32, 4, 4), ("mvn", 90, 4, 2), ("gmm", 11, 2, 2),
+                                           ("gmm", 40, 8, 4)])
+def test_batched_likelihood_rows_are_independent(fam, D, lpc, wpb):
+    """One call over more rows than the resident workgroups hold at once (each takes row groups in turn), at
+    16-byte aligned and unaligned row pointers, gives every row what calls of 1000 rows give it, bit for
+    bit, and writes nothing past the last row."""
+    import torch
+    from jaxns_amd.engine import DeviceBatch, RunSpec
+    say(f"batched rows {fam} D={D} lpc={lpc} wpb={wpb}")
+    model = (mvn_problem(D, seed=1) if fam == "mvn" else gmm_problem(D, seed=1))[0]
+    b = DeviceBatch([RunSpec(model=model, num_live_points=64, num_slices=2 * D, max_samples=640)],
+                    lanes_per_chain=lpc, waves_per_block=wpb)
+    B, dps = 200003, b.dps
+    gen = torch.Generator(device="cuda").manual_seed(5)
+    U = torch.rand(B * dps + 1, generator=gen, device="cuda") * 0.98 + 0.01
+
+    def run(shift, chunk):
+        u = U[:B * dps].clone() if shift == 0 else torch.cat([U[:1], U[:B * dps]])
+        L = torch.full((2, B + 1), 7.0, dtype=torch.float64, device="cuda")
+        g = torch.full(((B + 1) * dps + 1,), 7.0, dtype=torch.float32, device="cuda")
+        args = (ptr(b.runs_dev), b.runs_host, C.byref(b.bufs), C.byref(b.launch), _lib.stream_ptr())
+        for i in range(0, B, chunk):
+            n = min(chunk, B - i)
+            up, gp = ptr(u) + 4 * (shift + i * dps), ptr(g) + 4 * (shift + i * dps)
+            check(lib().hipns_log_likelihood(up, n, ptr(L[0]) + 8 * i, *args))
+            check(lib().hipns_log_likelihood_grad(up, n, ptr(L[1]) + 8 * i, gp, *args))
+        return L, g[shift:shift + (B + 1) * dps].view(B + 1, dps)
+
+    L0, g0 = run(0, 1000)
+    for shift in (0, 1):
+        L, g = run(shift, B)
+        assert torch.equal(L, L0) and torch.equal(g, g0), shift
+    assert torch.equal(L0[:, B], torch.full((2,), 7.0, dtype=torch.float64, device="cuda"))
+    assert bool((g0[B] == 7.0).all()) and bool((g0[:B, D:] == 7.0).all())
