@@ -190,7 +190,10 @@ int hipns_collect_shell(const hipns_run_desc_t* runs_dev, hipns_run_state_t* sta
  *  sample   : get_samples -> one UniDimSliceSampler (or UniformSampler) chain per discarded point
  *             (sharded_static.py:88-129, samplers/uni_slice_sampler.py:114-441, bases.py:63-74)
  *  replace  : live[:shell] = new; stable argsort; permute (sharded_static.py:262-279)
- *  register : evidence register + termination flag (sharded_static.py:281-323, termination.py:13-147) */
+ *  register : evidence register + termination flag (sharded_static.py:281-323, termination.py:13-147)
+ * Between sample and replace the live buffer that is not current holds nothing: the regression family's
+ * sampling launch may use its U rows (live_U[1 - buf]) as scratch.  Where the two live_U pointers are the
+ * same, or one is NULL, it does without. */
 int hipns_shell_discard(const hipns_run_desc_t* runs_dev, hipns_run_state_t* states_dev, int32_t R,
                         const hipns_run_desc_t* runs_host, const hipns_buffers_t* bufs, void* stream);
 int hipns_shell_sample(const hipns_run_desc_t* runs_dev, hipns_run_state_t* states_dev, int32_t R,

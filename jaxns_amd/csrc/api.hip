@@ -134,12 +134,14 @@ int num_cus() {
   return v;
 }
 
+// scratch_runs: the launch's run descriptors where its spare live buffers may serve as scratch, else NULL
 int sampler_launch(int mode, const hipns_launch_t* L, const hipns::SampleArgs& A0, int R, int max_chains, int maxD,
-                   int dps, int max_slices, hipStream_t s) {
+                   int dps, int max_slices, hipStream_t s, const hipns_run_desc_t* scratch_runs = nullptr) {
   int lpc = hipns::sampler_lpc(L->family, L->lanes_per_chain, dps, maxD);
   hipns::SampleArgs A = A0;
   int waves = L->waves_per_block, groups = L->waves_per_block;
   bool spread = false;  // regression rows spread over the most wavefronts of few workgroups
+  A.lr_split = 1;
   if (L->family == HIPNS_FAM_LINREG) {
     if (L->lr_terms == 5)
       return fail(HIPNS_EINVAL, "lr_terms 5 (the refinement form) is for hipns_log_likelihood; sampling takes 1, 3 or 4");
@@ -154,20 +156,43 @@ int sampler_launch(int mode, const hipns_launch_t* L, const hipns::SampleArgs& A
     A.lr_panels = lr.panels;
     A.lr_terms = lr.terms;
     // A launch whose workgroups cannot occupy every CU leaves most of the chip idle while each of its
-    // workgroups walks all data rows: it takes the fewest chain groups per workgroup that still fit one
-    // workgroup per CU, and the most wavefronts to share the rows.  A launch of more workgroups keeps the
-    // requested groups, one per wavefront, so that the workgroups of a CU overlap.  4096 x 16, 16 runs of
-    // 512 chains (64 workgroups of four groups, or 256 of one): 17.9 -> 6.5 us per chain step, 1 382 -> 515
-    // ms per batch; a 65536 x 128 shell of 2048 chains (32 workgroups, or 128): 318 -> 194 ms.
-    const int cw = HIPNS_WAVE / lpc;
+    // workgroups walks all data rows.
+    //  - Large data: clusters of 2, 4 or 8 workgroups per set of chain groups, as many as there are CUs for,
+    //    as long as a workgroup's share of the product takes 12 000 cycles of its matrix cores a step (5 us,
+    //    more than the exchange of the sums).  65536 x 128, one shell of 2048 chains: 318 ms without, 194
+    //    with the rule below alone, 46 with clusters of 8.
+    //  - Else the fewest chain groups per workgroup that still fit one workgroup per CU, and the most
+    //    wavefronts to share the rows.  4096 x 16, 16 runs of 512 chains (64 workgroups of four groups, or 256
+    //    of one): 17.9 -> 6.5 us per chain step, 1 382 -> 515 ms per batch.
+    // A launch of more workgroups keeps the requested groups, one per wavefront, so that the workgroups of a
+    // CU overlap.
+    const int cw = HIPNS_WAVE / lpc, nj = hipns::sampler_nj(maxD, lpc), wmax = hipns::lr_max_waves(nj);
     const int64_t per_run = (max_chains + cw - 1) / cw;
-    for (int g = 1; g <= L->waves_per_block; ++g) {
-      if (R * ((per_run + g - 1) / g) <= num_cus()) {
-        groups = g;
-        waves = hipns::lr_max_waves(hipns::sampler_nj(maxD, lpc));
-        if (waves < g) waves = g;
-        spread = true;
-        break;
+    auto blocks_of = [&](int g) { return R * ((per_run + g - 1) / g); };
+    const int tiles = L->lr_ndata / cw, nb = hipns::lr_row_blocks(tiles, lpc, nj);
+    const int64_t cycles = (int64_t)tiles * (nj / 8) * (lr.terms == 4 ? 4 : 3) * groups * (lpc == 2 ? 32 : 16) / 4;
+    if (mode == hipns::MODE_SLICE && lr.terms != 1 && scratch_runs) {
+      int h = hipns::LR_EIGHTHS;
+      while (h > 1 && (blocks_of(groups) * h > num_cus() || cycles / h < 12000 || nb / h < groups)) h /= 2;
+      for (int r = 0; h > 1 && r < R; ++r) {
+        const hipns_run_desc_t& d = scratch_runs[r];
+        const int64_t clusters = (d.shell + groups * cw - 1) / (groups * cw);
+        if (clusters * (int64_t)hipns::lr_cluster_bytes(groups, cw) > (int64_t)d.N * dps * (int64_t)sizeof(float)) h = 1;
+      }
+      A.lr_split = h;
+    }
+    if (A.lr_split > 1) {
+      waves = nb / A.lr_split < wmax ? nb / A.lr_split : wmax;
+      if (waves < groups) waves = groups;
+      spread = true;
+    } else {
+      for (int g = 1; g <= L->waves_per_block; ++g) {
+        if (blocks_of(g) <= num_cus()) {
+          groups = g;
+          waves = wmax < g ? g : wmax;
+          spread = true;
+          break;
+        }
       }
     }
   }
@@ -201,7 +226,9 @@ int sampler_launch(int mode, const hipns_launch_t* L, const hipns::SampleArgs& A
   }
   A.dir_ring = ring;
   if (spread) {
-    const size_t off = (lds / sizeof(float) + 3) / 4 * 4, end = (off + (size_t)L->lr_ndata) * sizeof(float);
+    // (a cluster's workgroup takes whole row blocks: at most one row more per block than its share)
+    const size_t rows = (size_t)L->lr_ndata / A.lr_split + (A.lr_split > 1 ? 64 : 0);
+    const size_t off = (lds / sizeof(float) + 3) / 4 * 4, end = (off + rows) * sizeof(float);
     if ((int64_t)end <= max_lds_bytes()) {
       A.lr_r0_off = (int32_t)off;
       lds = end;
@@ -436,7 +463,9 @@ int hipns_shell_sample(const hipns_run_desc_t* runs_dev, hipns_run_state_t* stat
     return fail(HIPNS_EINVAL, "gradient slice shells (sampler %d) run the MVN and mixture families; gradient-guided "
                               "regression shells step through hipns_ext_step", sampler);
   const int mode = sampler == 1 ? hipns::MODE_UNIF : (sampler >= 2 ? hipns::MODE_GSLICE : hipns::MODE_SLICE);
-  return sampler_launch(mode, launch, A, R, maxS, maxD, bufs->dps, max_slices, as_stream(stream));
+  const bool spare = bufs->live_U[0] && bufs->live_U[1] && bufs->live_U[0] != bufs->live_U[1];
+  return sampler_launch(mode, launch, A, R, maxS, maxD, bufs->dps, max_slices, as_stream(stream),
+                        spare ? runs_host : nullptr);
 }
 
 int hipns_shell_replace(const hipns_run_desc_t* runs_dev, hipns_run_state_t* states_dev, int32_t R,

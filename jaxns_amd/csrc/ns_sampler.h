@@ -32,6 +32,7 @@ struct SampleArgs {
   int32_t lr_panels;
   int32_t lr_terms;
   int32_t lr_groups;  // chain groups per workgroup (the other wavefronts only take rows)
+  int32_t lr_split;   // workgroups per cluster (1: none)
   int32_t lr_r0_off;  // LDS float offset of r0 (0: read from global memory)
   int32_t ring_off;   // LDS float offset of the direction rings (16-byte aligned)
   // injected-draw mode
@@ -60,8 +61,11 @@ struct LinRegLds {
   void* bops;          // [G][NG][3][64] B operands (8 bf16 each) published by every chain group
   double* partial;     // [2][G][row blocks][CW] partial sums (|r|^2, then y^T r)
   const float* r0;     // [npad] r0 = y - X w0 (computed in FP64, zero on padding rows)
-  float* r0l;          // r0 in LDS where `staged`
+  float* r0l;          // r0 in LDS where `staged` (the rows that this workgroup takes)
   bool staged;
+  int split, slice;    // workgroups of the cluster and this one's index (1, 0: no cluster)
+  uint32_t* flags;     // [G][8] step counters of the cluster
+  double* exchange;    // [2][G][8][CW] sums of the eighths of the rows
   const uint16_t* xh;  // [panels][npad][16] bf16 hi part of the column-scaled X
   const uint16_t* xl;  // [panels][npad][16] bf16 lo part (X - hi)
   const float* y;      // [npad] targets (zero on padding rows), read by the adjoint statistics only
@@ -116,10 +120,22 @@ __host__ __device__ constexpr int gmm_rows(int K) { return K <= 4 ? 4 : (K <= 6 
 // 8 slots need more than the 256 VGPRs that two wavefronts per SIMD leave each), and the fixed blocks that
 // the data rows are summed in, whatever the number of wavefronts that share them.  A block boundary costs a
 // cross-lane FP64 sum per group, so short data take 8 (one per wavefront of a full workgroup); from 1024
-// tiles on, 32 blocks (16 of the twice as wide ones at 2 lanes per chain: the same LDS) of at least 32
-// tiles.
+// tiles on, 32 blocks (16 for the widest instance at 2 lanes per chain, whose LDS they would fill) of at
+// least 32 tiles.
 __host__ __device__ constexpr int lr_max_waves(int nj) { return nj <= 8 ? 8 : 4; }
-__host__ __device__ inline int lr_row_blocks(int tiles, int lpc) { return tiles < 1024 ? 8 : (lpc == 2 ? 16 : 32); }
+__host__ __device__ inline int lr_row_blocks(int tiles, int lpc, int nj) {
+  return tiles < 1024 ? 8 : (lpc == 2 && nj > 16 ? 16 : 32);
+}
+
+// Clusters: a launch of large data and few chain groups runs H workgroups on the same chain groups, each
+// taking 1/H of the row blocks (cut at eighths) and exchanging the sums of its eighths every step through
+// device memory.  Scratch of a cluster of G groups of cw chains: [join word, step counters: 256 B]
+// [2 parities][G][8][cw] doubles.
+constexpr int LR_EIGHTHS = 8;
+constexpr size_t LR_CLUSTER_HEAD = 256;
+__host__ __device__ inline size_t lr_cluster_bytes(int G, int cw) {
+  return LR_CLUSTER_HEAD + (size_t)2 * G * LR_EIGHTHS * cw * sizeof(double);
+}
 
 // floats of dynamic LDS one sampler block needs (layout of load_params in ns_sampler_impl.h); npad: the
 // regression family's padded data rows, sums: row sums kept per point (2 for the adjoint statistics)
@@ -128,7 +144,7 @@ inline size_t sampler_lds_floats(int fam, int dps, int D, int K, int lpc, int G,
   if (fam == HIPNS_FAM_LINREG) {
     const size_t NG = (size_t)sampler_nj(D, lpc) / 8;
     const size_t CW = (size_t)(64 / lpc);
-    return (size_t)4 * dps + 4 + (size_t)G * NG * 3 * 64 * 4 + (size_t)sums * G * lr_row_blocks((int)(npad / CW), lpc) * CW * 2;
+    return (size_t)4 * dps + 4 + (size_t)G * NG * 3 * 64 * 4 + (size_t)sums * G * lr_row_blocks((int)(npad / CW), lpc, (int)NG * 8) * CW * 2;
   }
   if (fam == HIPNS_FAM_MVN) {
     const int nj = sampler_nj(D, lpc);
@@ -170,6 +186,7 @@ hipError_t launch_loglik(const float* U, int64_t B, double* out, const hipns_run
 }  // namespace hipns
 
 namespace hipns {
+__global__ void k_lr_clear(const hipns_run_desc_t* runs, const hipns_run_state_t* states, hipns_buffers_t B, int G, int cw);
 hipError_t launch_sampler_slice(const SampleArgs& A, int R, int max_chains, const hipns_launch_t& L, int dmax,
                                 size_t lds_bytes, hipStream_t s);
 hipError_t launch_sampler_unif(const SampleArgs& A, int R, int max_chains, const hipns_launch_t& L, int dmax,

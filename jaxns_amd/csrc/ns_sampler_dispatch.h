@@ -16,6 +16,7 @@ inline hipError_t launch_rows(const SampleArgs& A, int R, int max_chains, int wp
   int groups = (max_chains + CW - 1) / CW;
   int bx = (groups + per_block - 1) / per_block;
   if (bx < 1) bx = 1;
+  if (FAM == HIPNS_FAM_LINREG && MODE == MODE_SLICE) bx *= A.lr_split;
   dim3 grid(bx, R), block(wpb * HIPNS_WAVE);
   hipLaunchKernelGGL((k_sample<LPC, NJ, FAM, MODE, KT>), grid, block, lds_bytes, s, A);
   return hipGetLastError();

@@ -117,7 +117,8 @@ __device__ __forceinline__ double chain_sum_d(double v) {
 // takes its share of the data-row tiles and multiplies every row tile it loads against all G groups'
 // operands, so X is read once per step per workgroup instead of once per chain group.  The rows are cut
 // into lr_row_blocks fixed blocks, a wavefront takes whole blocks, and the blocks' sums meet in block
-// order, so a point's value depends on the data alone and not on G, W or the batch.  Each product is BF16x3
+// order, eighth of the rows by eighth, so a point's value depends on the data alone and not on G, W, the
+// cluster or the batch.  Each product is BF16x3
 // (hi.hi + hi.lo + lo.hi, FP32 accumulate; terms == 4 adds hi times the third bf16 part of w - w0,
 // which removes the error of the 16-bit weight split that every row shares): LPC=2 uses
 // v_mfma_f32_32x32x16_bf16 over 32-row tiles, LPC=4 v_mfma_f32_16x16x32_bf16 over 16-row tiles.
@@ -125,6 +126,29 @@ __device__ __forceinline__ double chain_sum_d(double v) {
 // of a tile are summed in FP32 and accumulated in FP64.  All W wavefronts must call this together (two
 // workgroup barriers).
 constexpr int LR_MAX_G = 4;
+
+// Forms a cluster: true once all H workgroups have joined, and then each of them is running and stays so, so
+// that the waits of every step end.  A workgroup that waits too long for the others (the GPU is busy with
+// other work) breaks the cluster: the join word goes to exactly one of "all joined" and "broken", later
+// workgroups see it, and workgroup 0 then takes all rows by itself.  One thread calls this.
+constexpr uint32_t LR_BROKEN = 0x80000000u;
+constexpr long long LR_JOIN_TICKS = 20000;  // of the 100 MHz constant clock
+__device__ inline bool lr_join(uint32_t* word, uint32_t H) {
+  const uint32_t before = __hip_atomic_fetch_add(word, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  if (before & LR_BROKEN) return false;
+  if (before + 1u == H) return true;
+  const long long t0 = wall_clock64();
+  for (;;) {
+    uint32_t v = __hip_atomic_load(word, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if (v & LR_BROKEN) return false;
+    if (v == H) return true;
+    if (wall_clock64() - t0 > LR_JOIN_TICKS &&
+        __hip_atomic_compare_exchange_strong(word, &v, v | LR_BROKEN, __ATOMIC_RELAXED, __ATOMIC_RELAXED,
+                                             __HIP_MEMORY_SCOPE_AGENT))
+      return false;
+    __builtin_amdgcn_s_sleep(4);
+  }
+}
 
 template <int LPC>
 __device__ __forceinline__ const uint16_t* lr_panel_ptr(const uint16_t* x, int npad, int gg, int row, int h) {
@@ -311,7 +335,7 @@ __device__ __forceinline__ void lr_bf16_tiles(const LinRegLds& P, const bf16x8_t
     }
   };
   if constexpr (R0L) {
-    constexpr int DEPTH = NG == 1 ? 4 : 2;
+    constexpr int DEPTH = NG == 1 && !(LPC == 2 && GG > 2) ? 4 : 2;
     bf16x8_t xh[DEPTH][NG], xl[DEPTH][NG];
 #pragma unroll
     for (int i = 0; i < DEPTH; ++i)
@@ -364,7 +388,7 @@ __device__ __forceinline__ void lr_bf16_tiles(const LinRegLds& P, const bf16x8_t
 template <int LPC, int NJ, bool STATS = false, bool F64T = false>
 __device__ __forceinline__ double lik_linreg(const float (&up)[NJ], int nj, int D, const LinRegLds& P, uint32_t tfm,
                                              int g, int G, int W, double log_const, double* rss = nullptr,
-                                             double* yr = nullptr) {
+                                             double* yr = nullptr, int step = 0) {
   constexpr int CW = HIPNS_WAVE / LPC;
   constexpr int NG = NJ / 8;  // k-groups of 8 owned dims
   const int l = lane_id();
@@ -431,12 +455,14 @@ __device__ __forceinline__ double lik_linreg(const float (&up)[NJ], int nj, int 
   }
   __syncthreads();
   const int tiles = P.npad / CW;
-  const int NB = lr_row_blocks(tiles, LPC);
+  const int NB = lr_row_blocks(tiles, LPC, NJ);
   constexpr int NR = (LPC == 2) ? 16 : 4;  // accumulator rows per lane
   // rows of tile tl held by this lane (the MFMA output layout)
   auto tile_row = [&](int tl, int i) { return (LPC == 2) ? tl * 32 + 8 * (i >> 2) + 4 * h + (i & 3) : tl * 16 + 4 * h + i; };
   // this wavefront's row blocks, each summed by itself (wavefront-uniform ranges: scalar loop control)
-  const int b0 = __builtin_amdgcn_readfirstlane(NB * g / W), b1 = __builtin_amdgcn_readfirstlane(NB * (g + 1) / W);
+  const int c0 = NB * P.slice / P.split, cn = NB * (P.slice + 1) / P.split - c0;  // the workgroup's blocks
+  const int b0 = __builtin_amdgcn_readfirstlane(c0 + cn * g / W);
+  const int b1 = __builtin_amdgcn_readfirstlane(c0 + cn * (g + 1) / W);
   for (int blk = b0; blk < b1; ++blk) {
     const int t0 = (int)(((long long)tiles * blk) / NB), t1 = (int)(((long long)tiles * (blk + 1)) / NB);
     double ss[LR_MAX_G], sy[LR_MAX_G];
@@ -539,9 +565,44 @@ __device__ __forceinline__ double lik_linreg(const float (&up)[NJ], int nj, int 
   __syncthreads();
   double tot = 0.0, toty = 0.0;
   if (g < G) {
-    for (int k = 0; k < NB; ++k) {
-      tot += P.partial[(g * NB + k) * CW + m];
-      if (STATS) toty += P.partial[((G + g) * NB + k) * CW + m];
+    // sums of the eighths of the rows, in order, and then their sum, in order
+    const int per = NB / LR_EIGHTHS;
+    auto eighth = [&](int row0, int k) {
+      double v = 0.0;
+      for (int j = k * per; j < (k + 1) * per; ++j) v += P.partial[(row0 * NB + j) * CW + m];
+      return v;
+    };
+    if (STATS || P.split == 1) {
+      for (int k = 0; k < LR_EIGHTHS; ++k) {
+        tot += eighth(g, k);
+        if (STATS) toty += eighth(G + g, k);
+      }
+    } else {
+      // exchange with the cluster's other workgroups: this one's eighths out, its step counter after them,
+      // then every workgroup's counter is awaited and all eighths come in.  The buffers alternate: a
+      // workgroup that writes step w + 2 has seen this one's counter of w + 1, which follows its reads of w.
+      double* ex = P.exchange + (size_t)((step & 1) * G + g) * LR_EIGHTHS * CW + m;
+      uint32_t* flags = P.flags + g * LR_EIGHTHS;
+      const uint32_t now = (uint32_t)step + 1u;
+      for (int k = LR_EIGHTHS * P.slice / P.split; k < LR_EIGHTHS * (P.slice + 1) / P.split; ++k) {
+        const double v = eighth(g, k);
+        if (h == 0) __hip_atomic_store(ex + k * CW, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      }
+      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
+      if (l == 0) __hip_atomic_store(flags + P.slice, now, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      for (;;) {
+        const uint32_t f =
+            l < P.split ? __hip_atomic_load(flags + l, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : now;
+        if (__all(f >= now)) break;
+        __builtin_amdgcn_s_sleep(1);
+      }
+      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
+      double v[LR_EIGHTHS];
+#pragma unroll
+      for (int k = 0; k < LR_EIGHTHS; ++k)
+        v[k] = __hip_atomic_load(ex + k * CW, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+#pragma unroll
+      for (int k = 0; k < LR_EIGHTHS; ++k) tot += v[k];
     }
   }
   if constexpr (STATS) {
@@ -1060,8 +1121,28 @@ __global__ void __launch_bounds__(FAM == HIPNS_FAM_LINREG ? HIPNS_WAVE * lr_max_
   const int c = l % CW;
   const int h = l / CW;
   const int nchains = (MODE == MODE_INIT) ? run.N : ((MODE == MODE_INJ) ? A.inj_C : run.shell);
-  const int chain0 = (blockIdx.x * G + wave) * CW;
-  if (blockIdx.x * G * CW >= nchains) return;  // whole block idle
+  // (clusters: consecutive workgroups share their chains, so that one slice of the rows stays on one XCD)
+  constexpr bool CLUSTER = COOP && MODE == MODE_SLICE;
+  int split = CLUSTER ? A.lr_split : 1;
+  const int block = (int)blockIdx.x / split, slice = (int)blockIdx.x % split;
+  const int chain0 = (block * G + wave) * CW;
+  if (block * G * CW >= nchains) return;  // whole block idle
+  unsigned char* cluster = nullptr;
+  if constexpr (CLUSTER) {
+    if (split > 1) {
+      // the live buffer that is not current is free until the replacement rewrites it
+      cluster = (unsigned char*)(A.B.live_U[1 - st->buf] + run.live_off * A.B.dps) + block * lr_cluster_bytes(G, CW);
+      if (threadIdx.x == 0) ((int*)lds)[0] = lr_join((uint32_t*)cluster, (uint32_t)split);
+      __syncthreads();
+      const bool joined = ((int*)lds)[0] != 0;
+      __syncthreads();
+      if (!joined) {
+        if (slice > 0) return;
+        split = 1;
+      }
+    }
+  }
+  const bool writer = slice == 0;
   const int dps = A.B.dps;
   const int D = run.D;
   const int DPr = ((D + 8 * LPC - 1) / (8 * LPC)) * (8 * LPC);
@@ -1075,11 +1156,19 @@ __global__ void __launch_bounds__(FAM == HIPNS_FAM_LINREG ? HIPNS_WAVE * lr_max_
               MODE == MODE_GSLICE);
   if (COOP) {
     lr.r0 = A.lr_r0;
-    lr.r0l = lds + A.lr_r0_off;
-    lr.staged = A.lr_r0_off > 0;
+    lr.split = split;
+    lr.slice = split > 1 ? slice : 0;
+    lr.flags = (uint32_t*)(cluster + 64);
+    lr.exchange = (double*)(cluster + LR_CLUSTER_HEAD);
+    // r0 of this workgroup's rows, in place before the first step's barriers (a workgroup left alone by a
+    // broken cluster has room for its own part only, and reads r0 from memory)
+    const int tiles = A.lr_npad / CW, NB = lr_row_blocks(tiles, LPC, NJ);
+    const int row0 = (int)((long long)tiles * (NB * lr.slice / split) / NB) * CW;
+    const int row1 = (int)((long long)tiles * (NB * (lr.slice + 1) / split) / NB) * CW;
+    lr.staged = A.lr_r0_off > 0 && split == A.lr_split;
+    lr.r0l = lds + A.lr_r0_off - row0;
     if (lr.staged) {
-      // in place before the first step's barriers
-      for (int i = threadIdx.x; i < A.lr_npad; i += blockDim.x) lr.r0l[i] = A.lr_r0[i];
+      for (int i = row0 + threadIdx.x; i < row1; i += blockDim.x) lr.r0l[i] = A.lr_r0[i];
     }
     lr.xh = A.lr_xh;
     lr.xl = A.lr_xl;
@@ -1278,7 +1367,7 @@ __global__ void __launch_bounds__(FAM == HIPNS_FAM_LINREG ? HIPNS_WAVE * lr_max_
     } else if constexpr (FAM == HIPNS_FAM_GMM) {
       L = lik_gmm<LPC, NJ, KT>(up, nj, D, gm, tfm);
     } else {
-      L = lik_linreg<LPC, NJ>(up, nj, D, lr, tfm, wave, G, wpb, run.log_const);
+      L = lik_linreg<LPC, NJ>(up, nj, D, lr, tfm, wave, G, wpb, run.log_const, nullptr, nullptr, w);
     }
 
     if (alive) {
@@ -1404,7 +1493,8 @@ __global__ void __launch_bounds__(FAM == HIPNS_FAM_LINREG ? HIPNS_WAVE * lr_max_
       }
     }
   }
-  if (cap_hits > 0 && h == 0 && MODE != MODE_INJ) {
+  // (the workgroups of a cluster hold the same chains and write the same values; counts are added once)
+  if (cap_hits > 0 && h == 0 && MODE != MODE_INJ && writer) {
     atomicAdd((unsigned long long*)&st->cap_hits, (unsigned long long)cap_hits);
     atomicOr(&st->flags, 1);
   }

@@ -55,6 +55,8 @@ __global__ void __launch_bounds__(256) k_loglik(const float* U, int64_t B, doubl
   MvnLds mv;
   GmmLds gm;
   LinRegLds lr = lrd;
+  lr.split = 1;
+  lr.slice = 0;
   const int wpb = blockDim.x / HIPNS_WAVE;
   load_params(FAM, Bf.params + run.param_off, dps, D, K, lds, mv, gm, LPC, &lr, wpb, NJ / 8);
   const int wave = threadIdx.x / HIPNS_WAVE;
@@ -238,6 +240,8 @@ __global__ void __launch_bounds__(64) k_linreg_stats(const float* U, int64_t B, 
   MvnLds mv;
   GmmLds gm;
   LinRegLds lr = lrd;
+  lr.split = 1;
+  lr.slice = 0;
   load_params(HIPNS_FAM_LINREG, Bf.params + run.param_off, dps, D, 1, lds, mv, gm, LPC, &lr, 1, NJ / 8);
   const int l = lane_id();
   const int c = l % CW, h = l / CW;

@@ -920,3 +920,29 @@ def test_mixture_component_rows(K, D, lpc):
     new_U, new_L = b.new_U[:32, :D].cpu().numpy(), b.new_logL[:32].cpu().numpy()
     f = model.forward_numpy(new_U.astype(np.float64))
     assert np.max(np.abs(new_L - f) / np.maximum(1.0, np.abs(f))) < 1e-5
+
+
+def test_concurrent_regression_clusters_match_sequential():
+    """Launches of several workgroups per set of chains (large data, few chains) on streams of their own: a
+    cluster whose workgroups do not all become resident in time gives its rows to one of them, so the
+    launches end whatever else holds the GPU, with the same samples as one batch after the other."""
+    from jaxns_amd.engine import DeviceBatch, RunSpec, run_concurrent
+    say("concurrent regression clusters")
+    model, _, _ = linreg_problem(40000, 9, seed=4, sigma=0.4, tau=1.0)
+    term = dict(max_samples=1500.0)
+
+    def batches():
+        return [DeviceBatch([RunSpec(model=model, num_live_points=300, num_slices=9, max_samples=3000, seed=10 * g + s)
+                             for s in range(g + 1)], lanes_per_chain=2, waves_per_block=4) for g in range(3)]
+
+    one, other = batches(), batches()
+    for b in one:
+        b.run(term, graph_iters=2)
+    run_concurrent(other, term, graph_iters=2)
+    for a, b in zip(one, other):
+        for r in range(a.R):
+            x, y = a.sample_collection(r), b.sample_collection(r)
+            n = int(a.states()[r].num_samples)
+            assert n == int(b.states()[r].num_samples) and n >= 1500
+            assert np.array_equal(x.log_L[:n], y.log_L[:n]) and np.array_equal(x.U_samples[:n], y.U_samples[:n])
+            assert np.array_equal(x.num_likelihood_evaluations[:n], y.num_likelihood_evaluations[:n])
