@@ -102,6 +102,29 @@ def slice_sampler_code(gradient_guided: bool, gradient_slice: bool) -> int:
     return 2 if gradient_guided else 0
 
 
+class _HostFlags:
+    """Device flags read by the host without holding up the stream: post() queues a copy to pinned memory
+    on the current stream, all_posted() / any_posted() waits for the last posted copy."""
+
+    def __init__(self, dev):
+        torch = _torch()
+        self.dev = dev
+        self.host = torch.empty(dev.shape, dtype=dev.dtype, pin_memory=True)
+        self.event = torch.cuda.Event()
+
+    def post(self, dev=None):
+        self.host.copy_(self.dev if dev is None else dev, non_blocking=True)
+        self.event.record()
+
+    def all_posted(self) -> bool:
+        self.event.synchronize()
+        return bool(np.all(self.host.numpy()))
+
+    def any_posted(self) -> bool:
+        self.event.synchronize()
+        return bool(np.any(self.host.numpy()))
+
+
 class DeviceBatch:
     """R independent runs sharing one likelihood family, advanced together."""
 
@@ -331,24 +354,33 @@ class DeviceBatch:
     def _ext_steps(self, mode: int, stream=None):
         """Step every chain until none runs, evaluating each step's proposals with the callable
         (Model.forward over the batch)."""
+        torch = _torch()
         s = self._s(stream)
         self.ext_flags.zero_()
+        # one step ahead of the flags (rows of finished chains hold 0.5 and stay as they are), except where
+        # they choose what to evaluate
+        flags = None if mode == 4 else _HostFlags(self.ext_flags.any())
         w = 0
         while True:
             check(lib().hipns_ext_step(ptr(self.runs_dev), ptr(self.states_dev), self.R, self.runs_host,
                                        C.byref(self.bufs), C.byref(self.launch), C.byref(self.ext), mode, w, s),
                   "hipns_ext_step")
-            if not bool((self.ext_flags & 1).any()):
-                break
-            if mode == 4 and bool((self.ext_flags & 8).any()):
-                torch = _torch()
-                with torch.enable_grad():
-                    U = self.ext_prop_U.detach().clone().requires_grad_(True)
-                    L = self.ext_like(U)
-                    g, = torch.autograd.grad(torch.where(torch.isfinite(L), L, torch.zeros_like(L)).sum(), U)
-                self.ext_prop_logL.copy_(L.detach())
-                self.ext_grad.copy_(torch.nan_to_num(g, nan=0.0, posinf=0.0, neginf=0.0))
+            if flags is None:
+                if not bool((self.ext_flags & 1).any()):
+                    break
+                if bool((self.ext_flags & 8).any()):
+                    with torch.enable_grad():
+                        U = self.ext_prop_U.detach().clone().requires_grad_(True)
+                        L = self.ext_like(U)
+                        g, = torch.autograd.grad(torch.where(torch.isfinite(L), L, torch.zeros_like(L)).sum(), U)
+                    self.ext_prop_logL.copy_(L.detach())
+                    self.ext_grad.copy_(torch.nan_to_num(g, nan=0.0, posinf=0.0, neginf=0.0))
+                else:
+                    self.ext_prop_logL.copy_(self.ext_like(self.ext_prop_U))
             else:
+                if w > 0 and not flags.any_posted():
+                    break
+                flags.post(self.ext_flags.any())
                 self.ext_prop_logL.copy_(self.ext_like(self.ext_prop_U))
             w += 1
 
@@ -588,7 +620,7 @@ class DeviceBatch:
                 it += graph_iters
                 if getattr(self, "_verbose", False):
                     print(self.report(0), flush=True)
-        else:
+        elif self.external or self.refine_fp32 or getattr(self, "_verbose", False):
             while it < max_iterations:
                 if np.all(self.done_flags()):
                     break
@@ -596,6 +628,22 @@ class DeviceBatch:
                 it += 1
                 if getattr(self, "_verbose", False):
                     print(self.report(0), flush=True)
+        else:
+            # one shell ahead of the done flags: a shell is queued while the host waits for the flags of the
+            # shell before it (a queued shell whose runs are all done does nothing on the device)
+            current = torch.cuda.current_stream()
+            s = stream if stream is not None else current
+            s.wait_stream(current)
+            with torch.cuda.stream(s):
+                flags = _HostFlags(self.states_dev.view(torch.int32).view(self.R, -1)[:, RunState.done.offset // 4])
+                flags.post()
+                while it < max_iterations:
+                    self.collect_shell(term, s)
+                    it += 1
+                    if flags.all_posted():
+                        break
+                    flags.post()
+            current.wait_stream(s)
 
     def _get_graph(self, term, iters):
         torch = _torch()
@@ -696,21 +744,48 @@ class DeviceBatch:
         s = self._s(stream)
         logL = self.samp_logL[off:off + L]
         sender = self.samp_sender[off:off + L]
-        si = torch.empty(L, dtype=torch.int64, device=dev)
-        nl = torch.empty(L, dtype=torch.int64, device=dev)
+        # every output in one block of 8-byte words, copied to the host at once: [final 8][H 4][phantoms 1]
+        # [sample indices][live-point counts] and, with full, [log L][per-sample 8][evals][log dp][log post]
+        # [U][X]
+        model, D = spec.model, spec.model.U_ndims
+        sizes = dict(fin=8, H=4, phantom=1, si=L, nl=L, lL=L)
+        if full:
+            sizes.update(per8=8 * L, ev=L, log_dp=L, lpost=L, U=L * D, X=0 if model.dynamic_prior else L * D)
+        block = torch.empty(sum(-(-n // 32) * 32 for n in sizes.values()), dtype=torch.float64, device=dev)
+        at, view = {}, {}
+        o = 0
+        for k, n in sizes.items():
+            at[k] = slice(o, o + n)
+            view[k] = block[o:o + n]
+            o += -(-n // 32) * 32  # (256-byte starts)
+        si, nl = view["si"].view(torch.int64), view["nl"].view(torch.int64)
         ws = torch.empty(int(lib().hipns_count_crossed_edges_workspace_size(L)), dtype=torch.uint8, device=dev)
         check(lib().hipns_count_crossed_edges(ptr(sender), ptr(logL), L, stop, ptr(si), ptr(nl), ptr(ws), ws.numel(),
                                               s), "hipns_count_crossed_edges")
-        lL = logL.index_select(0, si)
+        lL = torch.index_select(logL, 0, si, out=view["lL"])
         nld = nl.to(torch.float64)
-        per8 = torch.empty((8, L), dtype=torch.float64, device=dev)
-        fin8 = torch.empty(8, dtype=torch.float64, device=dev)
+        per8 = view["per8"].view(8, L) if full else None
         ws2 = torch.empty(int(lib().hipns_evidence_scan_workspace_size(L)), dtype=torch.uint8, device=dev)
-        check(lib().hipns_evidence_scan(ptr(lL), ptr(nld), L, stop, ptr(per8), ptr(fin8), ptr(ws2), ws2.numel(), s),
-              "hipns_evidence_scan")
-        fin = fin8.cpu().numpy()
+        check(lib().hipns_evidence_scan(ptr(lL), ptr(nld), L, stop, ptr(per8), ptr(view["fin"]), ptr(ws2), ws2.numel(),
+                                        s), "hipns_evidence_scan")
+        view["phantom"].view(torch.int64).copy_(self.samp_phantom[off:off + M].sum(dtype=torch.int64))
+        if full:
+            view["ev"].view(torch.int64).copy_(self.samp_evals[off:off + L].index_select(0, si))
+            ws3 = torch.empty(int(lib().hipns_results_finals_workspace_size(L)), dtype=torch.uint8, device=dev)
+            # (H of log Z = 0 here; log Z is added on the host)
+            check(lib().hipns_results_finals(ptr(per8[6]), ptr(lL), ptr(per8[1]), L, 0.0, ptr(view["log_dp"]),
+                                             ptr(view["H"]), ptr(ws3), ws3.numel(), s), "hipns_results_finals")
+            args = (ptr(self.samp_U) + off * self.dps * 4, self.dps, ptr(si), M, L, D, *self._prior_program_dev(model))
+            if model.dynamic_prior:
+                # a prior program that depends on earlier prior values: the model's generator forms X
+                check(lib().hipns_prior_finals(*args, None, ptr(view["U"]), None, None, s), "hipns_prior_finals")
+            else:
+                check(lib().hipns_prior_finals(*args, ptr(lL), ptr(view["U"]), ptr(view["X"]), ptr(view["lpost"]), s),
+                      "hipns_prior_finals")
+        host = block.cpu().numpy()
+        fin = host[at["fin"]]
         log_Z_mean, log_Z_var = _linear_to_log_stats(fin[3], fin[5])
-        total_phantom = int(self.samp_phantom[off:off + M].to(torch.int64).sum().item())
+        total_phantom = int(host[at["phantom"]].view(np.int64)[0])
         pf = total_phantom / M
         k = pf / (1.0 - pf)
         log_Z_uncert = math.sqrt(log_Z_var) * math.sqrt(1.0 + k)
@@ -721,37 +796,20 @@ class DeviceBatch:
         if self.refine_fp32:
             out["refined_below_contour"] = int(self.refine_below[r].item())
         if full:
-            model = spec.model
-            D = model.U_ndims
-            ev = self.samp_evals[off:off + L].index_select(0, si)
-            log_dp = torch.empty(L, dtype=torch.float64, device=dev)
-            H = torch.empty(4, dtype=torch.float64, device=dev)
-            ws3 = torch.empty(int(lib().hipns_results_finals_workspace_size(L)), dtype=torch.uint8, device=dev)
-            check(lib().hipns_results_finals(ptr(per8[6]), ptr(lL), ptr(per8[1]), L, float(log_Z_mean), ptr(log_dp),
-                                             ptr(H), ptr(ws3), ws3.numel(), s), "hipns_results_finals")
-            U = torch.empty((L, D), dtype=torch.float64, device=dev)
+            Uh = host[at["U"]].reshape(L, D)
+            lLh = host[at["lL"]]
             if model.dynamic_prior:
-                # a prior program that depends on earlier prior values: the model's generator forms X
-                check(lib().hipns_prior_finals(ptr(self.samp_U) + off * self.dps * 4, self.dps, ptr(si), M, L, D,
-                                               *self._prior_program_dev(model), None, ptr(U), None, None, s),
-                      "hipns_prior_finals")
-                Uh = U.cpu().numpy()
-                X = None
-                log_post = lL.cpu().numpy() + model.log_prob_prior_numpy(Uh)
+                X, log_post = None, lLh + model.log_prob_prior_numpy(Uh)
             else:
-                X = torch.empty((L, D), dtype=torch.float64, device=dev)
-                lpost = torch.empty(L, dtype=torch.float64, device=dev)
-                check(lib().hipns_prior_finals(ptr(self.samp_U) + off * self.dps * 4, self.dps, ptr(si), M, L, D,
-                                               *self._prior_program_dev(model), ptr(lL), ptr(U), ptr(X), ptr(lpost),
-                                               s), "hipns_prior_finals")
-                Uh = U.cpu().numpy()
-                X = X.cpu().numpy()
-                log_post = lpost.cpu().numpy()
-            Hh = H.cpu().numpy()
-            out.update(samples_indices=si.cpu().numpy(), num_live_points=nl.cpu().numpy(), log_L=lL.cpu().numpy(),
-                       per8=per8.cpu().numpy(), evals=ev.to(torch.int64).cpu().numpy(), U=Uh, X=X,
-                       log_dp=log_dp.cpu().numpy(), H_unstable=float(Hh[0]), H_stable=float(Hh[1]),
-                       H_mean=float(Hh[2]), log_posterior_density=log_post)
+                X, log_post = host[at["X"]].reshape(L, D), host[at["lpost"]]
+            Hh = host[at["H"]]
+            # H unstable = log Z - sum dp log L, the stable form where that is not finite
+            # (sharded_static.py:728-737)
+            H_unstable, H_stable = float(Hh[0]) + float(log_Z_mean), float(Hh[1])
+            out.update(samples_indices=host[at["si"]].view(np.int64), num_live_points=host[at["nl"]].view(np.int64),
+                       log_L=lLh, per8=host[at["per8"]].reshape(8, L), evals=host[at["ev"]].view(np.int64), U=Uh, X=X,
+                       log_dp=host[at["log_dp"]], H_unstable=H_unstable, H_stable=H_stable,
+                       H_mean=H_unstable if math.isfinite(H_unstable) else H_stable, log_posterior_density=log_post)
         return out
 
     def _prior_program_dev(self, model):

@@ -98,16 +98,26 @@ class LinRegAdjointStats:
         self.launch = _lib.Launch(_lib.FAM_LINREG, lanes_per_chain, 1, 1, npad, 512, panels, lr_terms, self.data_off)
         self.runs_host = (_lib.RunDesc * 1)()
         self.runs_dev = torch.zeros(C.sizeof(_lib.RunDesc), dtype=torch.uint8, device=dev)
-        f64 = torch.float64
-        self.logL = torch.empty(self.M, dtype=f64, device=dev)
-        self.rss = torch.empty(self.M, dtype=f64, device=dev)
-        self.yr = torch.empty(self.M, dtype=f64, device=dev)
+        self._block = None
+        if type(family) is LinearRegressionEvidenceModel:
+            model = family((0.0, 0.0))
+            self._block = model.log_likelihood.device_params(model, self.dps)[0]
+
+    def _device_params(self, theta):
+        """The model's device block and log_const at theta.  theta changes only the prior's scale and sigma
+        in the block, so the Model is built once; a family that forms its models otherwise builds one per theta."""
+        if self._block is None:
+            model = self.family(theta)
+            return model.log_likelihood.device_params(model, self.dps)
+        ls, lt = theta
+        lik = LinearRegressionLikelihood(sigma=float(np.exp(ls)), data=self.family.data)
+        return lik.scaled_params(self._block, self.dps, float(np.exp(lt))), float(lik.log_const)
 
     def __call__(self, theta) -> Tuple[Any, Any, Any]:
         torch = self.torch
         th = np.asarray(theta, dtype=np.float64)
-        model = self.family(th)
-        p, c = model.log_likelihood.device_params(model, self.dps)
+        logL, rss, yr = (torch.empty(self.M, dtype=torch.float64, device=self.U.device) for _ in range(3))
+        p, c = self._device_params(th)
         self.params[:self.n_run].copy_(torch.from_numpy(p))
         d = self.runs_host[0]
         d.D = self.D
@@ -115,10 +125,10 @@ class LinRegAdjointStats:
         d.param_off = 0
         d.log_const = c
         self.runs_dev.copy_(torch.frombuffer(bytearray(bytes(self.runs_host)), dtype=torch.uint8))
-        _lib.check(_lib.lib().hipns_linreg_stats(_lib.ptr(self.U), self.M, _lib.ptr(self.logL), _lib.ptr(self.rss),
-                                                 _lib.ptr(self.yr), _lib.ptr(self.runs_dev), self.runs_host,
-                                                 C.byref(self.bufs), C.byref(self.launch), _lib.stream_ptr()))
-        return self.logL.clone(), self.rss.clone(), self.yr.clone()
+        _lib.check(_lib.lib().hipns_linreg_stats(_lib.ptr(self.U), self.M, _lib.ptr(logL), _lib.ptr(rss), _lib.ptr(yr),
+                                                 _lib.ptr(self.runs_dev), self.runs_host, C.byref(self.bufs),
+                                                 C.byref(self.launch), _lib.stream_ptr()))
+        return logL, rss, yr
 
 
 def _autograd_function():

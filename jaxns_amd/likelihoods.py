@@ -14,6 +14,8 @@ likelihoods of the benchmark configurations.
 """
 from __future__ import annotations
 
+import copy
+
 import numpy as np
 from scipy.special import logsumexp
 
@@ -306,6 +308,15 @@ class LinearRegressionLikelihood(LikelihoodFamily):
         f64[2, :D] = self.data.w0 * c
         return np.concatenate([prm, f64.ravel().view(np.float32)]), float(self.log_const)
 
+    def scaled_params(self, block: np.ndarray, dps: int, tau: float) -> np.ndarray:
+        """device_params of a N(0, tau^2 I) prior at this sigma, from a block of the same prior of any scale."""
+        D, c = self.D, self.data.col_scale
+        prm = block.copy()
+        prm[2 * dps:2 * dps + D] = tau * c
+        prm[4 * dps:4 * dps + 2] = np.array([0.5 / self.sigma ** 2], np.float64).view(np.float32)
+        prm[4 * dps + 4:].view(np.float64)[dps:dps + D] = tau * c
+        return prm
+
     def log_evidence_normal_prior(self, tau) -> float:
         """Analytic log Z for w ~ N(0, tau^2 I): log N(y; 0, sigma^2 I + tau^2 X X^T) (Woodbury form)."""
         s2, t2 = self.sigma ** 2, float(tau) ** 2
@@ -343,10 +354,45 @@ class TorchLikelihood:
         self.fn = fn
         self.model = model
         self.torch = torch
+        self._priors = {}  # device -> [(distribution with its parameters there, width, event shape)]
+
+    def _inputs(self, U):
+        """model.likelihood_inputs_torch(U).  Where the prior model returns its priors' values, one each in
+        order, and none depends on another, the parameters stay on the device from the first batch on;
+        otherwise the generator is driven for every batch."""
+        if U.device not in self._priors:
+            self._priors[U.device] = self._fixed_priors(U.device)
+        priors = self._priors[U.device]
+        if not priors:
+            return self.model.likelihood_inputs_torch(U)
+        u64 = U[:, :self.model.U_ndims].double()
+        args, o = [], 0
+        for dist, w, shp in priors:
+            args.append(dist.forward_torch(u64[:, o:o + w].reshape((U.shape[0],) + shp)))
+            o += w
+        return tuple(args)
+
+    def _fixed_priors(self, device):
+        from . import distributions as tfpd
+        from .framework import _run_generator
+        if self.model.dynamic_prior:
+            return []
+        priors, out, xs = _run_generator(self.model.prior_model, np.full(self.model.U_ndims, 0.5))
+        outs = out if isinstance(out, tuple) else (out,)
+        if len(outs) != len(xs) or any(o is not x for o, x in zip(outs, xs)):
+            return []
+        fixed = []
+        for p in priors:
+            if p._type == "value" or type(p.dist) not in (tfpd.Normal, tfpd.Uniform, tfpd.MultivariateNormalTriL):
+                return []
+            d = copy.copy(p.dist)
+            d._raw = tuple(self.torch.as_tensor(v, dtype=self.torch.float64, device=device) for v in p.dist._raw)
+            fixed.append((d, p.base_ndims, tuple(getattr(p.dist, "event_shape", (p.base_ndims,)))))
+        return fixed
 
     def __call__(self, U):
         t = self.torch
-        L = self.fn(*self.model.likelihood_inputs_torch(U))
+        L = self.fn(*self._inputs(U))
         L = t.as_tensor(L, dtype=t.float64, device=U.device)
         L = L.expand(U.shape[0]) if L.dim() == 0 else L.reshape(-1)
-        return t.where(t.isnan(L), t.full_like(L, -float("inf")), L)
+        return t.nan_to_num(L, nan=-float("inf"), posinf=float("inf"), neginf=-float("inf"))

@@ -119,7 +119,7 @@ class _DeviceSamplerBase(AbstractSampler):
         U[pad:, :self.model.U_ndims] = state["U"]
         b.live_U[0][:N] = torch.from_numpy(U)
         b.live_logL[0][:N] = torch.from_numpy(L)
-        state["batch"], state["cap"] = b, (N, n)
+        state["batch"], state["cap"], state["sorted_log_L"] = b, (N, n), L
         return b
 
     def get_samples(self, key, log_L_constraint, sampler_state, num_samples: int) -> Tuple[Sample, Sample]:
@@ -133,7 +133,7 @@ class _DeviceSamplerBase(AbstractSampler):
         seed, iteration = (key if isinstance(key, tuple) else (key, 0))
         d.seed_lo, d.seed_hi = seed_words(seed)
         b.runs_dev.copy_(torch.frombuffer(bytearray(bytes(b.runs_host)), dtype=torch.uint8))
-        L = b.live_logL[0][:int(d.N)].cpu().numpy()
+        L = sampler_state["sorted_log_L"]
         contour = float(log_L_constraint)
         st = RunState()
         st.buf = 0
@@ -145,9 +145,10 @@ class _DeviceSamplerBase(AbstractSampler):
         check(lib().hipns_shell_sample(ptr(b.runs_dev), ptr(b.states_dev), 1, b.runs_host, C.byref(b.bufs),
                                        C.byref(b.launch), _lib.stream_ptr()), "hipns_shell_sample")
         D = self.model.U_ndims
-        s = Sample(U_sample=b.new_U[:n, :D].double().cpu().numpy(), log_L_constraint=np.full(n, contour),
+        # whole rows as they are, widened on the host
+        s = Sample(U_sample=b.new_U[:n].cpu().numpy()[:, :D].astype(np.float64), log_L_constraint=np.full(n, contour),
                    log_L=b.new_logL[:n].cpu().numpy(),
-                   num_likelihood_evaluations=b.new_evals[:n].to(torch.int64).cpu().numpy())
+                   num_likelihood_evaluations=b.new_evals[:n].cpu().numpy().astype(np.int64))
         k = self.num_phantom()
         if k:
             o = n  # the phantoms follow the shell in the collection (chain-major, k per chain)

@@ -327,3 +327,43 @@ def test_sample_evidence_moments():
     EZ = np.sum(np.exp(logL) * EX_prev / (n + 1.0))
     Z = np.exp(J.sample_evidence(5, n, logL, S=20000))
     assert abs(Z.mean() - EZ) < 4 * Z.std() / np.sqrt(Z.size)
+
+
+@pytest.mark.parametrize("theta", [(0.0, 0.0), (-1.3, 0.7), (2.0, -3.0)])
+def test_regression_block_of_a_theta(theta):
+    """The device block of one scale with another theta's scale and sigma written into it is the block
+    that the theta's own model packs, bit for bit."""
+    from jaxns_amd.evidence_maximisation import LinearRegressionEvidenceModel
+    from jaxns_amd.likelihoods import LinearRegressionLikelihood
+    model = linreg_problem(40, 5, seed=3)[0]
+    fam = LinearRegressionEvidenceModel(model.log_likelihood.data)
+    m0, m1 = fam((0.0, 0.0)), fam(theta)
+    block = m0.log_likelihood.device_params(m0, 32)[0]
+    want, const = m1.log_likelihood.device_params(m1, 32)
+    lik = LinearRegressionLikelihood(sigma=float(np.exp(theta[0])), data=fam.data)
+    assert lik.scaled_params(block, 32, float(np.exp(theta[1]))).tobytes() == want.tobytes()
+    assert lik.log_const == const
+
+
+@pytest.mark.parametrize("returned", ["each", "one", "swapped", "part", "computed"])
+def test_callable_inputs_match_the_generator(returned):
+    """The callable's inputs from parameters kept on the device equal those of the generator driven with
+    the batch, whichever of the two a prior model's return value takes."""
+    import torch
+    from jaxns_amd.likelihoods import TorchLikelihood
+
+    def prior_model():
+        a = yield J.Prior(tfpd.Normal(loc=0.5, scale=2.0), name="a")
+        if returned == "one":
+            return a
+        b = yield J.Prior(tfpd.Uniform(low=-2.0 * np.ones(2), high=np.ones(2)), name="b")
+        c = yield J.Prior(tfpd.MultivariateNormalTriL(np.arange(3.0), np.tril(np.ones((3, 3)))), name="c")
+        return {"each": (a, b, c), "swapped": (c, b, a), "part": (a, c), "computed": (a, b, c + 1.0)}[returned]
+
+    m = J.Model(prior_model, lambda *x: x[0])
+    like = TorchLikelihood(m.log_likelihood, m)
+    U = torch.rand(7, 32)
+    for _ in range(2):
+        got, want = like._inputs(U), m.likelihood_inputs_torch(U)
+        assert len(got) == len(want) and all(torch.equal(g, w) for g, w in zip(got, want))
+    assert bool(like._priors[U.device]) == (returned in ("each", "one"))
