@@ -197,6 +197,19 @@ int sampler_launch(int mode, const hipns_launch_t* L, const hipns::SampleArgs& A
     }
   }
   A.lr_groups = groups;
+  // A wavefront's step takes the time of its instructions, and what some chain needs (a slice's bracket and
+  // direction, the tail polynomial of the prior) is run for all: fewer chains make cheaper steps.  So a
+  // launch with few chains spreads them over more wavefronts, up to one on every other SIMD (every SIMD was
+  // slower where two-wavefront workgroups cannot be placed evenly).  G evaluations/s before and now: D=10,
+  // 250 chains 0.099 and 0.125; mixture D=4, 60 chains 0.029 and 0.036; D=32, 8 x 500 chains 1.367 and
+  // 1.405 (1.146 with every SIMD); 64 x 500 chains, which fill the chip, 10.62 and 10.64.
+  const int cw = HIPNS_WAVE / lpc;
+  A.chains_per_wave = cw;
+  if (L->family != HIPNS_FAM_LINREG && mode != hipns::MODE_INJ) {
+    int cpw = 1;
+    while (cpw < cw && (int64_t)R * ((max_chains + cpw - 1) / cpw) > 2 * num_cus()) ++cpw;
+    A.chains_per_wave = cpw;
+  }
   A.alpha_off =
       (int32_t)hipns::sampler_lds_floats(L->family, dps, maxD, L->gmm_K, lpc, groups, L->lr_ndata, 1,
                                          mode == hipns::MODE_GSLICE);
@@ -210,8 +223,8 @@ int sampler_launch(int mode, const hipns_launch_t* L, const hipns::SampleArgs& A
   int ring = 0;
   A.ring_off = (int32_t)((base_f + 3) / 4 * 4);
   if (hipns::has_dir_ring(mode, L->family, nj)) {
-    const int wpb = L->waves_per_block, cw = HIPNS_WAVE / lpc;
-    const int64_t blocks = (int64_t)R * ((max_chains + cw * wpb - 1) / (cw * wpb));
+    const int wpb = L->waves_per_block, per_block = A.chains_per_wave * wpb;
+    const int64_t blocks = (int64_t)R * ((max_chains + per_block - 1) / per_block);
     const int64_t most = (nj <= 8 ? 16 : 8) / wpb;  // by registers
     int64_t per_cu = (blocks + num_cus() - 1) / num_cus();
     if (per_cu > most) per_cu = most < 1 ? 1 : most;

@@ -23,6 +23,7 @@ struct SampleArgs {
   int32_t gmm_K;
   int32_t alpha_off;  // LDS float offset of the alpha table (after the model parameters)
   int32_t dir_ring;   // slice directions drawn ahead per chain (LDS ring depth; 0 = drawn at each slice start)
+  int32_t chains_per_wave;  // MVN and mixture families: chains of a wavefront (at most 64 / lanes per chain)
   // regression family: shared data of the batch
   const float* lr_r0;
   const uint16_t* lr_xh;

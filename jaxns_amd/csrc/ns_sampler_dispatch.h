@@ -13,7 +13,8 @@ template <int LPC, int NJ, int FAM, int MODE, int KT>
 inline hipError_t launch_rows(const SampleArgs& A, int R, int max_chains, int wpb, size_t lds_bytes, hipStream_t s) {
   constexpr int CW = HIPNS_WAVE / LPC;
   const int per_block = FAM == HIPNS_FAM_LINREG ? A.lr_groups : wpb;  // chain groups
-  int groups = (max_chains + CW - 1) / CW;
+  const int cpw = FAM == HIPNS_FAM_LINREG ? CW : A.chains_per_wave;
+  int groups = (max_chains + cpw - 1) / cpw;
   int bx = (groups + per_block - 1) / per_block;
   if (bx < 1) bx = 1;
   if (FAM == HIPNS_FAM_LINREG && MODE == MODE_SLICE) bx *= A.lr_split;

@@ -1125,8 +1125,10 @@ __global__ void __launch_bounds__(FAM == HIPNS_FAM_LINREG ? HIPNS_WAVE * lr_max_
   constexpr bool CLUSTER = COOP && MODE == MODE_SLICE;
   int split = CLUSTER ? A.lr_split : 1;
   const int block = (int)blockIdx.x / split, slice = (int)blockIdx.x % split;
-  const int chain0 = (block * G + wave) * CW;
-  if (block * G * CW >= nchains) return;  // whole block idle
+  // chains of a wavefront: a launch that leaves SIMDs idle gives each fewer than its lanes hold
+  const int cpw = COOP ? CW : A.chains_per_wave;
+  const int chain0 = (block * G + wave) * cpw;
+  if (block * G * cpw >= nchains) return;  // whole block idle
   unsigned char* cluster = nullptr;
   if constexpr (CLUSTER) {
     if (split > 1) {
@@ -1181,7 +1183,7 @@ __global__ void __launch_bounds__(FAM == HIPNS_FAM_LINREG ? HIPNS_WAVE * lr_max_
   const uint32_t tfm = transform_mask<LPC, NJ>(FAM == HIPNS_FAM_MVN ? mv.tf : gm.tf, h, nj);
 
   const int chain = chain0 + c;
-  bool alive = chain_wave && chain < nchains;
+  bool alive = chain_wave && c < cpw && chain < nchains;
   const int64_t iter = (MODE == MODE_INIT) ? 0xFFFFFFFFll : ((MODE == MODE_INJ) ? 0 : st->iteration);
   const uint32_t k0 = run.seed_lo, k1 = run.seed_hi;
   const uint32_t it32 = (uint32_t)iter;
