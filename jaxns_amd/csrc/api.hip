@@ -197,19 +197,6 @@ int sampler_launch(int mode, const hipns_launch_t* L, const hipns::SampleArgs& A
     }
   }
   A.lr_groups = groups;
-  // A wavefront's step takes the time of its instructions, and what some chain needs (a slice's bracket and
-  // direction, the tail polynomial of the prior) is run for all: fewer chains make cheaper steps.  So a
-  // launch with few chains spreads them over more wavefronts, up to one on every other SIMD (every SIMD was
-  // slower where two-wavefront workgroups cannot be placed evenly).  G evaluations/s before and now: D=10,
-  // 250 chains 0.099 and 0.125; mixture D=4, 60 chains 0.029 and 0.036; D=32, 8 x 500 chains 1.367 and
-  // 1.405 (1.146 with every SIMD); 64 x 500 chains, which fill the chip, 10.62 and 10.64.
-  const int cw = HIPNS_WAVE / lpc;
-  A.chains_per_wave = cw;
-  if (L->family != HIPNS_FAM_LINREG && mode != hipns::MODE_INJ) {
-    int cpw = 1;
-    while (cpw < cw && (int64_t)R * ((max_chains + cpw - 1) / cpw) > 2 * num_cus()) ++cpw;
-    A.chains_per_wave = cpw;
-  }
   A.alpha_off =
       (int32_t)hipns::sampler_lds_floats(L->family, dps, maxD, L->gmm_K, lpc, groups, L->lr_ndata, 1,
                                          mode == hipns::MODE_GSLICE);
@@ -217,12 +204,42 @@ int sampler_launch(int mode, const hipns_launch_t* L, const hipns::SampleArgs& A
   size_t lds = base_f * sizeof(float);
   if ((int)lds > max_lds_bytes())
     return fail(HIPNS_ERANGE, "model parameters need %zu B of LDS, device allows %d", lds, max_lds_bytes());
+  const int nj = hipns::sampler_nj(maxD, lpc), cw = HIPNS_WAVE / lpc;
+  A.ring_off = (int32_t)((base_f + 3) / 4 * 4);
+  A.chains_per_wave = cw;
+  A.columns = 1;
+  if (L->family != HIPNS_FAM_LINREG && mode != hipns::MODE_INJ) {
+    const int wpb = L->waves_per_block;
+    auto waves_of = [&](int cpw) { return (int64_t)(max_chains + cpw - 1) / cpw; };  // per run
+    if (mode == hipns::MODE_SLICE) {
+      // The most proposals of a chain per step (k_sample_spec) that leave every wavefront of the launch a SIMD
+      // of its own: beyond that the SIMDs' time is better spent on one proposal of more chains.  (64 runs of
+      // 500 chains, D=10, take one, 10.4 G evaluations/s.)  G evaluations/s of whole shells with one and with
+      // the rule's: 250 chains, D=10 0.125 and 0.226 (8 proposals); 16 x 500 2.83 and 5.8 (4); mixture D=4, 60
+      // chains 0.036 and 0.079 (8); D=32, 8 x 500 1.40 and 1.95 (2); D=100, 16 x 250 0.32 and 0.42 (2; with
+      // 4, which its LDS keeps from being resident, 0.24).
+      const size_t spec_lds = ((size_t)A.ring_off + (size_t)hipns::spec_lds_floats(nj) * wpb) * sizeof(float);
+      const int64_t by_lds = num_cus() * (int64_t)(max_lds_bytes() / spec_lds), by_simd = num_cus() * 4 / wpb;
+      const int64_t resident = by_lds < by_simd ? by_lds : by_simd;
+      int m = hipns::SPEC_COLUMNS_MAX;
+      while (m > 1 && R * ((waves_of(cw / m) + wpb - 1) / wpb) > resident) m /= 2;
+      A.columns = m;
+      if (m > 1) lds = spec_lds;
+    }
+    // A wavefront's step takes the time of its instructions, and what some chain needs (a slice's bracket and
+    // direction, the tail polynomial of the prior) is run for all: fewer chains make cheaper steps.  So a
+    // launch with few chains spreads them over more wavefronts, up to one on every other SIMD (every SIMD was
+    // slower where two-wavefront workgroups cannot be placed evenly).  G evaluations/s before and after, one
+    // proposal per step: D=10, 250 chains 0.099 and 0.125; mixture D=4, 60 chains 0.029 and 0.036; D=32, 8 x
+    // 500 chains 1.367 and 1.405 (1.146 with every SIMD); 64 x 500 chains, which fill the chip, 10.6 and 10.6.
+    int cpw = 1;
+    while (cpw < cw / A.columns && R * waves_of(cpw) > 2 * num_cus()) ++cpw;
+    A.chains_per_wave = cpw;
+  }
   // direction rings after the alpha table (16-byte aligned), as deep as the LDS of a CU allows with the
   // workgroups resident that the launch brings it; none where even DIR_RING_MIN slots exceed the limit
-  const int nj = hipns::sampler_nj(maxD, lpc);
   int ring = 0;
-  A.ring_off = (int32_t)((base_f + 3) / 4 * 4);
-  if (hipns::has_dir_ring(mode, L->family, nj)) {
+  if (A.columns == 1 && hipns::has_dir_ring(mode, L->family, nj)) {
     const int wpb = L->waves_per_block, per_block = A.chains_per_wave * wpb;
     const int64_t blocks = (int64_t)R * ((max_chains + per_block - 1) / per_block);
     const int64_t most = (nj <= 8 ? 16 : 8) / wpb;  // by registers
@@ -260,7 +277,10 @@ int sampler_launch(int mode, const hipns_launch_t* L, const hipns::SampleArgs& A
   L2.waves_per_block = waves;
   hipError_t e;
   switch (mode) {
-    case hipns::MODE_SLICE: e = hipns::launch_sampler_slice(A, R, max_chains, L2, maxD, lds, s); break;
+    case hipns::MODE_SLICE:
+      e = A.columns > 1 ? hipns::launch_sampler_spec(A, R, max_chains, L2, maxD, lds, s)
+                        : hipns::launch_sampler_slice(A, R, max_chains, L2, maxD, lds, s);
+      break;
     case hipns::MODE_UNIF: e = hipns::launch_sampler_unif(A, R, max_chains, L2, maxD, lds, s); break;
     case hipns::MODE_INIT: e = hipns::launch_sampler_init(A, R, max_chains, L2, maxD, lds, s); break;
     case hipns::MODE_GSLICE: e = hipns::launch_sampler_gslice(A, R, max_chains, L2, maxD, lds, s); break;

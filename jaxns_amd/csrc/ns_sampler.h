@@ -23,7 +23,9 @@ struct SampleArgs {
   int32_t gmm_K;
   int32_t alpha_off;  // LDS float offset of the alpha table (after the model parameters)
   int32_t dir_ring;   // slice directions drawn ahead per chain (LDS ring depth; 0 = drawn at each slice start)
-  int32_t chains_per_wave;  // MVN and mixture families: chains of a wavefront (at most 64 / lanes per chain)
+  int32_t chains_per_wave;  // MVN and mixture families: chains of a wavefront (times columns, at most 64 / lanes
+                            // per chain)
+  int32_t columns;          // proposals of a chain per step (1: k_sample, else k_sample_spec)
   // regression family: shared data of the batch
   const float* lr_r0;
   const uint16_t* lr_xh;
@@ -171,6 +173,11 @@ __host__ __device__ constexpr bool has_dir_ring(int mode, int fam, int nj) {
 // 16; depth 3 or 2), a small one goes to 8.
 constexpr int DIR_RING_MIN = 2, DIR_RING_MAX = 8;
 
+// k_sample_spec: most proposals of a chain per step, and LDS floats of a wavefront (one direction per column,
+// one Philox block of uniforms per lane, and the words that a read of SPEC_COLUMNS_MAX runs past them)
+constexpr int SPEC_COLUMNS_MAX = 8;
+__host__ __device__ constexpr int spec_lds_floats(int nj) { return (nj + 4) * 64 + SPEC_COLUMNS_MAX; }
+
 hipError_t launch_ext_step(const hipns_run_desc_t* runs, hipns_run_state_t* states, const hipns_buffers_t& B,
                            const hipns_ext_state_t& E, int mode, int w, int max_steps, int R, int max_chains, int lpc,
                            int wpb, int dmax, hipStream_t s);
@@ -190,6 +197,8 @@ namespace hipns {
 __global__ void k_lr_clear(const hipns_run_desc_t* runs, const hipns_run_state_t* states, hipns_buffers_t B, int G, int cw);
 hipError_t launch_sampler_slice(const SampleArgs& A, int R, int max_chains, const hipns_launch_t& L, int dmax,
                                 size_t lds_bytes, hipStream_t s);
+hipError_t launch_sampler_spec(const SampleArgs& A, int R, int max_chains, const hipns_launch_t& L, int dmax,
+                               size_t lds_bytes, hipStream_t s);
 hipError_t launch_sampler_unif(const SampleArgs& A, int R, int max_chains, const hipns_launch_t& L, int dmax,
                                size_t lds_bytes, hipStream_t s);
 hipError_t launch_sampler_init(const SampleArgs& A, int R, int max_chains, const hipns_launch_t& L, int dmax,

@@ -885,6 +885,36 @@ def test_runs_do_not_depend_on_direction_ring(fam, D, lpc):
             assert np.array_equal(x, y), (R, wpb)
 
 
+@pytest.mark.parametrize("max_steps,midpoint", [(512, True), (2, True), (5, False)])
+@pytest.mark.parametrize("fam,D,lpc,slices,k", [("mvn", 1, 2, 1, 0), ("mvn", 5, 2, 7, 3), ("mvn", 20, 2, 9, 8),
+                                                ("mvn", 30, 4, 17, 2), ("mvn", 90, 4, 8, 1), ("gmm", 4, 2, 12, 4),
+                                                ("gmm", 50, 4, 5, 4), ("gmm", 70, 8, 9, 0)])
+def test_proposals_evaluated_together(fam, D, lpc, slices, k, max_steps, midpoint):
+    """A small launch evaluates 8, 4 or 2 of a chain's next proposals per step (1, 40 and 160 runs of 35
+    chains), one of 3000 runs one: points, counts, phantoms and step-cap hits are the same bit for bit."""
+    from jaxns_amd.engine import DeviceBatch, RunSpec
+    say(f"proposals together {fam} D={D} lpc={lpc} slices={slices} k={k} max_steps={max_steps} midpoint={midpoint}")
+    model = (mvn_problem(D, seed=D) if fam == "mvn" else gmm_problem(D, seed=D))[0]
+
+    def shells(R, wpb):
+        specs = [RunSpec(model=model, num_live_points=70, num_slices=slices, max_samples=1500, seed=s, k_phantom=k,
+                         midpoint_shrink=midpoint) for s in range(R)]
+        b = DeviceBatch(specs, lanes_per_chain=lpc, waves_per_block=wpb, max_steps=max_steps)
+        b.init_state()
+        for _ in range(3):
+            b.collect_shell(dict(max_samples=1e18))
+        st = b.states()[0]
+        n = int(st.num_samples)
+        return [int(st.cap_hits)] + [x.cpu().numpy() for x in (
+            b.live_U[st.buf][:70], b.live_logL[st.buf][:70], b.live_evals[st.buf][:70], b.samp_U[:n, :D],
+            b.samp_logL[:n], b.samp_evals[:n], b.samp_phantom[:n])]
+
+    ref = shells(3000, 1)
+    for R, wpb in ((1, 1), (40, 2), (160, 4)):
+        for x, y in zip(ref, shells(R, wpb)):
+            assert np.array_equal(x, y), (R, wpb)
+
+
 @pytest.mark.parametrize("K", [1, 3, 4, 5, 6, 7, 8])
 @pytest.mark.parametrize("D,lpc", [(3, 2), (30, 4), (50, 8)])
 def test_mixture_component_rows(K, D, lpc):
