@@ -721,7 +721,14 @@ int hipns_linreg_stats(const float* U_dev, int64_t B, double* logL_dev, double* 
   const int lpc = bufs->dps > 64 ? 4 : launch->lanes_per_chain;
   if ((rc = check_panels(launch, D, lpc))) return rc;
   const size_t lds = hipns::sampler_lds_floats(HIPNS_FAM_LINREG, bufs->dps, D, 1, lpc, 1, launch->lr_ndata, 2) * sizeof(float);
-  hipError_t e = hipns::launch_linreg_stats(U_dev, B, logL_dev, rss_dev, yr_dev, runs_dev, *bufs, lpc, D, lds,
+  // Bound by the latency of the data rows where the workgroups leave SIMDs idle: as long as one wavefront each
+  // would, the most wavefronts share a workgroup's rows (in the same fixed blocks, so the sums are the same).
+  // 4096 x 16: 1 000 points 41.7 -> 14.2 us, 16 000 points 46.1 -> 25.6, 32 000 points (one wavefront per SIMD)
+  // 48.8 -> 45.7; beyond that there is nothing to gain (64 000 points 87.5 and 88.4 us), and few rows lose
+  // to the barriers (300 x 5, 200 000 points: 31 and 50 us).
+  const int cw = HIPNS_WAVE / lpc;
+  const int waves = (B + cw - 1) / cw <= 4 * num_cus() ? hipns::lr_max_waves(hipns::sampler_nj(D, lpc == 2 ? 2 : 4)) : 1;
+  hipError_t e = hipns::launch_linreg_stats(U_dev, B, logL_dev, rss_dev, yr_dev, runs_dev, *bufs, lpc, D, waves, lds,
                                             as_stream(stream), linreg_view(bufs, launch));
   if (e != hipSuccess) return hip_fail(e, "linreg stats launch");
   return HIPNS_OK;

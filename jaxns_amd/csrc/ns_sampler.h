@@ -182,7 +182,7 @@ hipError_t launch_ext_step(const hipns_run_desc_t* runs, hipns_run_state_t* stat
                            const hipns_ext_state_t& E, int mode, int w, int max_steps, int R, int max_chains, int lpc,
                            int wpb, int dmax, hipStream_t s);
 hipError_t launch_linreg_stats(const float* U, int64_t B, double* logL, double* rss, double* yr,
-                               const hipns_run_desc_t* runs, const hipns_buffers_t& Bf, int lpc, int dmax,
+                               const hipns_run_desc_t* runs, const hipns_buffers_t& Bf, int lpc, int dmax, int waves,
                                size_t lds, hipStream_t s, const LinRegLds& lr);
 hipError_t launch_loglik_grad(const float* U, int64_t B, double* out, float* grad, const hipns_run_desc_t* runs,
                               const hipns_buffers_t& Bf, const hipns_launch_t& L, int dmax, int gscr_off, size_t lds,

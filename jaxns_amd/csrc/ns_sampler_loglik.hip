@@ -226,9 +226,10 @@ static hipError_t launch_loglik_fam(const float* U, int64_t B, double* out, cons
 }
 
 // adjoint statistics of the regression likelihood over a batch of points: logL, |r|^2 and y^T r
-// per row of U (one wavefront per chain group; the host derives d logL / d(log sigma, log tau))
+// per row of U (the host derives d logL / d(log sigma, log tau)).  A workgroup's first wavefront holds one
+// group of 64 / LPC points, all of its wavefronts share the data rows.
 template <int LPC, int NJ>
-__global__ void __launch_bounds__(64) k_linreg_stats(const float* U, int64_t B, double* logL, double* rss, double* yr,
+__global__ void __launch_bounds__(HIPNS_WAVE * lr_max_waves(NJ)) k_linreg_stats(const float* U, int64_t B, double* logL, double* rss, double* yr,
                                                      const hipns_run_desc_t* runs, hipns_buffers_t Bf, LinRegLds lrd) {
   constexpr int CW = HIPNS_WAVE / LPC;
   extern __shared__ float lds[];
@@ -243,11 +244,11 @@ __global__ void __launch_bounds__(64) k_linreg_stats(const float* U, int64_t B, 
   lr.split = 1;
   lr.slice = 0;
   load_params(HIPNS_FAM_LINREG, Bf.params + run.param_off, dps, D, 1, lds, mv, gm, LPC, &lr, 1, NJ / 8);
-  const int l = lane_id();
+  const int l = lane_id(), wave = threadIdx.x / HIPNS_WAVE;
   const int c = l % CW, h = l / CW;
   const int64_t row = (int64_t)blockIdx.x * CW + c;
   float up[NJ];
-  const bool ok = row < B;
+  const bool ok = wave == 0 && row < B;
 #pragma unroll
   for (int j = 0; j < NJ; ++j) {
     int d = owned_dim<LPC>(h, j);
@@ -255,7 +256,7 @@ __global__ void __launch_bounds__(64) k_linreg_stats(const float* U, int64_t B, 
   }
   const uint32_t tfm = transform_mask<LPC, NJ>(lr.tf, h, nj);
   double ss = 0.0, sy = 0.0;
-  const double L = lik_linreg<LPC, NJ, true>(up, nj, D, lr, tfm, 0, 1, 1, run.log_const, &ss, &sy);
+  const double L = lik_linreg<LPC, NJ, true>(up, nj, D, lr, tfm, wave, 1, blockDim.x / HIPNS_WAVE, run.log_const, &ss, &sy);
   if (ok && h == 0) {
     logL[row] = L;
     rss[row] = ss;
@@ -265,10 +266,10 @@ __global__ void __launch_bounds__(64) k_linreg_stats(const float* U, int64_t B, 
 
 hipError_t launch_linreg_stats(const float* U, int64_t B, double* logL, double* rss, double* yr,
                                const hipns_run_desc_t* runs, const hipns_buffers_t& Bf, int lpc, int dmax,
-                               size_t lds, hipStream_t s, const LinRegLds& lr) {
+                               int waves, size_t lds, hipStream_t s, const LinRegLds& lr) {
   if (dmax > 64) lpc = 4;
   const int CW = HIPNS_WAVE / lpc;
-  dim3 grid((unsigned)((B + CW - 1) / CW)), block(HIPNS_WAVE);
+  dim3 grid((unsigned)((B + CW - 1) / CW)), block(HIPNS_WAVE * waves);
   if (lpc == 2) {
     if (dmax <= 16)
       hipLaunchKernelGGL((k_linreg_stats<2, 8>), grid, block, lds, s, U, B, logL, rss, yr, runs, Bf, lr);

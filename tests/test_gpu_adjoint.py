@@ -102,3 +102,28 @@ def test_evidence_maximisation_improves_analytic_evidence():
     assert abs(params[0] - ls_opt) < 0.02
     assert abs(params[1] - lt_opt) < abs(theta0[1] - lt_opt)
     assert z1 > z0 + 1.0
+
+
+@pytest.mark.parametrize("n,D,lpc", [(1, 1, 2), (33, 5, 2), (700, 16, 2), (4100, 30, 2), (257, 60, 2), (90, 20, 4),
+                                     (3000, 50, 4), (500, 100, 4)])
+def test_statistics_do_not_depend_on_batch_size(n, D, lpc):
+    """Few points share a workgroup's wavefronts by data rows, many take one wavefront per group of points; a
+    point's log L, |r|^2 and y^T r are the same bit for bit, and within 2e-5 of FP64 (the products' three
+    bf16 terms and FP32 sums)."""
+    import torch
+    say(f"statistics n={n} D={D} lpc={lpc}")
+    rng = np.random.default_rng(n + D)
+    X = rng.normal(size=(n, D))
+    y = X @ rng.normal(size=D) + 0.3 * rng.normal(size=n)
+    fam = LinearRegressionEvidenceModel(J.RegressionData(X, y))
+    U = rng.uniform(0.01, 0.99, size=(40000, D)).astype(np.float32)
+    theta = (-1.2, 0.3)
+    many = LinRegAdjointStats(fam, U, lanes_per_chain=lpc)(theta)
+    for B in (1, 17, 70):
+        few = LinRegAdjointStats(fam, U[:B], lanes_per_chain=lpc)(theta)
+        assert all(torch.equal(f, a[:B]) for f, a in zip(few, many))
+    from scipy.special import ndtri
+    W = math.exp(0.3) * ndtri(U[:70].astype(np.float64))
+    R = y[None, :] - W @ X.T
+    rss = (R * R).sum(1)
+    np.testing.assert_allclose(many[1][:70].cpu().numpy(), rss, rtol=2e-5, atol=2e-5 * float((y * y).sum()))
