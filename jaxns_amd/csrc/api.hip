@@ -142,6 +142,7 @@ int sampler_launch(int mode, const hipns_launch_t* L, const hipns::SampleArgs& A
   int waves = L->waves_per_block, groups = L->waves_per_block;
   bool spread = false;  // regression rows spread over the most wavefronts of few workgroups
   A.lr_split = 1;
+  A.columns = 1;
   if (L->family == HIPNS_FAM_LINREG) {
     if (L->lr_terms == 5)
       return fail(HIPNS_EINVAL, "lr_terms 5 (the refinement form) is for hipns_log_likelihood; sampling takes 1, 3 or 4");
@@ -163,7 +164,7 @@ int sampler_launch(int mode, const hipns_launch_t* L, const hipns::SampleArgs& A
     //    with the rule below alone, 46 with clusters of 8.
     //  - Else the fewest chain groups per workgroup that still fit one workgroup per CU, and the most
     //    wavefronts to share the rows.  4096 x 16, 16 runs of 512 chains (64 workgroups of four groups, or 256
-    //    of one): 17.9 -> 6.5 us per chain step, 1 382 -> 515 ms per batch.
+    //    of one): 17.9 -> 6.5 us per chain step, 1 382 -> 515 ms per batch (340 with the proposals below).
     // A launch of more workgroups keeps the requested groups, one per wavefront, so that the workgroups of a
     // CU overlap.
     const int cw = HIPNS_WAVE / lpc, nj = hipns::sampler_nj(maxD, lpc), wmax = hipns::lr_max_waves(nj);
@@ -194,6 +195,31 @@ int sampler_launch(int mode, const hipns_launch_t* L, const hipns::SampleArgs& A
           break;
         }
       }
+      // Spread launches also evaluate a chain's next proposals together (k_sample_spec), in columns of more
+      // workgroups where there are CUs for them, or of more groups per workgroup: m columns take 0.6, 0.4 and
+      // 0.31 of the steps at 2, 4 and 8 (one run of 512 chains, 4096 x 16: 77 ms with one, 46.5, 30.8, 23.8),
+      // a group's step its matrix cycles beside 10 000 for the chains and the barriers (4 columns: 30.8, 38.1,
+      // 51.5 ms at 1, 2, 4 groups).  16 such runs: 82.6 -> 59.0 ms with 4 columns, 4 groups.
+      if (mode == hipns::MODE_SLICE && spread) {
+        const double steps[4] = {1.0, 0.6, 0.4, 0.31}, matrix = (double)cycles / L->waves_per_block;
+        double best = 10000.0 + matrix * groups;
+        for (int g = 1; g <= hipns::LR_MAX_G; g *= 2) {
+          for (int e = 1; e < 4; ++e) {
+            const int m = 1 << e, chains = g * cw / m;
+            const double cost = steps[e] * (10000.0 + matrix * g);
+            const size_t lds_spec =
+                (hipns::sampler_lds_floats(L->family, dps, maxD, L->gmm_K, lpc, g, L->lr_ndata) + (size_t)max_slices +
+                 4 + (size_t)hipns::spec_lds_floats(nj) * g) * sizeof(float);
+            if (cost < best && R * (int64_t)((max_chains + chains - 1) / chains) <= num_cus() &&
+                lds_spec <= (size_t)max_lds_bytes()) {
+              best = cost;
+              groups = g;
+              A.columns = m;
+            }
+          }
+        }
+        if (waves < groups) waves = groups;
+      }
     }
   }
   A.lr_groups = groups;
@@ -206,8 +232,9 @@ int sampler_launch(int mode, const hipns_launch_t* L, const hipns::SampleArgs& A
     return fail(HIPNS_ERANGE, "model parameters need %zu B of LDS, device allows %d", lds, max_lds_bytes());
   const int nj = hipns::sampler_nj(maxD, lpc), cw = HIPNS_WAVE / lpc;
   A.ring_off = (int32_t)((base_f + 3) / 4 * 4);
-  A.chains_per_wave = cw;
-  A.columns = 1;
+  A.chains_per_wave = cw / A.columns;
+  if (L->family == HIPNS_FAM_LINREG && A.columns > 1)
+    lds = ((size_t)A.ring_off + (size_t)hipns::spec_lds_floats(nj) * groups) * sizeof(float);
   if (L->family != HIPNS_FAM_LINREG && mode != hipns::MODE_INJ) {
     const int wpb = L->waves_per_block;
     auto waves_of = [&](int cpw) { return (int64_t)(max_chains + cpw - 1) / cpw; };  // per run

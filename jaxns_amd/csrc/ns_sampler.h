@@ -134,7 +134,7 @@ __host__ __device__ inline int lr_row_blocks(int tiles, int lpc, int nj) {
 // taking 1/H of the row blocks (cut at eighths) and exchanging the sums of its eighths every step through
 // device memory.  Scratch of a cluster of G groups of cw chains: [join word, step counters: 256 B]
 // [2 parities][G][8][cw] doubles.
-constexpr int LR_EIGHTHS = 8;
+constexpr int LR_EIGHTHS = 8, LR_MAX_G = 4;  // (most chain groups of a workgroup)
 constexpr size_t LR_CLUSTER_HEAD = 256;
 __host__ __device__ inline size_t lr_cluster_bytes(int G, int cw) {
   return LR_CLUSTER_HEAD + (size_t)2 * G * LR_EIGHTHS * cw * sizeof(double);

@@ -125,7 +125,7 @@ __device__ __forceinline__ double chain_sum_d(double v) {
 // X is stored in 16-column panels ([panel][row][16] bf16) so both layouts read dense rows.  Squares
 // of a tile are summed in FP32 and accumulated in FP64.  All W wavefronts must call this together (two
 // workgroup barriers).
-constexpr int LR_MAX_G = 4;
+
 
 // Forms a cluster: true once all H workgroups have joined, and then each of them is running and stays so, so
 // that the waits of every step end.  A workgroup that waits too long for the others (the GPU is busy with

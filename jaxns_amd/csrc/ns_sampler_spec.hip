@@ -14,10 +14,13 @@ namespace hipns {
 // Bound by the latency of one step (about 1.5 us at 8 slots: 600 vector instructions and 8 MFMAs of 64
 // cycles, of a wavefront alone on its SIMD).  A slice takes 2.3 evaluations in early shells and 3.6 in late
 // ones, so with one proposal per step as many steps, with 8 about 1.05.  One run: D=10, 500 live points 8.06
-// -> 4.66 ms; mixture of 4, D=4, with phantoms 4.72 -> 2.90 ms.
+// -> 4.66 ms; mixture of 4, D=4, with phantoms 4.72 -> 2.90 ms.  The regression family runs it on launches that
+// spread their data rows: 16 runs of 512 chains, 4096 x 16, 515 -> 340 ms.
 template <int LPC, int NJ, int FAM, int KT>
-__global__ void __launch_bounds__(256) k_sample_spec(SampleArgs A) {
+__global__ void __launch_bounds__(FAM == HIPNS_FAM_LINREG ? HIPNS_WAVE * lr_max_waves(NJ) : 256)
+    k_sample_spec(SampleArgs A) {
   constexpr int CW = HIPNS_WAVE / LPC;
+  constexpr bool COOP = FAM == HIPNS_FAM_LINREG;  // wavefronts step together and share the data rows
   extern __shared__ float lds[];
   const int r = A.B.run_order ? A.B.run_order[blockIdx.y] : (int)blockIdx.y;
   const hipns_run_desc_t run = A.runs[r];
@@ -28,17 +31,36 @@ __global__ void __launch_bounds__(256) k_sample_spec(SampleArgs A) {
   const int c = l % CW, h = l / CW;
   const int m = A.columns;  // a power of two
   const int i = c & (m - 1), g = c / m;  // proposal of the step, chain of the wavefront
-  const int cpw = A.chains_per_wave;
-  if ((int)blockIdx.x * wpb * cpw >= run.shell) return;  // whole block idle
-  const int chain = ((int)blockIdx.x * wpb + wave) * cpw + g;
-  bool alive = g < cpw && chain < run.shell;
+  const int cpw = A.chains_per_wave, G = COOP ? A.lr_groups : wpb;  // (the wavefronts past G take rows only)
+  if ((int)blockIdx.x * G * cpw >= run.shell) return;  // whole block idle
+  const int chain = ((int)blockIdx.x * G + wave) * cpw + g;
+  bool alive = wave < G && g < cpw && chain < run.shell;
   const int dps = A.B.dps, D = run.D;
   const int DPr = ((D + 8 * LPC - 1) / (8 * LPC)) * (8 * LPC);
   const int nj = NJ == 8 ? 8 : DPr / LPC;
 
   MvnLds mv;
   GmmLds gm;
-  load_params(FAM, A.B.params + run.param_off, dps, D, A.gmm_K, lds, mv, gm, LPC, nullptr, 1, NJ / 8);
+  LinRegLds lr;
+  load_params(FAM, A.B.params + run.param_off, dps, D, A.gmm_K, lds, mv, gm, LPC, &lr, COOP ? G : 1, NJ / 8);
+  if (COOP) {
+    lr.r0 = A.lr_r0;
+    lr.split = 1;
+    lr.slice = 0;
+    // in place before the first step's barriers
+    lr.staged = A.lr_r0_off > 0;
+    lr.r0l = lds + A.lr_r0_off;
+    if (lr.staged) {
+      for (int q = threadIdx.x; q < A.lr_npad; q += blockDim.x) lr.r0l[q] = A.lr_r0[q];
+    }
+    lr.xh = A.lr_xh;
+    lr.xl = A.lr_xl;
+    lr.xf = A.lr_xf;
+    lr.y = nullptr;
+    lr.npad = A.lr_npad;
+    lr.panels = A.lr_panels;
+    lr.terms = A.lr_terms;
+  }
   const uint32_t tfm = transform_mask<LPC, NJ>(FAM == HIPNS_FAM_MVN ? mv.tf : gm.tf, h, nj);
   const uint32_t it32 = (uint32_t)st->iteration, k0 = run.seed_lo, k1 = run.seed_hi;
   const int cur = st->buf;
@@ -89,7 +111,7 @@ __global__ void __launch_bounds__(256) k_sample_spec(SampleArgs A) {
     right = t > 0.0f ? at : right;
   };
 
-  while (__any(alive)) {
+  while (COOP ? __syncthreads_or(alive) : __any(alive)) {
     if (__any(alive && evals + m > pick_end)) {
       if (alive) {
         blk0 = evals >> 2;
@@ -150,8 +172,10 @@ __global__ void __launch_bounds__(256) k_sample_spec(SampleArgs A) {
     double L;
     if constexpr (FAM == HIPNS_FAM_MVN)
       L = lik_mvn<LPC, NJ>(up, nj, D, dps, mv, run.log_const, tfm);
-    else
+    else if constexpr (FAM == HIPNS_FAM_GMM)
       L = lik_gmm<LPC, NJ, KT>(up, nj, D, gm, tfm);
+    else
+      L = lik_linreg<LPC, NJ>(up, nj, D, lr, tfm, wave, G, wpb, run.log_const);
 
     // _new_proposal acceptance (uni_slice_sampler.py:160-166); the step cap keeps the seed point
     const bool acc = alive && ((L > contour) || (logL0 == contour && L == contour));
@@ -219,8 +243,8 @@ __global__ void __launch_bounds__(256) k_sample_spec(SampleArgs A) {
 
 template <int LPC, int NJ, int FAM, int KT>
 static hipError_t launch_spec_rows(const SampleArgs& A, int R, int max_chains, int wpb, size_t lds, hipStream_t s) {
-  const int waves = (max_chains + A.chains_per_wave - 1) / A.chains_per_wave;
-  dim3 grid((waves + wpb - 1) / wpb, R), block(wpb * HIPNS_WAVE);
+  const int per_block = A.chains_per_wave * (FAM == HIPNS_FAM_LINREG ? A.lr_groups : wpb);
+  dim3 grid((max_chains + per_block - 1) / per_block, R), block(wpb * HIPNS_WAVE);
   hipLaunchKernelGGL((k_sample_spec<LPC, NJ, FAM, KT>), grid, block, lds, s, A);
   return hipGetLastError();
 }
@@ -262,6 +286,8 @@ hipError_t launch_sampler_spec(const SampleArgs& A, int R, int max_chains, const
                                size_t lds, hipStream_t s) {
   if (L.family == HIPNS_FAM_GMM)
     return launch_spec_fam<HIPNS_FAM_GMM>(A, R, max_chains, L.lanes_per_chain, L.waves_per_block, dmax, lds, s);
+  if (L.family == HIPNS_FAM_LINREG)
+    return launch_spec_fam<HIPNS_FAM_LINREG>(A, R, max_chains, L.lanes_per_chain, L.waves_per_block, dmax, lds, s);
   return launch_spec_fam<HIPNS_FAM_MVN>(A, R, max_chains, L.lanes_per_chain, L.waves_per_block, dmax, lds, s);
 }
 

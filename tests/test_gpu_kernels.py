@@ -888,13 +888,16 @@ def test_runs_do_not_depend_on_direction_ring(fam, D, lpc):
 @pytest.mark.parametrize("max_steps,midpoint", [(512, True), (2, True), (5, False)])
 @pytest.mark.parametrize("fam,D,lpc,slices,k", [("mvn", 1, 2, 1, 0), ("mvn", 5, 2, 7, 3), ("mvn", 20, 2, 9, 8),
                                                 ("mvn", 30, 4, 17, 2), ("mvn", 90, 4, 8, 1), ("gmm", 4, 2, 12, 4),
-                                                ("gmm", 50, 4, 5, 4), ("gmm", 70, 8, 9, 0)])
+                                                ("gmm", 50, 4, 5, 4), ("gmm", 70, 8, 9, 0), ("linreg", 3, 2, 9, 4),
+                                                ("linreg", 30, 2, 5, 0), ("linreg", 40, 2, 4, 1),
+                                                ("linreg", 20, 4, 7, 3), ("linreg", 90, 4, 4, 0)])
 def test_proposals_evaluated_together(fam, D, lpc, slices, k, max_steps, midpoint):
     """A small launch evaluates 8, 4 or 2 of a chain's next proposals per step (1, 40 and 160 runs of 35
-    chains), one of 3000 runs one: points, counts, phantoms and step-cap hits are the same bit for bit."""
+    chains; the regression family's also in 1, 2 or 4 groups of a workgroup), one of 3000 runs one: points, counts, phantoms and step-cap hits are the same bit for bit."""
     from jaxns_amd.engine import DeviceBatch, RunSpec
     say(f"proposals together {fam} D={D} lpc={lpc} slices={slices} k={k} max_steps={max_steps} midpoint={midpoint}")
-    model = (mvn_problem(D, seed=D) if fam == "mvn" else gmm_problem(D, seed=D))[0]
+    model = (mvn_problem(D, seed=D) if fam == "mvn" else gmm_problem(D, seed=D) if fam == "gmm" else
+             linreg_problem(333, D, seed=D))[0]
 
     def shells(R, wpb):
         specs = [RunSpec(model=model, num_live_points=70, num_slices=slices, max_samples=1500, seed=s, k_phantom=k,
