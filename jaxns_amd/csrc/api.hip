@@ -242,7 +242,7 @@ int sampler_launch(int mode, const hipns_launch_t* L, const hipns::SampleArgs& A
       // The most proposals of a chain per step (k_sample_spec) that leave every wavefront of the launch a SIMD
       // of its own: beyond that the SIMDs' time is better spent on one proposal of more chains.  (64 runs of
       // 500 chains, D=10, take one, 10.4 G evaluations/s.)  G evaluations/s of whole shells with one and with
-      // the rule's: 250 chains, D=10 0.125 and 0.226 (8 proposals); 16 x 500 2.83 and 5.8 (4); mixture D=4, 60
+      // the rule's: 250 chains, D=10 0.125 and 0.231 (8 proposals); 16 x 500 2.83 and 6.0 (4); mixture D=4, 60
       // chains 0.036 and 0.079 (8); D=32, 8 x 500 1.40 and 1.95 (2); D=100, 16 x 250 0.32 and 0.42 (2; with
       // 4, which its LDS keeps from being resident, 0.24).
       const size_t spec_lds = ((size_t)A.ring_off + (size_t)hipns::spec_lds_floats(nj) * wpb) * sizeof(float);

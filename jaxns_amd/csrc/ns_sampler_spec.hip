@@ -14,7 +14,7 @@ namespace hipns {
 // Bound by the latency of one step (about 1.5 us at 8 slots: 600 vector instructions and 8 MFMAs of 64
 // cycles, of a wavefront alone on its SIMD).  A slice takes 2.3 evaluations in early shells and 3.6 in late
 // ones, so with one proposal per step as many steps, with 8 about 1.05.  One run: D=10, 500 live points 8.06
-// -> 4.66 ms; mixture of 4, D=4, with phantoms 4.72 -> 2.90 ms.  The regression family runs it on launches that
+// -> 4.58 ms; mixture of 4, D=4, with phantoms 4.72 -> 2.80 ms.  The regression family runs it on launches that
 // spread their data rows: 16 runs of 512 chains, 4096 x 16, 515 -> 340 ms.
 template <int LPC, int NJ, int FAM, int KT>
 __global__ void __launch_bounds__(FAM == HIPNS_FAM_LINREG ? HIPNS_WAVE * lr_max_waves(NJ) : 256)
@@ -135,18 +135,27 @@ __global__ void __launch_bounds__(FAM == HIPNS_FAM_LINREG ? HIPNS_WAVE * lr_max_
       lds_order();
     }
     if (alive) {
+      // every LDS read of the step at once (a wavefront alone waits out each latency): the uniforms (those
+      // past m, of whatever follows, are not used), the slice's direction and alpha
+      const uint32_t* pw = picks + (evals - 4 * blk0);
+      uint32_t w[SPEC_COLUMNS_MAX];
+#pragma unroll
+      for (int q = 0; q < SPEC_COLUMNS_MAX; ++q) w[q] = pw[q];
+      const int from = h * CW + g * m + ((s - dir0) & (m - 1));
+      float4 v[NJ / 4];
+#pragma unroll
+      for (int j = 0; j < NJ / 4; ++j) v[j] = dirs[j * HIPNS_WAVE + from];
+      const float a = alpha_tab[s];
       if (need_begin) {
         need_begin = false;
         k = 0;
-        alpha = midpoint ? alpha_tab[s] : 1.0f;
-        const int from = h * CW + g * m + (s - dir0);
+        alpha = midpoint ? a : 1.0f;
 #pragma unroll
-        for (int j = 0; j < NJ; j += 4) {
-          const float4 v = dirs[(j / 4) * HIPNS_WAVE + from];
-          nv[j] = v.x;
-          nv[j + 1] = v.y;
-          nv[j + 2] = v.z;
-          nv[j + 3] = v.w;
+        for (int j = 0; j < NJ / 4; ++j) {
+          nv[4 * j] = v[j].x;
+          nv[4 * j + 1] = v[j].y;
+          nv[4 * j + 2] = v[j].z;
+          nv[4 * j + 3] = v[j].w;
         }
         slice_bracket<LPC, NJ>(U0, nv, left, right);
       } else {
@@ -154,10 +163,6 @@ __global__ void __launch_bounds__(FAM == HIPNS_FAM_LINREG ? HIPNS_WAVE * lr_max_
       }
       // the picks up to this column's own (_pick_point_in_interval, _shrink_interval,
       // uni_slice_sampler.py:67-111)
-      const uint32_t* pw = picks + (evals - 4 * blk0);
-      uint32_t w[SPEC_COLUMNS_MAX];
-#pragma unroll
-      for (int q = 0; q < SPEC_COLUMNS_MAX; ++q) w[q] = pw[q];  // (those past m, of whatever follows, are not used)
       t = pick_t(left, right, u01f(w[0]));
 #pragma unroll
       for (int q = 1; q < SPEC_COLUMNS_MAX; ++q) {
@@ -190,9 +195,11 @@ __global__ void __launch_bounds__(FAM == HIPNS_FAM_LINREG ? HIPNS_WAVE * lr_max_
         if (((unsigned)(capped >> (g * m)) >> f) & 1u) {
           ++cap_hits;
         } else {
-#pragma unroll
-          for (int j = 0; j < NJ; ++j) U0[j] = __shfl(up[j], from);
+          // the accepted point again from its t: fewer lane exchanges than slots
+          const float ta = __shfl(t, from);
           logL0 = __shfl(L, from);
+#pragma unroll
+          for (int j = 0; j < NJ; ++j) U0[j] = point_on_line(U0[j], ta, nv[j]);
         }
         // phantom samples: x[-(k+1):-1] (uni_slice_sampler.py:432-440), evals 0
         const int pidx = s - (num_slices - 1 - kph);
