@@ -1,7 +1,7 @@
 // hipns_dev.h -- device helpers shared by the gfx950 kernels of libhipns.
 //
 // Wavefront-64 idioms, the Philox4x32-10 counter PRNG, the inverse normal
-// CDF used by the prior transform, FP64 log-space arithmetic and the
+// CDF used by the prior transform, FP64 numbers of any magnitude and the
 // composition algebra of the evidence recurrence.
 #pragma once
 #include <hip/hip_runtime.h>

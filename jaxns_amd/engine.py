@@ -592,7 +592,7 @@ class DeviceBatch:
     def run(self, term: dict, *, init_efficiency_threshold: float = 0.1, graph_iters: int = 0,
             max_iterations: int = 1_000_000, stream=None, verbose: bool = False):
         """create_init_state -> phases -> consume.  graph_iters > 0 replays a captured
-        hipGraph of that many shells between host checks; 0 syncs after every shell.  verbose prints
+        hipGraph of that many shells between host checks; 0 checks every shell, one shell late.  verbose prints
         run 0's register after every host check (every shell without a graph)."""
         torch = _torch()
         self._verbose = verbose
