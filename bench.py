@@ -57,7 +57,7 @@ MEASURED_VALU = {("c2", 1024): 1.1726e10}
 # 1024 runs at 2 lanes per chain and one wavefront per workgroup), keyed by (workload, lanes per chain);
 # times a step's evaluations per second it gives the VALU issue rate the step sustains
 # (profiles/k_sample_gmm_mixture_r256.md, profiles/k_sample_mvn_d10_n300_r1024.md)
-MEASURED_VALU_PER_EVAL = {("c3", 8): 82.58, ("c1", 2): 21.74}
+MEASURED_VALU_PER_EVAL = {("c3", 8): 63.42, ("c1", 2): 20.35}
 # the oracle ensemble of the same workload (tests/golden/oracle_logZ_ensembles.json) beside the
 # device's log Z statistics
 # runs of a step streamed through this many device slots (engine.run_queue) instead of one batch: none
