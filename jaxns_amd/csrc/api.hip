@@ -136,7 +136,8 @@ int num_cus() {
 
 // scratch_runs: the launch's run descriptors where its spare live buffers may serve as scratch, else NULL
 int sampler_launch(int mode, const hipns_launch_t* L, const hipns::SampleArgs& A0, int R, int max_chains, int maxD,
-                   int dps, int max_slices, hipStream_t s, const hipns_run_desc_t* scratch_runs = nullptr) {
+                   int dps, int max_slices, hipStream_t s, const hipns_run_desc_t* runs = nullptr,
+                   bool spare = false) {
   int lpc = hipns::sampler_lpc(L->family, L->lanes_per_chain, dps, maxD);
   hipns::SampleArgs A = A0;
   int waves = L->waves_per_block, groups = L->waves_per_block;
@@ -172,11 +173,11 @@ int sampler_launch(int mode, const hipns_launch_t* L, const hipns::SampleArgs& A
     auto blocks_of = [&](int g) { return R * ((per_run + g - 1) / g); };
     const int tiles = L->lr_ndata / cw, nb = hipns::lr_row_blocks(tiles, lpc, nj);
     const int64_t cycles = (int64_t)tiles * (nj / 8) * (lr.terms == 4 ? 4 : 3) * groups * (lpc == 2 ? 32 : 16) / 4;
-    if (mode == hipns::MODE_SLICE && lr.terms != 1 && scratch_runs) {
+    if (mode == hipns::MODE_SLICE && lr.terms != 1 && spare) {
       int h = hipns::LR_EIGHTHS;
       while (h > 1 && (blocks_of(groups) * h > num_cus() || cycles / h < 12000 || nb / h < groups)) h /= 2;
       for (int r = 0; h > 1 && r < R; ++r) {
-        const hipns_run_desc_t& d = scratch_runs[r];
+        const hipns_run_desc_t& d = runs[r];
         const int64_t clusters = (d.shell + groups * cw - 1) / (groups * cw);
         if (clusters * (int64_t)hipns::lr_cluster_bytes(groups, cw) > (int64_t)d.N * dps * (int64_t)sizeof(float)) h = 1;
       }
@@ -238,18 +239,30 @@ int sampler_launch(int mode, const hipns_launch_t* L, const hipns::SampleArgs& A
   if (L->family != HIPNS_FAM_LINREG && mode != hipns::MODE_INJ) {
     const int wpb = L->waves_per_block;
     auto waves_of = [&](int cpw) { return (int64_t)(max_chains + cpw - 1) / cpw; };  // per run
-    if (mode == hipns::MODE_SLICE) {
-      // The most proposals of a chain per step (k_sample_spec) that leave every wavefront of the launch a SIMD
-      // of its own: beyond that the SIMDs' time is better spent on one proposal of more chains.  (64 runs of
-      // 500 chains, D=10, take one, 10.4 G evaluations/s.)  G evaluations/s of whole shells with one and with
-      // the rule's: 250 chains, D=10 0.125 and 0.231 (8 proposals); 16 x 500 2.83 and 6.0 (4); mixture D=4, 60
-      // chains 0.036 and 0.079 (8); D=32, 8 x 500 1.40 and 1.95 (2); D=100, 16 x 250 0.32 and 0.42 (2; with
-      // 4, which its LDS keeps from being resident, 0.24).
+    if (mode == hipns::MODE_SLICE && runs) {
+      // The most proposals of a chain per step (k_sample_spec) that bring no SIMD more than 2.5 wavefronts on
+      // average and no CU more workgroups than its LDS holds: beyond that the SIMDs' time is better spent on one
+      // proposal of more chains.  A run counts by the square of its slices against the most of any run: its
+      // chains last that part of a launch, and a run of fewer dimensions ends after fewer shells (64 uneven
+      // mixture runs, D to 64: 611 ms with one, 438 with the rule's 2).  Whole runs with 1, 2, 4 and 8, the rule's in brackets: D=10, 16 x 500
+      // chains 8.2, 5.8, 4.7, [5.0] ms; 64 x 500 10.0, [8.4], 7.4, 10.4; 1024 x 150 [22.5], 24.0, 27.2, 42.2;
+      // D=32, 8 x 500 28.1, 19.4, 17.4, [15.9]; 24 x 500 37.2, [24.8], 26.9, 34.4; 64 x 500 [39.0], 39.0, 48.5,
+      // 81.4; mixture D=20, 16 x 200 53.0, 35.5, 26.9, [21.0]; D=60, 8 lanes a chain, 20 x 400 160, [129], 130,
+      // 202; 64 x 400 [267], 282, 344, 582; D=100, 16 x 250 416, [261], 347 (its LDS keeps one workgroup on a
+      // CU), 614.
       const size_t spec_lds = ((size_t)A.ring_off + (size_t)hipns::spec_lds_floats(nj) * wpb) * sizeof(float);
-      const int64_t by_lds = num_cus() * (int64_t)(max_lds_bytes() / spec_lds), by_simd = num_cus() * 4 / wpb;
-      const int64_t resident = by_lds < by_simd ? by_lds : by_simd;
+      const double by_lds = (double)num_cus() * (int)(max_lds_bytes() / spec_lds), by_simd = 10.0 * num_cus() / wpb;
+      auto blocks_at = [&](int m) {
+        const int per_block = cw / m * wpb;
+        double blocks = 0.0;
+        for (int r = 0; r < R; ++r) {
+          const double f = (double)runs[r].num_slices / max_slices;
+          blocks += (double)((runs[r].shell + per_block - 1) / per_block) * f * f;
+        }
+        return blocks;
+      };
       int m = hipns::SPEC_COLUMNS_MAX;
-      while (m > 1 && R * ((waves_of(cw / m) + wpb - 1) / wpb) > resident) m /= 2;
+      while (m > 1 && (blocks_at(m) > by_lds || blocks_at(m) > by_simd)) m /= 2;
       A.columns = m;
       if (m > 1) lds = spec_lds;
     }
@@ -525,8 +538,7 @@ int hipns_shell_sample(const hipns_run_desc_t* runs_dev, hipns_run_state_t* stat
                               "regression shells step through hipns_ext_step", sampler);
   const int mode = sampler == 1 ? hipns::MODE_UNIF : (sampler >= 2 ? hipns::MODE_GSLICE : hipns::MODE_SLICE);
   const bool spare = bufs->live_U[0] && bufs->live_U[1] && bufs->live_U[0] != bufs->live_U[1];
-  return sampler_launch(mode, launch, A, R, maxS, maxD, bufs->dps, max_slices, as_stream(stream),
-                        spare ? runs_host : nullptr);
+  return sampler_launch(mode, launch, A, R, maxS, maxD, bufs->dps, max_slices, as_stream(stream), runs_host, spare);
 }
 
 int hipns_shell_replace(const hipns_run_desc_t* runs_dev, hipns_run_state_t* states_dev, int32_t R,

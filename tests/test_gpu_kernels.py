@@ -892,8 +892,8 @@ def test_runs_do_not_depend_on_direction_ring(fam, D, lpc):
                                                 ("linreg", 30, 2, 5, 0), ("linreg", 40, 2, 4, 1),
                                                 ("linreg", 20, 4, 7, 3), ("linreg", 90, 4, 4, 0)])
 def test_proposals_evaluated_together(fam, D, lpc, slices, k, max_steps, midpoint):
-    """A small launch evaluates 8, 4 or 2 of a chain's next proposals per step (1, 40 and 160 runs of 35
-    chains; the regression family's also in 1, 2 or 4 groups of a workgroup), one of 3000 runs one: points, counts, phantoms and step-cap hits are the same bit for bit."""
+    """A small launch evaluates 8, 4 or 2 of a chain's next proposals per step (1 to 800 runs of 35 chains; the
+    regression family's also in 1, 2 or 4 groups of a workgroup), one of 3000 runs one: points, counts, phantoms and step-cap hits are the same bit for bit."""
     from jaxns_amd.engine import DeviceBatch, RunSpec
     say(f"proposals together {fam} D={D} lpc={lpc} slices={slices} k={k} max_steps={max_steps} midpoint={midpoint}")
     model = (mvn_problem(D, seed=D) if fam == "mvn" else gmm_problem(D, seed=D) if fam == "gmm" else
@@ -913,7 +913,7 @@ def test_proposals_evaluated_together(fam, D, lpc, slices, k, max_steps, midpoin
             b.samp_logL[:n], b.samp_evals[:n], b.samp_phantom[:n])]
 
     ref = shells(3000, 1)
-    for R, wpb in ((1, 1), (40, 2), (160, 4)):
+    for R, wpb in ((1, 1), (40, 2), (160, 4), (400, 1), (800, 1)):
         for x, y in zip(ref, shells(R, wpb)):
             assert np.array_equal(x, y), (R, wpb)
 
