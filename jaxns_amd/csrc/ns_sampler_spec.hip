@@ -1,4 +1,4 @@
-// ns_sampler_spec.hip -- slice chains of a launch that leaves most of the chip idle: a chain evaluates its
+// ns_sampler_spec.hip -- slice chains of a launch that does not fill the chip: a chain evaluates its
 // next proposals together.
 #include "ns_sampler_impl.h"
 
