@@ -358,10 +358,13 @@ class TorchLikelihood:
 
     def _inputs(self, U):
         """model.likelihood_inputs_torch(U).  Where the prior model returns its priors' values, one each in
-        order, and none depends on another, the parameters stay on the device from the first batch on;
-        otherwise the generator is driven for every batch."""
+        order and untouched, and none depends on another, the parameters stay on the device from the first
+        batch on; otherwise the generator is driven for every batch."""
         if U.device not in self._priors:
-            self._priors[U.device] = self._fixed_priors(U.device)
+            try:
+                self._priors[U.device] = self._fixed_priors(U.device)
+            except Exception:  # a prior model that fails at the probe's points may not at the caller's
+                self._priors[U.device] = []
         priors = self._priors[U.device]
         if not priors:
             return self.model.likelihood_inputs_torch(U)
@@ -373,21 +376,49 @@ class TorchLikelihood:
         return tuple(args)
 
     def _fixed_priors(self, device):
+        """[(distribution with its parameters on the device, width, event shape)], or [] unless the prior
+        model, driven with two batches of different points as likelihood_inputs_torch drives it, yields plain
+        distributions of the same parameters and returns the very tensors it was sent, none written to."""
         from . import distributions as tfpd
-        from .framework import _run_generator
+        torch = self.torch
         if self.model.dynamic_prior:
             return []
-        priors, out, xs = _run_generator(self.model.prior_model, np.full(self.model.U_ndims, 0.5))
-        outs = out if isinstance(out, tuple) else (out,)
-        if len(outs) != len(xs) or any(o is not x for o, x in zip(outs, xs)):
-            return []
-        fixed = []
-        for p in priors:
-            if p._type == "value" or type(p.dist) not in (tfpd.Normal, tfpd.Uniform, tfpd.MultivariateNormalTriL):
+        seen = []
+        for rows in (2, 3):
+            # (different values throughout: multiples of the golden ratio modulo 1)
+            u = (0.5 + 0.6180339887498949 * torch.arange(1, rows * self.model.U_ndims + 1, dtype=torch.float64)) % 1.0
+            u = u.reshape(rows, -1).to(device)
+            gen = self.model.prior_model()
+            resp, o, sent, dists = None, 0, [], []
+            while True:
+                try:
+                    p = gen.send(resp)
+                except StopIteration as e:
+                    out = e.value
+                    break
+                if p._type == "value" or type(p.dist) not in (tfpd.Normal, tfpd.Uniform, tfpd.MultivariateNormalTriL):
+                    return []
+                if any(torch.is_tensor(v) for v in p.dist._raw):
+                    return []  # (parameters formed from earlier values)
+                ref = self.model.priors[len(dists)]
+                w = ref.base_ndims
+                shp = tuple(getattr(ref.dist, "event_shape", (w,)))
+                resp = p.dist.forward_torch(u[:, o:o + w].reshape((rows,) + shp))
+                o += w
+                sent.append((resp, resp._version))
+                dists.append((p.dist, w, shp))
+            outs = out if isinstance(out, tuple) else (out,)
+            if len(outs) != len(sent) or any(x is not t or t._version != v for x, (t, v) in zip(outs, sent)):
                 return []
-            d = copy.copy(p.dist)
-            d._raw = tuple(self.torch.as_tensor(v, dtype=self.torch.float64, device=device) for v in p.dist._raw)
-            fixed.append((d, p.base_ndims, tuple(getattr(p.dist, "event_shape", (p.base_ndims,)))))
+            seen.append(dists)
+        for (a, _, _), (b, _, _) in zip(*seen):
+            if type(a) is not type(b) or not all(np.array_equal(x, y) for x, y in zip(a._raw, b._raw)):
+                return []
+        fixed = []
+        for dist, w, shp in seen[0]:
+            d = copy.copy(dist)
+            d._raw = tuple(torch.as_tensor(v, dtype=torch.float64, device=device) for v in dist._raw)
+            fixed.append((d, w, shp))
         return fixed
 
     def __call__(self, U):

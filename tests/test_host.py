@@ -367,3 +367,39 @@ def test_callable_inputs_match_the_generator(returned):
         got, want = like._inputs(U), m.likelihood_inputs_torch(U)
         assert len(got) == len(want) and all(torch.equal(g, w) for g, w in zip(got, want))
     assert bool(like._priors[U.device]) == (returned in ("each", "one"))
+
+
+@pytest.mark.parametrize("form", ["in place", "in place, one", "tail in place", "symmetric", "tail", "alias",
+                                  "fails early"])
+def test_callable_inputs_of_prior_models_that_look_fixed(form):
+    """Prior models whose return values are the yielded objects themselves but not the untouched prior values,
+    or whose parameters depend on earlier values in a way that the midpoint and a pair of points about it do
+    not show: the callable's inputs equal those of the generator driven with the batch."""
+    import torch
+    from jaxns_amd.likelihoods import TorchLikelihood
+
+    def prior_model():
+        a = yield J.Prior(tfpd.Normal(loc=np.zeros(2), scale=np.ones(2)), name="a")
+        if form.startswith("in place"):
+            a += 1.0
+        if form == "in place, one":
+            return a
+        if form == "tail in place":
+            a[a > 2.0] = 2.0
+        scale = 1.0 if form != "symmetric" else abs(a[..., 0])
+        if form == "tail":
+            scale = 1.0 + 1.0 * (a[..., 0] > 2.0)
+        b = yield J.Prior(tfpd.Normal(loc=0.0, scale=scale), name="b")
+        if form == "alias":
+            c = a
+            c *= 2.0
+        if form == "fails early" and torch.is_tensor(a) and a.shape[0] < 10:
+            raise RuntimeError("few rows")
+        return a, b
+
+    m = J.Model(prior_model, lambda *x: x[0])
+    like = TorchLikelihood(m.log_likelihood, m)
+    U = torch.rand(1000, 32, generator=torch.Generator().manual_seed(1))
+    for _ in range(2):
+        got, want = like._inputs(U), m.likelihood_inputs_torch(U)
+        assert len(got) == len(want) and all(torch.equal(g, w) for g, w in zip(got, want))
