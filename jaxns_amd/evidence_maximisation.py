@@ -105,8 +105,9 @@ class LinRegAdjointStats:
 
     def _device_params(self, theta):
         """The model's device block and log_const at theta.  theta changes only the prior's scale and sigma
-        in the block, so the Model is built once; a family that forms its models otherwise builds one per theta."""
-        if self._block is None:
+        in the block, so the Model is built once; a family that forms its models otherwise builds one per theta,
+        and so does a theta that is not finite (the packing refuses a prior of NaN scale)."""
+        if self._block is None or not np.all(np.isfinite(np.asarray(theta, dtype=np.float64))):
             model = self.family(theta)
             return model.log_likelihood.device_params(model, self.dps)
         ls, lt = theta

@@ -403,3 +403,18 @@ def test_callable_inputs_of_prior_models_that_look_fixed(form):
     for _ in range(2):
         got, want = like._inputs(U), m.likelihood_inputs_torch(U)
         assert len(got) == len(want) and all(torch.equal(g, w) for g, w in zip(got, want))
+
+
+def test_regression_theta_that_is_not_finite_is_refused():
+    """A NaN prior scale is no diagonal prior: refused by the adjoint statistics as by the model's own packing,
+    and a theta of infinities takes what the model packs."""
+    from jaxns_amd.evidence_maximisation import LinearRegressionEvidenceModel, LinRegAdjointStats
+    fam = LinearRegressionEvidenceModel(linreg_problem(40, 5, seed=3)[0].log_likelihood.data)
+    stats = LinRegAdjointStats(fam, np.full((3, 5), 0.5), device="cpu")
+    with pytest.raises(ValueError):
+        stats._device_params(np.array([0.0, np.nan]))
+    for theta in ((0.0, -np.inf), (np.inf, 0.0), (0.3, -0.2)):
+        model = fam(theta)
+        want, const = model.log_likelihood.device_params(model, 32)
+        got, c = stats._device_params(np.array(theta))
+        assert got.tobytes() == want.tobytes() and c == const
