@@ -916,10 +916,11 @@ __device__ __forceinline__ void load_params(int fam, const float* prm, int dps, 
     gm.inv2s2 = lds + 3 * dps + KT * dps;
     gm.logc = gm.inv2s2 + KT;
     gm.dps = dps;
-    // padding dimensions and the rows past K hold zeros (log weight -inf)
+    // padding dimensions and the means past K hold zeros; a row past K has log weight -inf and precision 1, so
+    // that it comes out as -inf for every |x|^2, also one beyond FP32 (0 times that would be NaN)
     for (int i = tid; i < (3 + KT) * dps; i += nt) lds[i] = (i < (3 + K) * dps && i % dps < D) ? prm[i] : 0.0f;
     for (int k = tid; k < KT; k += nt) {
-      gm.inv2s2[k] = k < K ? prm[(3 + K) * dps + k] : 0.0f;
+      gm.inv2s2[k] = k < K ? prm[(3 + K) * dps + k] : 1.0f;
       gm.logc[k] = k < K ? prm[(3 + K) * dps + K + k] : -__builtin_inff();
     }
   }

@@ -979,3 +979,52 @@ def test_concurrent_regression_clusters_match_sequential():
             assert n == int(b.states()[r].num_samples) and n >= 1500
             assert np.array_equal(x.log_L[:n], y.log_L[:n]) and np.array_equal(x.U_samples[:n], y.U_samples[:n])
             assert np.array_equal(x.num_likelihood_evaluations[:n], y.num_likelihood_evaluations[:n])
+
+
+@pytest.mark.parametrize("K", [1, 2, 3, 5, 7])
+@pytest.mark.parametrize("D,lpc", [(1, 2), (3, 2), (30, 4), (50, 8)])
+def test_mixture_of_large_coordinates(K, D, lpc):
+    """Component means of 2e19 to 4e19, whose squares are beyond FP32 while every residual's is not: the
+    component rows past K stay without weight.  log L within 1e-5 relative of FP64 and the gradient within
+    2e-5 of its row's largest component (a residual carries the roundings of p, q u, x and the mean, at most
+    4.4e12 or 2.2e-5 sigma, on 1.5 sigma and more)."""
+    torch = _torch()
+    import jaxns_amd as J
+    from jaxns_amd import distributions as tfpd
+    from jaxns_amd.engine import DeviceBatch, RunSpec
+    say(f"mixture of large coordinates K={K} D={D} lpc={lpc}")
+    sig = 2e17
+    means = np.repeat(2.2e19 + 2e18 * np.arange(K), D).reshape(K, D)
+
+    def prior_model():
+        x = yield J.Prior(tfpd.Uniform(low=2e19 * np.ones(D), high=4e19 * np.ones(D)), name="x")
+        return x
+
+    model = J.Model(prior_model, J.GaussianMixtureLikelihood(means, np.full(K, sig)))
+    b = DeviceBatch([RunSpec(model=model, num_live_points=64, num_slices=2 * D, max_samples=640, seed=1)],
+                    lanes_per_chain=lpc, waves_per_block=2)
+    rng = np.random.default_rng(K)
+    B = 197
+    z = rng.uniform(1.5, 3.0, size=(B, D)) * rng.choice([-1.0, 1.0], size=(B, D))
+    U = np.full((B, b.dps), 0.5, np.float32)
+    U[:, :D] = (means[rng.integers(0, K, B)] + sig * z - 2e19) / 2e19
+    Ud = torch.from_numpy(U).cuda()
+    L = [torch.empty(B, dtype=torch.float64, device="cuda") for _ in range(2)]
+    g = torch.zeros((B, b.dps), dtype=torch.float32, device="cuda")
+    args = (ptr(b.runs_dev), b.runs_host, C.byref(b.bufs), C.byref(b.launch), _stream())
+    check(lib().hipns_log_likelihood(ptr(Ud), B, ptr(L[0]), *args))
+    check(lib().hipns_log_likelihood_grad(ptr(Ud), B, ptr(L[1]), ptr(g), *args))
+    u = torch.from_numpy(U[:, :D].astype(np.float64)).requires_grad_(True)
+    ref = model.log_likelihood.torch_log_prob(2e19 + 2e19 * u)
+    gref, = torch.autograd.grad(ref.sum(), u)
+    ref, gref = ref.detach().numpy(), gref.numpy()
+    for x in L:
+        assert np.max(np.abs(x.cpu().numpy() - ref) / np.maximum(1.0, np.abs(ref))) < 1e-5
+    err = np.abs(g.cpu().numpy()[:, :D] - gref) / np.max(np.abs(gref), axis=1, keepdims=True)
+    assert err.max() < 2e-5, err.max()
+    if D == 1:  # (log L is finite over the whole prior)
+        b.init_state()
+        b.collect_shell(dict(max_samples=640.0))
+        new_U, new_L = b.new_U[:32, :D].cpu().numpy(), b.new_logL[:32].cpu().numpy()
+        f = model.forward_numpy(new_U.astype(np.float64))
+        assert np.max(np.abs(new_L - f) / np.maximum(1.0, np.abs(f))) < 1e-5
