@@ -106,7 +106,8 @@ typedef struct hipns_term_cond {
 } hipns_term_cond_t;
 
 /* Device buffers of a batch of runs.  U rows have stride `dps` floats
- * (dps = padded dimension, a multiple of 32, >= every run's D). */
+ * (dps = padded dimension, a multiple of 32, >= every run's D).  What a row holds
+ * past the run's D (and a parameter block past it) does not change any result. */
 typedef struct hipns_buffers {
   float* live_U[2];
   double* live_logL[2];

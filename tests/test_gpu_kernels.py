@@ -1028,3 +1028,34 @@ def test_mixture_of_large_coordinates(K, D, lpc):
         new_U, new_L = b.new_U[:32, :D].cpu().numpy(), b.new_logL[:32].cpu().numpy()
         f = model.forward_numpy(new_U.astype(np.float64))
         assert np.max(np.abs(new_L - f) / np.maximum(1.0, np.abs(f))) < 1e-5
+
+
+@pytest.mark.parametrize("fam,D,lpc", [("mvn", 5, 2), ("mvn", 20, 2), ("mvn", 20, 4), ("mvn", 40, 4), ("gmm", 5, 4),
+                                       ("gmm", 20, 2), ("gmm", 70, 8), ("linreg", 5, 2), ("linreg", 40, 4)])
+def test_live_row_padding_is_not_read(fam, D, lpc):
+    """Whatever a caller's live rows hold past the run's dimensions (NaN, infinities, large numbers), a
+    sampling launch gives the same points, log L and counts: one run (proposals together), 1200 runs (one
+    proposal a step), and gradient slices."""
+    torch = _torch()
+    from jaxns_amd.engine import DeviceBatch, RunSpec
+    say(f"row padding {fam} D={D} lpc={lpc}")
+    model = (mvn_problem(D, seed=D) if fam == "mvn" else gmm_problem(D, seed=D) if fam == "gmm" else
+             linreg_problem(333, D, seed=D))[0]
+    for R, grad in ((1, False), (1200, False), (2, True)):
+        if grad and fam == "linreg":
+            continue
+        b = DeviceBatch([RunSpec(model=model, num_live_points=70, num_slices=6, max_samples=1500, seed=s, k_phantom=1)
+                         for s in range(R)], lanes_per_chain=lpc, waves_per_block=2, gradient_guided=grad,
+                        gradient_slice=grad)
+        b.init_state()
+        run = (ptr(b.runs_dev), ptr(b.states_dev), b.R, b.runs_host, C.byref(b.bufs))
+        check(lib().hipns_shell_discard(*run, _stream()))
+        out = []
+        pad = b.live_U[0][:, D:]
+        assert pad.shape[1] > 0
+        for v in (0.5, float("nan"), float("inf"), -1e30):
+            pad.fill_(v)
+            check(lib().hipns_shell_sample(*run, C.byref(b.launch), _stream()))
+            out.append([x.clone() for x in (b.new_U[:, :D], b.new_logL, b.new_evals)])
+        for o in out[1:]:
+            assert all(torch.equal(x, y) for x, y in zip(o, out[0]))
