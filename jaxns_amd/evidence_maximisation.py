@@ -107,10 +107,10 @@ class LinRegAdjointStats:
         """The model's device block and log_const at theta.  theta changes only the prior's scale and sigma
         in the block, so the Model is built once; a family that forms its models otherwise builds one per theta,
         and so does a theta that is not finite (the packing refuses a prior of NaN scale)."""
-        if self._block is None or not np.all(np.isfinite(np.asarray(theta, dtype=np.float64))):
+        ls, lt = theta
+        if self._block is None or not (math.isfinite(ls) and math.isfinite(lt)):
             model = self.family(theta)
             return model.log_likelihood.device_params(model, self.dps)
-        ls, lt = theta
         lik = LinearRegressionLikelihood(sigma=float(np.exp(ls)), data=self.family.data)
         return lik.scaled_params(self._block, self.dps, float(np.exp(lt))), float(lik.log_const)
 
