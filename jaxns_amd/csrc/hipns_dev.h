@@ -324,12 +324,19 @@ __device__ __forceinline__ Sc sc_zero() { return {0.0, -__builtin_inf()}; }
 __device__ __forceinline__ Sc sc_mul(const Sc& x, const Sc& y) { return {x.m * y.m, x.e + y.e}; }
 __device__ __forceinline__ Sc sc_scale(const Sc& x, double c) { return {x.m * c, x.e}; }
 
-// both mantissas shifted to the larger exponent (the conversion saturates, and a shift that far is zero;
-// two zeros have a NaN difference, which converts to 0)
+// a difference of exponents as a shift: saturating, NaN to 0.  That is the instruction's own rule; a cast is
+// undefined for both, and a compiler that knows the operand may take any value.
+__device__ __forceinline__ int sc_shift(double d) {
+  int r;
+  asm("v_cvt_i32_f64 %0, %1" : "=v"(r) : "v"(d));
+  return r;
+}
+
+// both mantissas shifted to the larger exponent (a saturated shift gives zero; two zeros have a NaN difference)
 __device__ __forceinline__ Sc sc_add(const Sc& x, const Sc& y) {
 #pragma clang fp contract(off)
   const double e = fmax(x.e, y.e);
-  return {__builtin_amdgcn_ldexp(x.m, (int)(x.e - e)) + __builtin_amdgcn_ldexp(y.m, (int)(y.e - e)), e};
+  return {__builtin_amdgcn_ldexp(x.m, sc_shift(x.e - e)) + __builtin_amdgcn_ldexp(y.m, sc_shift(y.e - e)), e};
 }
 
 // m in [1/2, 1)
