@@ -215,6 +215,48 @@ def test_evidence_scan_closed_form_large():
     np.testing.assert_allclose(f[1], M * np.log(X1), rtol=1e-9)
 
 
+def test_evidence_scan_several_tiles_per_thread():
+    """5 000 003 samples: 1221 tiles of 4096, so threads of the tile scan compose two each.  L = 1 with n = N
+    throughout against closed forms (log X_i = i log(N/(N+1)), log X2_i = i log(N/(N+2)),
+    Z_i = (1 - X_1)/2 + X_1 - X_i), with a workspace and without; rising log L of changing n against a scan of
+    the first 4 000 000 samples, one tile per thread."""
+    torch = _torch()
+    M, N, T = 5_000_003, 4096.0, 4096
+    say(f"evidence_scan of {M} samples")
+    assert M <= lib().hipns_evidence_scan_noalloc_max()
+    L = torch.zeros(M, dtype=torch.float64, device="cuda")
+    n = torch.full((M,), N, dtype=torch.float64, device="cuda")
+    ws = torch.empty(lib().hipns_evidence_scan_workspace_size(M), dtype=torch.uint8, device="cuda")
+
+    def scan(m, per_sample=True, noalloc=False):
+        per = torch.full((8, m), 7.0, dtype=torch.float64, device="cuda")
+        fin = torch.empty(8, dtype=torch.float64, device="cuda")
+        args = (ptr(L), ptr(n), m, -1, ptr(per) if per_sample else None, ptr(fin))
+        if noalloc:
+            check(lib().hipns_evidence_scan_noalloc(*args, _stream()))
+        else:
+            check(lib().hipns_evidence_scan(*args, ptr(ws), ws.numel(), _stream()))
+        return per, fin.cpu().numpy()
+
+    i = np.array([1, 2, T - 1, T, T + 1, 2 * T - 1, 2 * T, 2 * T + 1, 3 * T, 1024 * T - 1, 1024 * T, 1024 * T + 1,
+                  1220 * T, 1220 * T + 1, M], dtype=np.int64)
+    logX = -i * np.log1p(1.0 / N)
+    Z = 0.5 / (N + 1.0) - N / (N + 1.0) * np.expm1(-(i - 1) * np.log1p(1.0 / N))
+    for noalloc in (False, True):
+        per, fin = scan(M, noalloc=noalloc)
+        p = per[:, torch.from_numpy(i - 1).cuda()].cpu().numpy()
+        np.testing.assert_allclose(p[1], logX, rtol=1e-12, atol=1e-15)
+        np.testing.assert_allclose(p[2], -i * np.log1p(2.0 / N), rtol=1e-12, atol=1e-15)
+        np.testing.assert_allclose(p[3], np.log(Z), rtol=0, atol=1e-11)
+        assert np.array_equal(p[:, -1], fin)
+    np.testing.assert_allclose(scan(M, per_sample=False)[1], fin, rtol=1e-12, atol=1e-14)
+    rng = np.random.default_rng(3)
+    L.copy_(torch.from_numpy(np.sort(-50.0 * rng.exponential(size=M))))
+    n.copy_(torch.from_numpy(rng.integers(2000, 4000, size=M).astype(np.float64)))
+    whole, head = scan(M)[0], scan(4_000_000)[0]
+    assert torch.allclose(whole[:, :4_000_000], head, rtol=1e-12, atol=1e-11)
+
+
 def test_argsort_stable_vs_numpy():
     torch = _torch()
     rng = np.random.default_rng(3)
