@@ -67,6 +67,7 @@ struct LinRegLds {
   float* r0l;          // r0 in LDS where `staged` (the rows that this workgroup takes)
   bool staged;
   int split, slice;    // workgroups of the cluster and this one's index (1, 0: no cluster)
+  int b0, b1;          // row blocks of this wavefront
   uint32_t* flags;     // [G][8] step counters of the cluster
   double* exchange;    // [2][G][8][CW] sums of the eighths of the rows
   const uint16_t* xh;  // [panels][npad][16] bf16 hi part of the column-scaled X
@@ -126,9 +127,10 @@ __host__ __device__ constexpr int gmm_rows(int K) { return K <= 4 ? 4 : (K <= 6 
 // tiles on, 32 blocks (16 for the widest instance at 2 lanes per chain, whose LDS they would fill) of at
 // least 32 tiles.
 __host__ __device__ constexpr int lr_max_waves(int nj) { return nj <= 8 ? 8 : 4; }
-__host__ __device__ inline int lr_row_blocks(int tiles, int lpc, int nj) {
-  return tiles < 1024 ? 8 : (lpc == 2 && nj > 16 ? 16 : 32);
+__host__ __device__ inline int lr_row_shift(int tiles, int lpc, int nj) {  // log2 of the number of blocks
+  return tiles < 1024 ? 3 : (lpc == 2 && nj > 16 ? 4 : 5);
 }
+__host__ __device__ inline int lr_row_blocks(int tiles, int lpc, int nj) { return 1 << lr_row_shift(tiles, lpc, nj); }
 
 // Clusters: a launch of large data and few chain groups runs H workgroups on the same chain groups, each
 // taking 1/H of the row blocks (cut at eighths) and exchanging the sums of its eighths every step through

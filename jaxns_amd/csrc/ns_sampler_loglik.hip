@@ -42,8 +42,12 @@ static unsigned loglik_blocks(int64_t groups, int wpb, int nj, size_t lds) {
 // batched likelihood (Model.forward over a batch) through the same device code:
 // row i of U plays the role of chain i of a single wavefront tile.
 // ---------------------------------------------------------------------------
+// (the widest regression instances at one wavefront per SIMD: at the 254 VGPRs that the 2-lane one needs, two
+// would fit, and a launch that does not fill the chip then has two wavefronts share a SIMD's matrix unit beside
+// idle ones: 33000 x 60, 20 000 points in FP32, 1.14 against 2.01 ms)
 template <int LPC, int NJ, int FAM, int KT>
-__global__ void __launch_bounds__(256) k_loglik(const float* U, int64_t B, double* out, const hipns_run_desc_t* runs,
+__global__ void __launch_bounds__(256)
+    __attribute__((amdgpu_waves_per_eu(1, FAM == HIPNS_FAM_LINREG && NJ == 32 ? 1 : 8))) k_loglik(const float* U, int64_t B, double* out, const hipns_run_desc_t* runs,
                                                 hipns_buffers_t Bf, int K, LinRegLds lrd) {
   constexpr int CW = HIPNS_WAVE / LPC;
   extern __shared__ float lds[];
@@ -60,6 +64,7 @@ __global__ void __launch_bounds__(256) k_loglik(const float* U, int64_t B, doubl
   const int wpb = blockDim.x / HIPNS_WAVE;
   load_params(FAM, Bf.params + run.param_off, dps, D, K, lds, mv, gm, LPC, &lr, wpb, NJ / 8);
   const int wave = threadIdx.x / HIPNS_WAVE;
+  if constexpr (FAM == HIPNS_FAM_LINREG) lr_take_blocks<LPC, NJ>(lr, wave, wpb);
   const int l = lane_id();
   const int c = l % CW, h = l / CW;
   const uint32_t tfm = transform_mask<LPC, NJ>(FAM == HIPNS_FAM_MVN ? mv.tf : gm.tf, h, nj);
@@ -68,7 +73,7 @@ __global__ void __launch_bounds__(256) k_loglik(const float* U, int64_t B, doubl
   float up[NJ];
   load_row<LPC, NJ>(up, U, row, row < B, dps, D, nj, h, vec);
   if constexpr (FAM == HIPNS_FAM_LINREG) {
-    const double L = lik_linreg<LPC, NJ, false, true>(up, nj, D, lr, tfm, wave, wpb, wpb, run.log_const);
+    const double L = lik_linreg<LPC, NJ, false, true>(up, nj, D, lr, tfm, wave, wpb, run.log_const);
     if (row < B && h == 0) out[row] = L;
   } else {
     const int64_t stride = (int64_t)gridDim.x * wpb * CW;
@@ -246,6 +251,7 @@ __global__ void __launch_bounds__(HIPNS_WAVE * lr_max_waves(NJ)) k_linreg_stats(
   load_params(HIPNS_FAM_LINREG, Bf.params + run.param_off, dps, D, 1, lds, mv, gm, LPC, &lr, 1, NJ / 8);
   const int l = lane_id(), wave = threadIdx.x / HIPNS_WAVE;
   const int c = l % CW, h = l / CW;
+  lr_take_blocks<LPC, NJ>(lr, wave, blockDim.x / HIPNS_WAVE);
   const int64_t row = (int64_t)blockIdx.x * CW + c;
   float up[NJ];
   const bool ok = wave == 0 && row < B;
@@ -256,7 +262,7 @@ __global__ void __launch_bounds__(HIPNS_WAVE * lr_max_waves(NJ)) k_linreg_stats(
   }
   const uint32_t tfm = transform_mask<LPC, NJ>(lr.tf, h, nj);
   double ss = 0.0, sy = 0.0;
-  const double L = lik_linreg<LPC, NJ, true>(up, nj, D, lr, tfm, wave, 1, blockDim.x / HIPNS_WAVE, run.log_const, &ss, &sy);
+  const double L = lik_linreg<LPC, NJ, true>(up, nj, D, lr, tfm, wave, 1, run.log_const, &ss, &sy);
   if (ok && h == 0) {
     logL[row] = L;
     rss[row] = ss;

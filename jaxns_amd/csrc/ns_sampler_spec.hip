@@ -60,6 +60,7 @@ __global__ void __launch_bounds__(FAM == HIPNS_FAM_LINREG ? HIPNS_WAVE * lr_max_
     lr.npad = A.lr_npad;
     lr.panels = A.lr_panels;
     lr.terms = A.lr_terms;
+    lr_take_blocks<LPC, NJ>(lr, wave, wpb);
   }
   const uint32_t tfm = transform_mask<LPC, NJ>(FAM == HIPNS_FAM_MVN ? mv.tf : gm.tf, h, nj);
   const uint32_t it32 = (uint32_t)st->iteration, k0 = run.seed_lo, k1 = run.seed_hi;
@@ -182,7 +183,7 @@ __global__ void __launch_bounds__(FAM == HIPNS_FAM_LINREG ? HIPNS_WAVE * lr_max_
     else if constexpr (FAM == HIPNS_FAM_GMM)
       L = lik_gmm<LPC, NJ, KT>(up, nj, D, gm, tfm);
     else
-      L = lik_linreg<LPC, NJ>(up, nj, D, lr, tfm, wave, G, wpb, run.log_const);
+      L = lik_linreg<LPC, NJ>(up, nj, D, lr, tfm, wave, G, run.log_const);
 
     // _new_proposal acceptance (uni_slice_sampler.py:160-166); the step cap keeps the seed point
     const bool acc = alive && ((L > contour) || (logL0 == contour && L == contour));
