@@ -875,18 +875,30 @@ __device__ __forceinline__ double lik_gmm(const float (&up)[NJ], int nj, int D, 
 #pragma unroll
       for (int k = 0; k < KT; ++k)
         wk[k] = -2.0f * P.inv2s2[k] * __builtin_amdgcn_exp2f((part[k] - mx) * 1.44269504088896341f) * inv_sum;
+      // (padding dimensions: x, the means and q are zero, so g is)
 #pragma unroll
-      for (int j = 0; j < NJ; ++j) {
-        const int d = owned_dim<LPC>(h, j);
-        const bool in = j < nj && d < D;
-        float dx = 0.0f;
-        if (in) {
-          const float x = xv[j];
+      for (int j = 0; j < NJ; j += 4) {
+        if (j < nj) {  // uniform per run
+          // (the means of these slots are read here: kept from the loop above, or read ahead of their turn, they
+          // take KT * NJ registers; K=8, D=20, 400 000 rows with the gradient: 49 -> 35 us)
+          asm volatile("" ::: "memory");
+          const int d0 = owned_dim<LPC>(h, j);
+          float dx[4] = {0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
-          for (int k = 0; k < KT; ++k)
-            dx = fmaf(wk[k], x - P.mean[k * P.dps + d], dx);
+          for (int k = 0; k < KT; ++k) {
+            const float4 m = *reinterpret_cast<const float4*>(P.mean + k * P.dps + d0);
+            const float mv[4] = {m.x, m.y, m.z, m.w};
+#pragma unroll
+            for (int i = 0; i < 4; ++i) dx[i] = fmaf(wk[k], xv[j + i] - mv[i], dx[i]);
+          }
+          const float4 q4 = *reinterpret_cast<const float4*>(P.q + d0);
+          const float q[4] = {q4.x, q4.y, q4.z, q4.w};
+#pragma unroll
+          for (int i = 0; i < 4; ++i) g[j + i] = dx[i] * q[i] * dq_du(qv[j + i], (tfm >> (j + i)) & 1u);
+        } else {
+#pragma unroll
+          for (int i = 0; i < 4; ++i) g[j + i] = 0.0f;
         }
-        g[j] = in ? dx * P.q[d] * dq_du(qv[j], (tfm >> j) & 1u) : 0.0f;
       }
     }
   }
@@ -1131,11 +1143,12 @@ __device__ __forceinline__ void uniform_point(float (&up)[NJ], int chain, uint32
   }
 }
 
-// (the 8-slot mixture instances of up to six components fit the 128 VGPRs of four wavefronts per SIMD; that
-// of eight would spill 32 of them there, 9.2 against 9.6 G evaluations/s at D=32, K=8, 512 runs)
+// (the 8-slot mixture instances of up to six components are held to the 128 VGPRs of four wavefronts per SIMD,
+// of which that of six spills 6; that of eight would spill 32, 9.2 against 9.6 G evaluations/s at D=32, K=8,
+// 512 runs.  The 16-slot gradient instances are held to two wavefronts.)
 template <int LPC, int NJ, int FAM, int MODE, int KT>
 __global__ void __launch_bounds__(FAM == HIPNS_FAM_LINREG ? HIPNS_WAVE * lr_max_waves(NJ) : 256,
-                                  FAM == HIPNS_FAM_GMM && NJ == 8 && KT <= 6 && MODE != MODE_GSLICE ? 4 : 1)
+                                  FAM != HIPNS_FAM_GMM ? 1 : MODE == MODE_GSLICE ? (NJ == 16 ? 2 : 1) : NJ == 8 && KT <= 6 ? 4 : 1)
     k_sample(SampleArgs A) {
   constexpr int CW = HIPNS_WAVE / LPC;
   // the regression family multiplies the data rows against every chain group of the workgroup

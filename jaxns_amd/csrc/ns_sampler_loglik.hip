@@ -78,7 +78,7 @@ __global__ void __launch_bounds__(256)
   } else {
     const int64_t stride = (int64_t)gridDim.x * wpb * CW;
     for (; __any(row < B); row += stride) {
-      float nx[NJ];  // the next rows load while these are evaluated
+        float nx[NJ];  // the next rows load while these are evaluated
       if (__any(row + stride < B)) load_row<LPC, NJ>(nx, U, row + stride, row + stride < B, dps, D, nj, h, vec);
       double L;
       if constexpr (FAM == HIPNS_FAM_MVN)
@@ -93,9 +93,11 @@ __global__ void __launch_bounds__(256)
 }
 
 // the same with d logL / dU (MVN and mixture families), the device form the gradient-guided chains
-// use: grad[row * dps + d] for d < D; the wavefront's gradient scratch follows the parameters in LDS
+// use: grad[row * dps + d] for d < D; the wavefront's gradient scratch follows the parameters in LDS.
+// (the 32-slot mixture instances at two wavefronts per SIMD, some spilling up to 128 B a lane: D=100, 400 000
+// rows 330 -> 157 us with 6 component rows, 385 -> 267 with 8)
 template <int LPC, int NJ, int FAM, int KT>
-__global__ void __launch_bounds__(256) k_loglik_grad(const float* U, int64_t B, double* out, float* grad,
+__global__ void __launch_bounds__(256, FAM == HIPNS_FAM_GMM && NJ == 32 ? 2 : 1) k_loglik_grad(const float* U, int64_t B, double* out, float* grad,
                                                      const hipns_run_desc_t* runs, hipns_buffers_t Bf, int K,
                                                      int gscr_off) {
   constexpr int CW = HIPNS_WAVE / LPC;
