@@ -134,7 +134,13 @@ int num_cus() {
   return v;
 }
 
-// scratch_runs: the launch's run descriptors where its spare live buffers may serve as scratch, else NULL
+// (a tenth less than the LDS: four workgroups of 37.6 KiB did not stay resident in 160 KiB)
+size_t lds_to_fill() { return (size_t)max_lds_bytes() * 9 / 10; }
+
+hipns::LoglikChip loglik_chip() { return {num_cus(), lds_to_fill()}; }
+
+// runs: the launch's run descriptors (proposals together), else NULL; spare: the live buffer that is not current
+// may serve as scratch
 int sampler_launch(int mode, const hipns_launch_t* L, const hipns::SampleArgs& A0, int R, int max_chains, int maxD,
                    int dps, int max_slices, hipStream_t s, const hipns_run_desc_t* runs = nullptr,
                    bool spare = false) {
@@ -286,8 +292,7 @@ int sampler_launch(int mode, const hipns_launch_t* L, const hipns::SampleArgs& A
     int64_t per_cu = (blocks + num_cus() - 1) / num_cus();
     if (per_cu > most) per_cu = most < 1 ? 1 : most;
     const size_t slot = (size_t)HIPNS_WAVE * nj * wpb * sizeof(float), fixed = (size_t)A.ring_off * sizeof(float);
-    // (a tenth less than the LDS: four workgroups of 37.6 KiB did not stay resident in 160 KiB)
-    const size_t budget = (size_t)max_lds_bytes() * 9 / 10 / per_cu;
+    const size_t budget = lds_to_fill() / per_cu;
     ring = budget > fixed ? (int)((budget - fixed) / slot) : 0;
     if (ring > hipns::DIR_RING_MAX) ring = hipns::DIR_RING_MAX;
     if (ring < hipns::DIR_RING_MIN) ring = hipns::DIR_RING_MIN;
@@ -713,7 +718,8 @@ int hipns_log_likelihood(const float* U_dev, int64_t B, double* logL_dev, const 
     if ((rc = check_panels(launch, D, lpc))) return rc;
     lr = linreg_view(bufs, launch);
   }
-  hipError_t e = hipns::launch_loglik(U_dev, B, logL_dev, runs_dev, *bufs, L2, D, lds, as_stream(stream), lr);
+  hipError_t e =
+      hipns::launch_loglik(U_dev, B, logL_dev, runs_dev, *bufs, L2, D, lds, loglik_chip(), as_stream(stream), lr);
   if (e != hipSuccess) return hip_fail(e, "loglik launch");
   return HIPNS_OK;
 }
@@ -743,8 +749,8 @@ int hipns_log_likelihood_grad(const float* U_dev, int64_t B, double* logL_dev, f
   if ((int)lds > max_lds_bytes()) return fail(HIPNS_ERANGE, "parameters and gradient scratch exceed LDS");
   hipns_launch_t L2 = *launch;
   L2.lanes_per_chain = lpc;
-  hipError_t e =
-      hipns::launch_loglik_grad(U_dev, B, logL_dev, grad_dev, runs_dev, *bufs, L2, D, gscr_off, lds, as_stream(stream));
+  hipError_t e = hipns::launch_loglik_grad(U_dev, B, logL_dev, grad_dev, runs_dev, *bufs, L2, D, gscr_off, lds,
+                                           loglik_chip(), as_stream(stream));
   if (e != hipSuccess) return hip_fail(e, "loglik grad launch");
   return HIPNS_OK;
 }

@@ -186,12 +186,16 @@ hipError_t launch_ext_step(const hipns_run_desc_t* runs, hipns_run_state_t* stat
 hipError_t launch_linreg_stats(const float* U, int64_t B, double* logL, double* rss, double* yr,
                                const hipns_run_desc_t* runs, const hipns_buffers_t& Bf, int lpc, int dmax, int waves,
                                size_t lds, hipStream_t s, const LinRegLds& lr);
+struct LoglikChip {
+  int cus;
+  size_t lds;  // of a CU, that resident workgroups may fill
+};
 hipError_t launch_loglik_grad(const float* U, int64_t B, double* out, float* grad, const hipns_run_desc_t* runs,
                               const hipns_buffers_t& Bf, const hipns_launch_t& L, int dmax, int gscr_off, size_t lds,
-                              hipStream_t s);
+                              const LoglikChip& chip, hipStream_t s);
 hipError_t launch_loglik(const float* U, int64_t B, double* out, const hipns_run_desc_t* runs,
-                         const hipns_buffers_t& Bf, const hipns_launch_t& L, int dmax, size_t lds, hipStream_t s,
-                         const LinRegLds& lr);
+                         const hipns_buffers_t& Bf, const hipns_launch_t& L, int dmax, size_t lds,
+                         const LoglikChip& chip, hipStream_t s, const LinRegLds& lr);
 
 }  // namespace hipns
 

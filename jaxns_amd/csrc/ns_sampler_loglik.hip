@@ -25,17 +25,26 @@ __device__ __forceinline__ void load_row(float (&up)[NJ], const float* U, int64_
   }
 }
 
-// Workgroups of a batched-likelihood launch over `groups` row groups: as many as stay resident (registers:
-// 6, 4 or 2 wavefronts per SIMD at 8, 16 and 32 slots; LDS), each taking row groups in turn, so that the
-// parameter block is read into LDS once per workgroup and not once per 4 wavefronts of rows.  400 000 rows
-// of MVN D=32: 40 -> 24 us, with the gradient 63 -> 42.
-static unsigned loglik_blocks(int64_t groups, int wpb, int nj, size_t lds) {
-  int64_t per_cu = (nj <= 8 ? 24 : (nj <= 16 ? 16 : 8)) / wpb;
-  const int64_t by_lds = lds ? (int64_t)(147456 / lds) : per_cu;
+// Workgroups of a batched-likelihood launch over `groups` row groups: as many as stay resident by the instance's
+// registers and the LDS of a CU, each taking row groups in turn, so that the parameter block is read into LDS
+// once per workgroup and not once per 4 wavefronts of rows.  400 000 rows of MVN D=32: 40 -> 24 us, with the
+// gradient 63 -> 42.
+static unsigned loglik_blocks(int64_t groups, int wpb, int waves_per_simd, size_t lds, const LoglikChip& chip) {
+  int64_t per_cu = 4 * waves_per_simd / wpb;
+  const int64_t by_lds = lds ? (int64_t)(chip.lds / lds) : per_cu;
   if (per_cu > by_lds) per_cu = by_lds;
   if (per_cu < 1) per_cu = 1;
-  const int64_t blocks = (groups + wpb - 1) / wpb, most = 256 * per_cu;
+  const int64_t blocks = (groups + wpb - 1) / wpb, most = chip.cus * per_cu;
   return (unsigned)(blocks < most ? blocks : most);
+}
+
+// wavefronts of a kernel that a SIMD holds by its registers (512 a lane, given in eights; at most 8)
+template <class Kernel>
+static int waves_by_registers(Kernel* kernel) {
+  hipFuncAttributes a{};
+  if (hipFuncGetAttributes(&a, (const void*)kernel) != hipSuccess || a.numRegs < 1) return 1;
+  const int waves = 512 / ((a.numRegs + 7) / 8 * 8);
+  return waves < 1 ? 1 : (waves > 8 ? 8 : waves);
 }
 
 // ---------------------------------------------------------------------------
@@ -146,90 +155,101 @@ __global__ void __launch_bounds__(256, FAM == HIPNS_FAM_GMM && NJ == 32 ? 2 : 1)
   }
 }
 
+template <int LPC, int NJ, int FAM, int KT>
+static hipError_t launch_loglik_grad_rows(const float* U, int64_t B, double* out, float* grad,
+                                          const hipns_run_desc_t* runs, const hipns_buffers_t& Bf, int K, int wpb,
+                                          int gscr_off, size_t lds, const LoglikChip& chip, hipStream_t s) {
+  static const int waves = waves_by_registers(k_loglik_grad<LPC, NJ, FAM, KT>);
+  constexpr int CW = HIPNS_WAVE / LPC;
+  dim3 grid(loglik_blocks((B + CW - 1) / CW, wpb, waves, lds, chip)), block(wpb * HIPNS_WAVE);
+  hipLaunchKernelGGL((k_loglik_grad<LPC, NJ, FAM, KT>), grid, block, lds, s, U, B, out, grad, runs, Bf, K, gscr_off);
+  return hipGetLastError();
+}
+
 template <int LPC, int NJ, int FAM>
 static hipError_t launch_loglik_grad_one(const float* U, int64_t B, double* out, float* grad,
                                          const hipns_run_desc_t* runs, const hipns_buffers_t& Bf, int K, int wpb,
-                                         int gscr_off, size_t lds, hipStream_t s) {
-  constexpr int CW = HIPNS_WAVE / LPC;
-  int64_t groups = (B + CW - 1) / CW;
-  dim3 grid(loglik_blocks(groups, wpb, NJ, lds)), block(wpb * HIPNS_WAVE);
+                                         int gscr_off, size_t lds, const LoglikChip& chip, hipStream_t s) {
   if constexpr (FAM == HIPNS_FAM_GMM) {
-    const int rows = gmm_rows(K);
-    if (rows == 4)
-      hipLaunchKernelGGL((k_loglik_grad<LPC, NJ, FAM, 4>), grid, block, lds, s, U, B, out, grad, runs, Bf, K, gscr_off);
-    else if (rows == 6)
-      hipLaunchKernelGGL((k_loglik_grad<LPC, NJ, FAM, 6>), grid, block, lds, s, U, B, out, grad, runs, Bf, K, gscr_off);
-    else
-      hipLaunchKernelGGL((k_loglik_grad<LPC, NJ, FAM, HIPNS_MAX_GMM_K>), grid, block, lds, s, U, B, out, grad, runs, Bf, K,
-                         gscr_off);
-  } else {
-    hipLaunchKernelGGL((k_loglik_grad<LPC, NJ, FAM, 1>), grid, block, lds, s, U, B, out, grad, runs, Bf, K, gscr_off);
+    switch (gmm_rows(K)) {
+      case 4: return launch_loglik_grad_rows<LPC, NJ, FAM, 4>(U, B, out, grad, runs, Bf, K, wpb, gscr_off, lds, chip, s);
+      case 6: return launch_loglik_grad_rows<LPC, NJ, FAM, 6>(U, B, out, grad, runs, Bf, K, wpb, gscr_off, lds, chip, s);
+      default: break;
+    }
   }
-  return hipGetLastError();
+  constexpr int KT = FAM == HIPNS_FAM_GMM ? HIPNS_MAX_GMM_K : 1;
+  return launch_loglik_grad_rows<LPC, NJ, FAM, KT>(U, B, out, grad, runs, Bf, K, wpb, gscr_off, lds, chip, s);
 }
 
 template <int FAM>
 static hipError_t launch_loglik_grad_fam(const float* U, int64_t B, double* out, float* grad,
                                          const hipns_run_desc_t* runs, const hipns_buffers_t& Bf, int K, int lpc,
-                                         int wpb, int dmax, int gscr_off, size_t lds, hipStream_t s) {
+                                         int wpb, int dmax, int gscr_off, size_t lds, const LoglikChip& chip,
+                                         hipStream_t s) {
   if constexpr (FAM == HIPNS_FAM_GMM) {
     if (lpc == 8 && dmax <= 128) {
-      if (dmax <= 64) return launch_loglik_grad_one<8, 8, FAM>(U, B, out, grad, runs, Bf, K, wpb, gscr_off, lds, s);
-      return launch_loglik_grad_one<8, 16, FAM>(U, B, out, grad, runs, Bf, K, wpb, gscr_off, lds, s);
+      if (dmax <= 64) return launch_loglik_grad_one<8, 8, FAM>(U, B, out, grad, runs, Bf, K, wpb, gscr_off, lds, chip, s);
+      return launch_loglik_grad_one<8, 16, FAM>(U, B, out, grad, runs, Bf, K, wpb, gscr_off, lds, chip, s);
     }
   }
   if (lpc == 4 || lpc == 8 || dmax > 64) {
-    if (dmax <= 32) return launch_loglik_grad_one<4, 8, FAM>(U, B, out, grad, runs, Bf, K, wpb, gscr_off, lds, s);
-    if (dmax <= 64) return launch_loglik_grad_one<4, 16, FAM>(U, B, out, grad, runs, Bf, K, wpb, gscr_off, lds, s);
-    return launch_loglik_grad_one<4, 32, FAM>(U, B, out, grad, runs, Bf, K, wpb, gscr_off, lds, s);
+    if (dmax <= 32) return launch_loglik_grad_one<4, 8, FAM>(U, B, out, grad, runs, Bf, K, wpb, gscr_off, lds, chip, s);
+    if (dmax <= 64) return launch_loglik_grad_one<4, 16, FAM>(U, B, out, grad, runs, Bf, K, wpb, gscr_off, lds, chip, s);
+    return launch_loglik_grad_one<4, 32, FAM>(U, B, out, grad, runs, Bf, K, wpb, gscr_off, lds, chip, s);
   }
-  if (dmax <= 16) return launch_loglik_grad_one<2, 8, FAM>(U, B, out, grad, runs, Bf, K, wpb, gscr_off, lds, s);
-  if (dmax <= 32) return launch_loglik_grad_one<2, 16, FAM>(U, B, out, grad, runs, Bf, K, wpb, gscr_off, lds, s);
-  return launch_loglik_grad_one<2, 32, FAM>(U, B, out, grad, runs, Bf, K, wpb, gscr_off, lds, s);
+  if (dmax <= 16) return launch_loglik_grad_one<2, 8, FAM>(U, B, out, grad, runs, Bf, K, wpb, gscr_off, lds, chip, s);
+  if (dmax <= 32) return launch_loglik_grad_one<2, 16, FAM>(U, B, out, grad, runs, Bf, K, wpb, gscr_off, lds, chip, s);
+  return launch_loglik_grad_one<2, 32, FAM>(U, B, out, grad, runs, Bf, K, wpb, gscr_off, lds, chip, s);
+}
+
+template <int LPC, int NJ, int FAM, int KT>
+static hipError_t launch_loglik_rows(const float* U, int64_t B, double* out, const hipns_run_desc_t* runs,
+                                     const hipns_buffers_t& Bf, int K, int wpb, size_t lds, const LoglikChip& chip,
+                                     hipStream_t s, const LinRegLds& lr) {
+  static const int waves = waves_by_registers(k_loglik<LPC, NJ, FAM, KT>);
+  constexpr int CW = HIPNS_WAVE / LPC;
+  const int64_t groups = (B + CW - 1) / CW;
+  // (the regression family reads all its data rows per row group, beside which its parameters are nothing)
+  dim3 grid(FAM == HIPNS_FAM_LINREG ? (unsigned)((groups + wpb - 1) / wpb) : loglik_blocks(groups, wpb, waves, lds, chip));
+  dim3 block(wpb * HIPNS_WAVE);
+  hipLaunchKernelGGL((k_loglik<LPC, NJ, FAM, KT>), grid, block, lds, s, U, B, out, runs, Bf, K, lr);
+  return hipGetLastError();
 }
 
 template <int LPC, int NJ, int FAM>
 static hipError_t launch_loglik_one(const float* U, int64_t B, double* out, const hipns_run_desc_t* runs,
-                                   const hipns_buffers_t& Bf, int K, int wpb, size_t lds, hipStream_t s,
-                                   const LinRegLds& lr) {
-  constexpr int CW = HIPNS_WAVE / LPC;
-  int64_t groups = (B + CW - 1) / CW;
-  // (the regression family reads all its data rows per row group, beside which its parameters are nothing)
-  dim3 grid(FAM == HIPNS_FAM_LINREG ? (unsigned)((groups + wpb - 1) / wpb) : loglik_blocks(groups, wpb, NJ, lds));
-  dim3 block(wpb * HIPNS_WAVE);
+                                    const hipns_buffers_t& Bf, int K, int wpb, size_t lds, const LoglikChip& chip,
+                                    hipStream_t s, const LinRegLds& lr) {
   if constexpr (FAM == HIPNS_FAM_GMM) {
-    const int rows = gmm_rows(K);
-    if (rows == 4)
-      hipLaunchKernelGGL((k_loglik<LPC, NJ, FAM, 4>), grid, block, lds, s, U, B, out, runs, Bf, K, lr);
-    else if (rows == 6)
-      hipLaunchKernelGGL((k_loglik<LPC, NJ, FAM, 6>), grid, block, lds, s, U, B, out, runs, Bf, K, lr);
-    else
-      hipLaunchKernelGGL((k_loglik<LPC, NJ, FAM, HIPNS_MAX_GMM_K>), grid, block, lds, s, U, B, out, runs, Bf, K, lr);
-  } else {
-    hipLaunchKernelGGL((k_loglik<LPC, NJ, FAM, 1>), grid, block, lds, s, U, B, out, runs, Bf, K, lr);
+    switch (gmm_rows(K)) {
+      case 4: return launch_loglik_rows<LPC, NJ, FAM, 4>(U, B, out, runs, Bf, K, wpb, lds, chip, s, lr);
+      case 6: return launch_loglik_rows<LPC, NJ, FAM, 6>(U, B, out, runs, Bf, K, wpb, lds, chip, s, lr);
+      default: break;
+    }
   }
-  return hipGetLastError();
+  constexpr int KT = FAM == HIPNS_FAM_GMM ? HIPNS_MAX_GMM_K : 1;
+  return launch_loglik_rows<LPC, NJ, FAM, KT>(U, B, out, runs, Bf, K, wpb, lds, chip, s, lr);
 }
 
 // the same instance choice as the sampler launchers (sampler_nj)
 template <int FAM>
 static hipError_t launch_loglik_fam(const float* U, int64_t B, double* out, const hipns_run_desc_t* runs,
-                                   const hipns_buffers_t& Bf, int K, int lpc, int wpb, int dmax, size_t lds,
-                                   hipStream_t s, const LinRegLds& lr) {
+                                    const hipns_buffers_t& Bf, int K, int lpc, int wpb, int dmax, size_t lds,
+                                    const LoglikChip& chip, hipStream_t s, const LinRegLds& lr) {
   if constexpr (FAM == HIPNS_FAM_GMM) {
     if (lpc == 8 && dmax <= 128) {
-      if (dmax <= 64) return launch_loglik_one<8, 8, FAM>(U, B, out, runs, Bf, K, wpb, lds, s, lr);
-      return launch_loglik_one<8, 16, FAM>(U, B, out, runs, Bf, K, wpb, lds, s, lr);
+      if (dmax <= 64) return launch_loglik_one<8, 8, FAM>(U, B, out, runs, Bf, K, wpb, lds, chip, s, lr);
+      return launch_loglik_one<8, 16, FAM>(U, B, out, runs, Bf, K, wpb, lds, chip, s, lr);
     }
   }
   if (lpc == 4 || lpc == 8 || dmax > 64) {
-    if (dmax <= 32) return launch_loglik_one<4, 8, FAM>(U, B, out, runs, Bf, K, wpb, lds, s, lr);
-    if (dmax <= 64) return launch_loglik_one<4, 16, FAM>(U, B, out, runs, Bf, K, wpb, lds, s, lr);
-    return launch_loglik_one<4, 32, FAM>(U, B, out, runs, Bf, K, wpb, lds, s, lr);
+    if (dmax <= 32) return launch_loglik_one<4, 8, FAM>(U, B, out, runs, Bf, K, wpb, lds, chip, s, lr);
+    if (dmax <= 64) return launch_loglik_one<4, 16, FAM>(U, B, out, runs, Bf, K, wpb, lds, chip, s, lr);
+    return launch_loglik_one<4, 32, FAM>(U, B, out, runs, Bf, K, wpb, lds, chip, s, lr);
   }
-  if (dmax <= 16) return launch_loglik_one<2, 8, FAM>(U, B, out, runs, Bf, K, wpb, lds, s, lr);
-  if (dmax <= 32) return launch_loglik_one<2, 16, FAM>(U, B, out, runs, Bf, K, wpb, lds, s, lr);
-  return launch_loglik_one<2, 32, FAM>(U, B, out, runs, Bf, K, wpb, lds, s, lr);
+  if (dmax <= 16) return launch_loglik_one<2, 8, FAM>(U, B, out, runs, Bf, K, wpb, lds, chip, s, lr);
+  if (dmax <= 32) return launch_loglik_one<2, 16, FAM>(U, B, out, runs, Bf, K, wpb, lds, chip, s, lr);
+  return launch_loglik_one<2, 32, FAM>(U, B, out, runs, Bf, K, wpb, lds, chip, s, lr);
 }
 
 // adjoint statistics of the regression likelihood over a batch of points: logL, |r|^2 and y^T r
@@ -298,23 +318,24 @@ hipError_t launch_linreg_stats(const float* U, int64_t B, double* logL, double* 
 
 hipError_t launch_loglik_grad(const float* U, int64_t B, double* out, float* grad, const hipns_run_desc_t* runs,
                               const hipns_buffers_t& Bf, const hipns_launch_t& L, int dmax, int gscr_off, size_t lds,
-                              hipStream_t s) {
+                              const LoglikChip& chip, hipStream_t s) {
   const int lpc = L.lanes_per_chain, wpb = L.waves_per_block, K = L.gmm_K;
   if (L.family == HIPNS_FAM_GMM)
-    return launch_loglik_grad_fam<HIPNS_FAM_GMM>(U, B, out, grad, runs, Bf, K, lpc, wpb, dmax, gscr_off, lds, s);
+    return launch_loglik_grad_fam<HIPNS_FAM_GMM>(U, B, out, grad, runs, Bf, K, lpc, wpb, dmax, gscr_off, lds, chip, s);
   if (L.family == HIPNS_FAM_MVN)
-    return launch_loglik_grad_fam<HIPNS_FAM_MVN>(U, B, out, grad, runs, Bf, K, lpc, wpb, dmax, gscr_off, lds, s);
+    return launch_loglik_grad_fam<HIPNS_FAM_MVN>(U, B, out, grad, runs, Bf, K, lpc, wpb, dmax, gscr_off, lds, chip, s);
   return hipErrorInvalidValue;
 }
 
 hipError_t launch_loglik(const float* U, int64_t B, double* out, const hipns_run_desc_t* runs,
-                         const hipns_buffers_t& Bf, const hipns_launch_t& L, int dmax, size_t lds, hipStream_t s,
-                         const LinRegLds& lr) {
+                         const hipns_buffers_t& Bf, const hipns_launch_t& L, int dmax, size_t lds,
+                         const LoglikChip& chip, hipStream_t s, const LinRegLds& lr) {
   const int lpc = L.lanes_per_chain, wpb = L.waves_per_block, K = L.gmm_K;
-  if (L.family == HIPNS_FAM_GMM) return launch_loglik_fam<HIPNS_FAM_GMM>(U, B, out, runs, Bf, K, lpc, wpb, dmax, lds, s, lr);
+  if (L.family == HIPNS_FAM_GMM)
+    return launch_loglik_fam<HIPNS_FAM_GMM>(U, B, out, runs, Bf, K, lpc, wpb, dmax, lds, chip, s, lr);
   if (L.family == HIPNS_FAM_LINREG)
-    return launch_loglik_fam<HIPNS_FAM_LINREG>(U, B, out, runs, Bf, K, lpc, wpb, dmax, lds, s, lr);
-  return launch_loglik_fam<HIPNS_FAM_MVN>(U, B, out, runs, Bf, K, lpc, wpb, dmax, lds, s, lr);
+    return launch_loglik_fam<HIPNS_FAM_LINREG>(U, B, out, runs, Bf, K, lpc, wpb, dmax, lds, chip, s, lr);
+  return launch_loglik_fam<HIPNS_FAM_MVN>(U, B, out, runs, Bf, K, lpc, wpb, dmax, lds, chip, s, lr);
 }
 
 }  // namespace hipns
