@@ -3,6 +3,7 @@
 #include <stdio.h>
 #include <string.h>
 
+#include <algorithm>
 #include <string>
 
 #include "hipns_dev.h"
@@ -247,17 +248,22 @@ int sampler_launch(int mode, const hipns_launch_t* L, const hipns::SampleArgs& A
     auto waves_of = [&](int cpw) { return (int64_t)(max_chains + cpw - 1) / cpw; };  // per run
     if (mode == hipns::MODE_SLICE && runs) {
       // The most proposals of a chain per step (k_sample_spec) that bring no SIMD more than 2.5 wavefronts on
-      // average and no CU more workgroups than its LDS holds: beyond that the SIMDs' time is better spent on one
-      // proposal of more chains.  A run counts by the square of its slices against the most of any run: its
-      // chains last that part of a launch, and a run of fewer dimensions ends after fewer shells (64 uneven
-      // mixture runs, D to 64: 611 ms with one, 438 with the rule's 2).  Whole runs with 1, 2, 4 and 8, the rule's in brackets: D=10, 16 x 500
-      // chains 8.2, 5.8, 4.7, [5.0] ms; 64 x 500 10.0, [8.4], 7.4, 10.4; 1024 x 150 [22.5], 24.0, 27.2, 42.2;
-      // D=32, 8 x 500 28.1, 19.4, 17.4, [15.9]; 24 x 500 37.2, [24.8], 26.9, 34.4; 64 x 500 [39.0], 39.0, 48.5,
-      // 81.4; mixture D=20, 16 x 200 53.0, 35.5, 26.9, [21.0]; D=60, 8 lanes a chain, 20 x 400 160, [129], 130,
-      // 202; 64 x 400 [267], 282, 344, 582; D=100, 16 x 250 416, [261], 347 (its LDS keeps one workgroup on a
-      // CU), 614.
+      // average, or than it holds of the instance (1 at 32 slots, 2 at 16), and no CU more workgroups than its LDS
+      // holds: beyond that the SIMDs' time is better spent on one proposal of more chains.  A run counts by the
+      // square of its slices against the most of any run: its chains last that part of a launch, and a run of
+      // fewer dimensions ends after fewer shells (64 uneven mixture runs, D to 64: 611 ms with one, 438 with the
+      // rule's 2).  Whole runs with 1, 2, 4 and 8, the rule's in brackets: D=10, 16 x 500 chains 8.2, 5.8, 4.7,
+      // [5.0] ms; 64 x 500 10.0, [8.4], 7.4, 10.4; 1024 x 150 [22.5], 24.0, 27.2, 42.2; D=32, 8 x 500 28.1, 19.4,
+      // 17.4, [15.9]; 24 x 500 37.2, [24.8], 26.9, 34.4; 64 x 500 [39.0], 39.0, 48.5, 81.4; mixture D=20, 16 x 200
+      // 53.0, 35.5, 26.9, [21.0]; D=60, 8 lanes a chain, 20 x 400 160, [129], 130, 202; 64 x 400 [267], 282, 344,
+      // 582; D=100, 16 x 250 416, [261], 347 (its LDS keeps one workgroup on a CU), 614.  Shells of 200 chains by
+      // 2.5 wavefronts whatever the instance and by what it holds: mixture at 2 lanes, D=60, 28 runs 459 and 258
+      // us, 80 runs 707 and 458 (612 with one proposal); at 4 lanes, D=100, K=8, 40 runs 1497 and 842 (1123); MVN
+      // at 2 lanes, D=60, 40 runs 773 and 552 (834); at 4 lanes, D=60, 80 runs, 2.03 wavefronts, 645 and 751 (762).
+      const int resident = hipns::sampler_spec_waves(L->family, L->gmm_K, lpc, maxD);
       const size_t spec_lds = ((size_t)A.ring_off + (size_t)hipns::spec_lds_floats(nj) * wpb) * sizeof(float);
-      const double by_lds = (double)num_cus() * (int)(max_lds_bytes() / spec_lds), by_simd = 10.0 * num_cus() / wpb;
+      const double by_lds = (double)num_cus() * (int)(max_lds_bytes() / spec_lds);
+      const double by_simd = 4.0 * num_cus() * std::min(2.5, (double)resident) / wpb;
       auto blocks_at = [&](int m) {
         const int per_block = cw / m * wpb;
         double blocks = 0.0;

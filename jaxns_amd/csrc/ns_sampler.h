@@ -203,6 +203,18 @@ namespace hipns {
 __global__ void k_lr_clear(const hipns_run_desc_t* runs, const hipns_run_state_t* states, hipns_buffers_t B, int G, int cw);
 hipError_t launch_sampler_slice(const SampleArgs& A, int R, int max_chains, const hipns_launch_t& L, int dmax,
                                 size_t lds_bytes, hipStream_t s);
+// wavefronts of a kernel that a SIMD holds by its registers (512 a lane, given in eights; at most 8)
+template <class Kernel>
+inline int waves_by_registers(Kernel* kernel) {
+  hipFuncAttributes a{};
+  if (hipFuncGetAttributes(&a, (const void*)kernel) != hipSuccess || a.numRegs < 1) return 1;
+  const int waves = 512 / ((a.numRegs + 7) / 8 * 8);
+  return waves < 1 ? 1 : (waves > 8 ? 8 : waves);
+}
+
+// ... of the k_sample_spec instance that launch_sampler_spec takes for these
+int sampler_spec_waves(int family, int K, int lpc, int dmax);
+
 hipError_t launch_sampler_spec(const SampleArgs& A, int R, int max_chains, const hipns_launch_t& L, int dmax,
                                size_t lds_bytes, hipStream_t s);
 hipError_t launch_sampler_unif(const SampleArgs& A, int R, int max_chains, const hipns_launch_t& L, int dmax,

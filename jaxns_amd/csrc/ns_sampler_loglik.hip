@@ -38,15 +38,6 @@ static unsigned loglik_blocks(int64_t groups, int wpb, int waves_per_simd, size_
   return (unsigned)(blocks < most ? blocks : most);
 }
 
-// wavefronts of a kernel that a SIMD holds by its registers (512 a lane, given in eights; at most 8)
-template <class Kernel>
-static int waves_by_registers(Kernel* kernel) {
-  hipFuncAttributes a{};
-  if (hipFuncGetAttributes(&a, (const void*)kernel) != hipSuccess || a.numRegs < 1) return 1;
-  const int waves = 512 / ((a.numRegs + 7) / 8 * 8);
-  return waves < 1 ? 1 : (waves > 8 ? 8 : waves);
-}
-
 // ---------------------------------------------------------------------------
 // batched likelihood (Model.forward over a batch) through the same device code:
 // row i of U plays the role of chain i of a single wavefront tile.

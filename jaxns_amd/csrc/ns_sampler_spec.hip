@@ -251,54 +251,75 @@ __global__ void __launch_bounds__(FAM == HIPNS_FAM_LINREG ? HIPNS_WAVE * lr_max_
   }
 }
 
+// A call of the instance that a launch takes: the launch itself, or the wavefronts that a SIMD holds of it.
+struct SpecCall {
+  const SampleArgs* A;  // NULL: the wavefronts
+  int R, max_chains, wpb;
+  size_t lds;
+  hipStream_t s;
+  int waves;
+  hipError_t err;
+};
+
 template <int LPC, int NJ, int FAM, int KT>
-static hipError_t launch_spec_rows(const SampleArgs& A, int R, int max_chains, int wpb, size_t lds, hipStream_t s) {
-  const int per_block = A.chains_per_wave * (FAM == HIPNS_FAM_LINREG ? A.lr_groups : wpb);
-  dim3 grid((max_chains + per_block - 1) / per_block, R), block(wpb * HIPNS_WAVE);
-  hipLaunchKernelGGL((k_sample_spec<LPC, NJ, FAM, KT>), grid, block, lds, s, A);
-  return hipGetLastError();
+static void spec_rows(SpecCall& c) {
+  if (!c.A) {
+    static const int waves = waves_by_registers(k_sample_spec<LPC, NJ, FAM, KT>);
+    c.waves = waves;
+    return;
+  }
+  const int per_block = c.A->chains_per_wave * (FAM == HIPNS_FAM_LINREG ? c.A->lr_groups : c.wpb);
+  dim3 grid((c.max_chains + per_block - 1) / per_block, c.R), block(c.wpb * HIPNS_WAVE);
+  hipLaunchKernelGGL((k_sample_spec<LPC, NJ, FAM, KT>), grid, block, c.lds, c.s, *c.A);
+  c.err = hipGetLastError();
 }
 
 template <int LPC, int NJ, int FAM>
-static hipError_t launch_spec_one(const SampleArgs& A, int R, int max_chains, int wpb, size_t lds, hipStream_t s) {
+static void spec_one(SpecCall& c, int K) {
   if constexpr (FAM == HIPNS_FAM_GMM) {
-    switch (gmm_rows(A.gmm_K)) {
-      case 4: return launch_spec_rows<LPC, NJ, FAM, 4>(A, R, max_chains, wpb, lds, s);
-      case 6: return launch_spec_rows<LPC, NJ, FAM, 6>(A, R, max_chains, wpb, lds, s);
-      default: return launch_spec_rows<LPC, NJ, FAM, HIPNS_MAX_GMM_K>(A, R, max_chains, wpb, lds, s);
+    switch (gmm_rows(K)) {
+      case 4: return spec_rows<LPC, NJ, FAM, 4>(c);
+      case 6: return spec_rows<LPC, NJ, FAM, 6>(c);
+      default: return spec_rows<LPC, NJ, FAM, HIPNS_MAX_GMM_K>(c);
     }
   } else {
-    return launch_spec_rows<LPC, NJ, FAM, 1>(A, R, max_chains, wpb, lds, s);
+    return spec_rows<LPC, NJ, FAM, 1>(c);
   }
 }
 
 // the same instance choice as the sampler launchers (sampler_nj)
 template <int FAM>
-static hipError_t launch_spec_fam(const SampleArgs& A, int R, int max_chains, int lpc, int wpb, int dmax, size_t lds,
-                                  hipStream_t s) {
+static void spec_fam(SpecCall& c, int K, int lpc, int dmax) {
   if constexpr (FAM == HIPNS_FAM_GMM) {
-    if (lpc == 8 && dmax <= 128) {
-      if (dmax <= 64) return launch_spec_one<8, 8, FAM>(A, R, max_chains, wpb, lds, s);
-      return launch_spec_one<8, 16, FAM>(A, R, max_chains, wpb, lds, s);
-    }
+    if (lpc == 8 && dmax <= 128) return dmax <= 64 ? spec_one<8, 8, FAM>(c, K) : spec_one<8, 16, FAM>(c, K);
   }
   if (lpc == 4 || lpc == 8 || dmax > 64) {
-    if (dmax <= 32) return launch_spec_one<4, 8, FAM>(A, R, max_chains, wpb, lds, s);
-    if (dmax <= 64) return launch_spec_one<4, 16, FAM>(A, R, max_chains, wpb, lds, s);
-    return launch_spec_one<4, 32, FAM>(A, R, max_chains, wpb, lds, s);
+    if (dmax <= 32) return spec_one<4, 8, FAM>(c, K);
+    if (dmax <= 64) return spec_one<4, 16, FAM>(c, K);
+    return spec_one<4, 32, FAM>(c, K);
   }
-  if (dmax <= 16) return launch_spec_one<2, 8, FAM>(A, R, max_chains, wpb, lds, s);
-  if (dmax <= 32) return launch_spec_one<2, 16, FAM>(A, R, max_chains, wpb, lds, s);
-  return launch_spec_one<2, 32, FAM>(A, R, max_chains, wpb, lds, s);
+  if (dmax <= 16) return spec_one<2, 8, FAM>(c, K);
+  if (dmax <= 32) return spec_one<2, 16, FAM>(c, K);
+  return spec_one<2, 32, FAM>(c, K);
+}
+
+static void spec_call(SpecCall& c, int family, int K, int lpc, int dmax) {
+  if (family == HIPNS_FAM_GMM) return spec_fam<HIPNS_FAM_GMM>(c, K, lpc, dmax);
+  if (family == HIPNS_FAM_LINREG) return spec_fam<HIPNS_FAM_LINREG>(c, K, lpc, dmax);
+  return spec_fam<HIPNS_FAM_MVN>(c, K, lpc, dmax);
 }
 
 hipError_t launch_sampler_spec(const SampleArgs& A, int R, int max_chains, const hipns_launch_t& L, int dmax,
                                size_t lds, hipStream_t s) {
-  if (L.family == HIPNS_FAM_GMM)
-    return launch_spec_fam<HIPNS_FAM_GMM>(A, R, max_chains, L.lanes_per_chain, L.waves_per_block, dmax, lds, s);
-  if (L.family == HIPNS_FAM_LINREG)
-    return launch_spec_fam<HIPNS_FAM_LINREG>(A, R, max_chains, L.lanes_per_chain, L.waves_per_block, dmax, lds, s);
-  return launch_spec_fam<HIPNS_FAM_MVN>(A, R, max_chains, L.lanes_per_chain, L.waves_per_block, dmax, lds, s);
+  SpecCall c{&A, R, max_chains, L.waves_per_block, lds, s, 0, hipSuccess};
+  spec_call(c, L.family, A.gmm_K, L.lanes_per_chain, dmax);
+  return c.err;
+}
+
+int sampler_spec_waves(int family, int K, int lpc, int dmax) {
+  SpecCall c{};
+  spec_call(c, family, K, lpc, dmax);
+  return c.waves;
 }
 
 }  // namespace hipns
