@@ -71,21 +71,30 @@ __global__ void __launch_bounds__(256)
   const bool vec = ((uintptr_t)U & 15u) == 0;
   int64_t row = ((int64_t)blockIdx.x * wpb + wave) * CW + c;
   float up[NJ];
-  load_row<LPC, NJ>(up, U, row, row < B, dps, D, nj, h, vec);
   if constexpr (FAM == HIPNS_FAM_LINREG) {
+    load_row<LPC, NJ>(up, U, row, row < B, dps, D, nj, h, vec);
     const double L = lik_linreg<LPC, NJ, false, true>(up, nj, D, lr, tfm, wave, wpb, run.log_const);
     if (row < B && h == 0) out[row] = L;
   } else {
     const int64_t stride = (int64_t)gridDim.x * wpb * CW;
-    for (; __any(row < B); row += stride) {
-        float nx[NJ];  // the next rows load while these are evaluated
-      if (__any(row + stride < B)) load_row<LPC, NJ>(nx, U, row + stride, row + stride < B, dps, D, nj, h, vec);
-      double L;
-      if constexpr (FAM == HIPNS_FAM_MVN)
-        L = lik_mvn<LPC, NJ>(up, nj, D, dps, mv, run.log_const, tfm);
-      else
-        L = lik_gmm<LPC, NJ, KT>(up, nj, D, gm, tfm);
-      if (row < B && h == 0) out[row] = L;
+    int64_t next = row;
+    for (bool first = true;; first = false) {
+      // the next rows load while these are evaluated (at one place, the first rows' too: a small batch's time is
+      // its instructions' way to the CU)
+      const bool more = __any(next < B);
+      float nx[NJ];
+      if (more) load_row<LPC, NJ>(nx, U, next, next < B, dps, D, nj, h, vec);
+      if (!first) {
+        double L;
+        if constexpr (FAM == HIPNS_FAM_MVN)
+          L = lik_mvn<LPC, NJ>(up, nj, D, dps, mv, run.log_const, tfm);
+        else
+          L = lik_gmm<LPC, NJ, KT>(up, nj, D, gm, tfm);
+        if (row < B && h == 0) out[row] = L;
+      }
+      if (!more) break;
+      row = next;
+      next += stride;
 #pragma unroll
       for (int j = 0; j < NJ; ++j) up[j] = nx[j];
     }
