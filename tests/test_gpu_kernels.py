@@ -1101,3 +1101,35 @@ def test_live_row_padding_is_not_read(fam, D, lpc):
             out.append([x.clone() for x in (b.new_U[:, :D], b.new_logL, b.new_evals)])
         for o in out[1:]:
             assert all(torch.equal(x, y) for x, y in zip(o, out[0]))
+
+
+@pytest.mark.parametrize("rows,D,lpc,N", [(40000, 9, 2, 1024), (40000, 30, 2, 1024), (40000, 60, 2, 300),
+                                          (33000, 40, 4, 700), (16500, 100, 4, 1024)])
+@pytest.mark.parametrize("terms", [3, 4])
+def test_regression_cluster_matches_one_workgroup(rows, D, lpc, N, terms):
+    """Large data and few chains: 4 or 8 workgroups share a set of chains where the live buffer that is not
+    current may hold their exchange, and one takes all rows where it may not (a NULL pointer).  Points, log L
+    and counts are the same bit for bit, on the instances of 8, 16 and 32 slots."""
+    torch = _torch()
+    from jaxns_amd.engine import DeviceBatch, RunSpec
+    say(f"regression cluster {rows}x{D} lpc={lpc} N={N} terms={terms}")
+    model, _, _ = linreg_problem(rows, D, seed=rows + D, sigma=0.4, tau=1.0)
+    b = DeviceBatch([RunSpec(model=model, num_live_points=N, num_slices=5, k_phantom=1, max_samples=20 * N, seed=s)
+                     for s in range(2)], lanes_per_chain=lpc, waves_per_block=4, lr_terms=terms)
+    b.init_state()
+    for _ in range(2):
+        b.collect_shell(dict(max_samples=1e18))
+    run = (ptr(b.runs_dev), ptr(b.states_dev), b.R, b.runs_host)
+    check(lib().hipns_shell_discard(*run, C.byref(b.bufs), _stream()))
+    bufs = _lib.Buffers.from_buffer_copy(b.bufs)
+    assert len({st.buf for st in b.states()}) == 1
+    bufs.live_U[1 - b.states()[0].buf] = None
+    out = []
+    for f in (b.bufs, bufs, b.bufs):
+        for t in (b.new_U, b.new_logL, b.new_evals, b.samp_logL):
+            t.fill_(7)
+        check(lib().hipns_shell_sample(*run, C.byref(f), C.byref(b.launch), _stream()))
+        out.append([t.clone() for t in (b.new_U, b.new_logL, b.new_evals, b.samp_logL)])
+    for o in out[1:]:
+        assert all(torch.equal(x, y) for x, y in zip(o, out[0]))
+    assert bool((out[0][2][:b.specs[0].shell] >= 5).all())
