@@ -38,7 +38,7 @@ def _key(specs, lr_terms) -> str:
     if fam == 2:
         extra = f"-rows{lik.N}-t{lr_terms}"
     h = hashlib.sha1(repr(shape).encode()).hexdigest()[:12]
-    return f"fam{fam}{extra}-R{len(specs)}-{h}-{name}-c5"
+    return f"fam{fam}{extra}-R{len(specs)}-{h}-{name}-c6"
 
 
 def measure(specs, lpc, wpb, shells=3, lr_terms=3, min_time=0.02, max_shells=12) -> float:
