@@ -141,7 +141,8 @@ typedef struct hipns_launch {
   int32_t family;
   int32_t lanes_per_chain;
   int32_t waves_per_block;  /* chain groups (one per wavefront) per workgroup; LinReg multiplies each row
-                             * tile against all of them */
+                             * tile against all of them, and regroups the chains of a launch that leaves CUs
+                             * idle */
   int32_t gmm_K;
   int32_t lr_ndata;         /* LinReg: data rows padded to a multiple of 32 */
   int32_t max_steps;        /* step cap per slice (safety bound on the shrink loop) */
@@ -226,8 +227,8 @@ size_t hipns_collect_shell_workspace_size(int32_t R, const hipns_run_desc_t* run
  * ------------------------------------------------------------------- */
 
 /* compute_evidence_stats (internals/shrinkage_statistics.py:131-157): the
- * _update_evidence_calc_op recurrence (:43-94) over M samples as a single-pass
- * log-space scan.  per_sample_dev: [8][M] SoA (field-major, may be NULL);
+ * _update_evidence_calc_op recurrence (:43-94) over M samples as a scan of its
+ * step maps.  per_sample_dev: [8][M] SoA (field-major, may be NULL);
  * final_dev: [8].  stop_idx < 0 => static scan, else outputs past stop_idx hold
  * the initial state (cumulative_op_dynamic, internals/cumulative_ops.py:82-130). */
 int hipns_evidence_scan(const double* log_L_dev, const double* num_live_points_dev, int64_t M, int64_t stop_idx,

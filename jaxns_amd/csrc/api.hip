@@ -186,7 +186,8 @@ int sampler_launch(int mode, const hipns_launch_t* L, const hipns::SampleArgs& A
       for (int r = 0; h > 1 && r < R; ++r) {
         const hipns_run_desc_t& d = runs[r];
         const int64_t clusters = (d.shell + groups * cw - 1) / (groups * cw);
-        if (clusters * (int64_t)hipns::lr_cluster_bytes(groups, cw) > (int64_t)d.N * dps * (int64_t)sizeof(float)) h = 1;
+        const int64_t scratch = clusters * (int64_t)hipns::lr_cluster_bytes(groups, cw);
+        if (scratch > (int64_t)d.N * dps * (int64_t)sizeof(float)) h = 1;
       }
       A.lr_split = h;
     }
@@ -777,14 +778,16 @@ int hipns_linreg_stats(const float* U_dev, int64_t B, double* logL_dev, double* 
   if (D < 1 || D > bufs->dps) return fail(HIPNS_EINVAL, "D outside [1, dps]");
   const int lpc = bufs->dps > 64 ? 4 : launch->lanes_per_chain;
   if ((rc = check_panels(launch, D, lpc))) return rc;
-  const size_t lds = hipns::sampler_lds_floats(HIPNS_FAM_LINREG, bufs->dps, D, 1, lpc, 1, launch->lr_ndata, 2) * sizeof(float);
+  const size_t lds =
+      hipns::sampler_lds_floats(HIPNS_FAM_LINREG, bufs->dps, D, 1, lpc, 1, launch->lr_ndata, 2) * sizeof(float);
   // Bound by the latency of the data rows where the workgroups leave SIMDs idle: as long as one wavefront each
   // would, the most wavefronts share a workgroup's rows (in the same fixed blocks, so the sums are the same).
   // 4096 x 16: 1 000 points 41.7 -> 14.2 us, 16 000 points 46.1 -> 25.6, 32 000 points (one wavefront per SIMD)
   // 48.8 -> 45.7; beyond that there is nothing to gain (64 000 points 87.5 and 88.4 us), and few rows lose
   // to the barriers (300 x 5, 200 000 points: 31 and 50 us).
   const int cw = HIPNS_WAVE / lpc;
-  const int waves = (B + cw - 1) / cw <= 4 * num_cus() ? hipns::lr_max_waves(hipns::sampler_nj(D, lpc == 2 ? 2 : 4)) : 1;
+  const int most = hipns::lr_max_waves(hipns::sampler_nj(D, lpc == 2 ? 2 : 4));
+  const int waves = (B + cw - 1) / cw <= 4 * num_cus() ? most : 1;
   hipError_t e = hipns::launch_linreg_stats(U_dev, B, logL_dev, rss_dev, yr_dev, runs_dev, *bufs, lpc, D, waves, lds,
                                             as_stream(stream), linreg_view(bufs, launch));
   if (e != hipSuccess) return hip_fail(e, "linreg stats launch");

@@ -544,7 +544,9 @@ __device__ __forceinline__ EvState evmap_apply(const EvMap& f, const EvState& s)
 __device__ __forceinline__ Sc ev_X2(const EvState& s) { return sc_mul(sc_of(s.X), sc_of(s.Q)); }
 __device__ __forceinline__ Sc ev_ZX(const EvState& s) { return sc_mul(sc_of(s.X), s.Y); }
 
-__device__ __forceinline__ Sc sc_shfl_down(const Sc& x, int o) { return {__shfl_down(x.m, o, 64), __shfl_down(x.e, o, 64)}; }
+__device__ __forceinline__ Sc sc_shfl_down(const Sc& x, int o) {
+  return {__shfl_down(x.m, o, 64), __shfl_down(x.e, o, 64)};
+}
 __device__ __forceinline__ Sc sc_shfl_up(const Sc& x, int o) { return {__shfl_up(x.m, o, 64), __shfl_up(x.e, o, 64)}; }
 __device__ __forceinline__ Scd sc_shfl_down(const Scd& x, int o) {
   return {__shfl_down(x.m, o, 64), __shfl_down(x.lo, o, 64), __shfl_down(x.e, o, 64)};

@@ -149,7 +149,8 @@ inline size_t sampler_lds_floats(int fam, int dps, int D, int K, int lpc, int G,
   if (fam == HIPNS_FAM_LINREG) {
     const size_t NG = (size_t)sampler_nj(D, lpc) / 8;
     const size_t CW = (size_t)(64 / lpc);
-    return (size_t)4 * dps + 4 + (size_t)G * NG * 3 * 64 * 4 + (size_t)sums * G * lr_row_blocks((int)(npad / CW), lpc, (int)NG * 8) * CW * 2;
+    const size_t blocks = (size_t)lr_row_blocks((int)(npad / CW), lpc, (int)NG * 8);
+    return (size_t)4 * dps + 4 + (size_t)G * NG * 3 * 64 * 4 + (size_t)sums * G * blocks * CW * 2;
   }
   if (fam == HIPNS_FAM_MVN) {
     const int nj = sampler_nj(D, lpc);
@@ -200,7 +201,8 @@ hipError_t launch_loglik(const float* U, int64_t B, double* out, const hipns_run
 }  // namespace hipns
 
 namespace hipns {
-__global__ void k_lr_clear(const hipns_run_desc_t* runs, const hipns_run_state_t* states, hipns_buffers_t B, int G, int cw);
+__global__ void k_lr_clear(const hipns_run_desc_t* runs, const hipns_run_state_t* states, hipns_buffers_t B, int G,
+                           int cw);
 hipError_t launch_sampler_slice(const SampleArgs& A, int R, int max_chains, const hipns_launch_t& L, int dmax,
                                 size_t lds_bytes, hipStream_t s);
 // wavefronts of a kernel that a SIMD holds by its registers (512 a lane, given in eights; at most 8)

@@ -1148,7 +1148,10 @@ __device__ __forceinline__ void uniform_point(float (&up)[NJ], int chain, uint32
 // 512 runs.  The 16-slot gradient instances are held to two wavefronts.)
 template <int LPC, int NJ, int FAM, int MODE, int KT>
 __global__ void __launch_bounds__(FAM == HIPNS_FAM_LINREG ? HIPNS_WAVE * lr_max_waves(NJ) : 256,
-                                  FAM != HIPNS_FAM_GMM ? 1 : MODE == MODE_GSLICE ? (NJ == 16 ? 2 : 1) : NJ == 8 && KT <= 6 ? 4 : 1)
+                                  FAM != HIPNS_FAM_GMM     ? 1
+                                  : MODE == MODE_GSLICE    ? (NJ == 16 ? 2 : 1)
+                                  : (NJ == 8 && KT <= 6)   ? 4
+                                                           : 1)
     k_sample(SampleArgs A) {
   constexpr int CW = HIPNS_WAVE / LPC;
   // the regression family multiplies the data rows against every chain group of the workgroup

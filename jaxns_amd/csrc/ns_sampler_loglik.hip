@@ -47,8 +47,9 @@ static unsigned loglik_blocks(int64_t groups, int wpb, int waves_per_simd, size_
 // idle ones: 33000 x 60, 20 000 points in FP32, 1.14 against 2.01 ms)
 template <int LPC, int NJ, int FAM, int KT>
 __global__ void __launch_bounds__(256)
-    __attribute__((amdgpu_waves_per_eu(1, FAM == HIPNS_FAM_LINREG && NJ == 32 ? 1 : 8))) k_loglik(const float* U, int64_t B, double* out, const hipns_run_desc_t* runs,
-                                                hipns_buffers_t Bf, int K, LinRegLds lrd) {
+    __attribute__((amdgpu_waves_per_eu(1, FAM == HIPNS_FAM_LINREG && NJ == 32 ? 1 : 8)))
+    k_loglik(const float* U, int64_t B, double* out, const hipns_run_desc_t* runs, hipns_buffers_t Bf, int K,
+             LinRegLds lrd) {
   constexpr int CW = HIPNS_WAVE / LPC;
   extern __shared__ float lds[];
   const hipns_run_desc_t run = runs[0];
@@ -106,9 +107,9 @@ __global__ void __launch_bounds__(256)
 // (the 32-slot mixture instances at two wavefronts per SIMD, some spilling up to 128 B a lane: D=100, 400 000
 // rows 330 -> 157 us with 6 component rows, 385 -> 267 with 8)
 template <int LPC, int NJ, int FAM, int KT>
-__global__ void __launch_bounds__(256, FAM == HIPNS_FAM_GMM && NJ == 32 ? 2 : 1) k_loglik_grad(const float* U, int64_t B, double* out, float* grad,
-                                                     const hipns_run_desc_t* runs, hipns_buffers_t Bf, int K,
-                                                     int gscr_off) {
+__global__ void __launch_bounds__(256, FAM == HIPNS_FAM_GMM && NJ == 32 ? 2 : 1)
+    k_loglik_grad(const float* U, int64_t B, double* out, float* grad, const hipns_run_desc_t* runs,
+                  hipns_buffers_t Bf, int K, int gscr_off) {
   constexpr int CW = HIPNS_WAVE / LPC;
   extern __shared__ float lds[];
   const hipns_run_desc_t run = runs[0];
@@ -172,8 +173,10 @@ static hipError_t launch_loglik_grad_one(const float* U, int64_t B, double* out,
                                          int gscr_off, size_t lds, const LoglikChip& chip, hipStream_t s) {
   if constexpr (FAM == HIPNS_FAM_GMM) {
     switch (gmm_rows(K)) {
-      case 4: return launch_loglik_grad_rows<LPC, NJ, FAM, 4>(U, B, out, grad, runs, Bf, K, wpb, gscr_off, lds, chip, s);
-      case 6: return launch_loglik_grad_rows<LPC, NJ, FAM, 6>(U, B, out, grad, runs, Bf, K, wpb, gscr_off, lds, chip, s);
+      case 4:
+        return launch_loglik_grad_rows<LPC, NJ, FAM, 4>(U, B, out, grad, runs, Bf, K, wpb, gscr_off, lds, chip, s);
+      case 6:
+        return launch_loglik_grad_rows<LPC, NJ, FAM, 6>(U, B, out, grad, runs, Bf, K, wpb, gscr_off, lds, chip, s);
       default: break;
     }
   }
@@ -186,20 +189,19 @@ static hipError_t launch_loglik_grad_fam(const float* U, int64_t B, double* out,
                                          const hipns_run_desc_t* runs, const hipns_buffers_t& Bf, int K, int lpc,
                                          int wpb, int dmax, int gscr_off, size_t lds, const LoglikChip& chip,
                                          hipStream_t s) {
+  auto call = [&](auto launch) { return launch(U, B, out, grad, runs, Bf, K, wpb, gscr_off, lds, chip, s); };
   if constexpr (FAM == HIPNS_FAM_GMM) {
-    if (lpc == 8 && dmax <= 128) {
-      if (dmax <= 64) return launch_loglik_grad_one<8, 8, FAM>(U, B, out, grad, runs, Bf, K, wpb, gscr_off, lds, chip, s);
-      return launch_loglik_grad_one<8, 16, FAM>(U, B, out, grad, runs, Bf, K, wpb, gscr_off, lds, chip, s);
-    }
+    if (lpc == 8 && dmax <= 128)
+      return call(dmax <= 64 ? launch_loglik_grad_one<8, 8, FAM> : launch_loglik_grad_one<8, 16, FAM>);
   }
   if (lpc == 4 || lpc == 8 || dmax > 64) {
-    if (dmax <= 32) return launch_loglik_grad_one<4, 8, FAM>(U, B, out, grad, runs, Bf, K, wpb, gscr_off, lds, chip, s);
-    if (dmax <= 64) return launch_loglik_grad_one<4, 16, FAM>(U, B, out, grad, runs, Bf, K, wpb, gscr_off, lds, chip, s);
-    return launch_loglik_grad_one<4, 32, FAM>(U, B, out, grad, runs, Bf, K, wpb, gscr_off, lds, chip, s);
+    if (dmax <= 32) return call(launch_loglik_grad_one<4, 8, FAM>);
+    if (dmax <= 64) return call(launch_loglik_grad_one<4, 16, FAM>);
+    return call(launch_loglik_grad_one<4, 32, FAM>);
   }
-  if (dmax <= 16) return launch_loglik_grad_one<2, 8, FAM>(U, B, out, grad, runs, Bf, K, wpb, gscr_off, lds, chip, s);
-  if (dmax <= 32) return launch_loglik_grad_one<2, 16, FAM>(U, B, out, grad, runs, Bf, K, wpb, gscr_off, lds, chip, s);
-  return launch_loglik_grad_one<2, 32, FAM>(U, B, out, grad, runs, Bf, K, wpb, gscr_off, lds, chip, s);
+  if (dmax <= 16) return call(launch_loglik_grad_one<2, 8, FAM>);
+  if (dmax <= 32) return call(launch_loglik_grad_one<2, 16, FAM>);
+  return call(launch_loglik_grad_one<2, 32, FAM>);
 }
 
 template <int LPC, int NJ, int FAM, int KT>
@@ -210,8 +212,9 @@ static hipError_t launch_loglik_rows(const float* U, int64_t B, double* out, con
   constexpr int CW = HIPNS_WAVE / LPC;
   const int64_t groups = (B + CW - 1) / CW;
   // (the regression family reads all its data rows per row group, beside which its parameters are nothing)
-  dim3 grid(FAM == HIPNS_FAM_LINREG ? (unsigned)((groups + wpb - 1) / wpb) : loglik_blocks(groups, wpb, waves, lds, chip));
-  dim3 block(wpb * HIPNS_WAVE);
+  const unsigned blocks =
+      FAM == HIPNS_FAM_LINREG ? (unsigned)((groups + wpb - 1) / wpb) : loglik_blocks(groups, wpb, waves, lds, chip);
+  dim3 grid(blocks), block(wpb * HIPNS_WAVE);
   hipLaunchKernelGGL((k_loglik<LPC, NJ, FAM, KT>), grid, block, lds, s, U, B, out, runs, Bf, K, lr);
   return hipGetLastError();
 }
@@ -256,8 +259,9 @@ static hipError_t launch_loglik_fam(const float* U, int64_t B, double* out, cons
 // per row of U (the host derives d logL / d(log sigma, log tau)).  A workgroup's first wavefront holds one
 // group of 64 / LPC points, all of its wavefronts share the data rows.
 template <int LPC, int NJ>
-__global__ void __launch_bounds__(HIPNS_WAVE * lr_max_waves(NJ)) k_linreg_stats(const float* U, int64_t B, double* logL, double* rss, double* yr,
-                                                     const hipns_run_desc_t* runs, hipns_buffers_t Bf, LinRegLds lrd) {
+__global__ void __launch_bounds__(HIPNS_WAVE * lr_max_waves(NJ))
+    k_linreg_stats(const float* U, int64_t B, double* logL, double* rss, double* yr, const hipns_run_desc_t* runs,
+                   hipns_buffers_t Bf, LinRegLds lrd) {
   constexpr int CW = HIPNS_WAVE / LPC;
   extern __shared__ float lds[];
   const hipns_run_desc_t run = runs[0];

@@ -157,26 +157,26 @@ __global__ void __launch_bounds__(1024) k_replace(const hipns_run_desc_t* runs, 
   }
   const int NS = N - S;
   auto merge = [&](const double* surv) {  // survivors, sorted
-  for (int i = tid; i < S; i += nt) {
-    double kk = keys[i];
-    int lo = 0, hi = NS;  // survivors strictly less than kk
-    while (lo < hi) {
-      int mid = (lo + hi) >> 1;
-      if (kless(surv[mid], kk)) lo = mid + 1;
-      else hi = mid;
+    for (int i = tid; i < S; i += nt) {
+      double kk = keys[i];
+      int lo = 0, hi = NS;  // survivors strictly less than kk
+      while (lo < hi) {
+        int mid = (lo + hi) >> 1;
+        if (kless(surv[mid], kk)) lo = mid + 1;
+        else hi = mid;
+      }
+      perm[i + lo] = idx[i];
     }
-    perm[i + lo] = idx[i];
-  }
-  for (int j = tid; j < NS; j += nt) {
-    double kk = surv[j];
-    int lo = 0, hi = S;  // new samples with key <= kk
-    while (lo < hi) {
-      int mid = (lo + hi) >> 1;
-      if (!kless(kk, keys[mid])) lo = mid + 1;
-      else hi = mid;
+    for (int j = tid; j < NS; j += nt) {
+      double kk = surv[j];
+      int lo = 0, hi = S;  // new samples with key <= kk
+      while (lo < hi) {
+        int mid = (lo + hi) >> 1;
+        if (!kless(kk, keys[mid])) lo = mid + 1;
+        else hi = mid;
+      }
+      perm[j + lo] = S + j;
     }
-    perm[j + lo] = S + j;
-  }
   };
   if (staged > 0)
     merge((const double*)(smem + staged));
@@ -313,7 +313,8 @@ __global__ void __launch_bounds__(1024) k_register(const hipns_run_desc_t* runs,
   // n = N, N-1, ..., 1 (sharded_static.py:292-299), wavefronts split in proportion to their lengths
   const int nw = blockDim.x / HIPNS_WAVE;
   const int w1 = max(1, min(nw - 1, (int)(((int64_t)nw * S + (S + N) / 2) / (S + N))));
-  two_sequence_maps(SeqSpec{disc, S, (double)N, 0, st->evidence_calc[0]}, SeqSpec{live, N, 0.0, N, disc[S - 1]}, w1, lds_maps);
+  two_sequence_maps(SeqSpec{disc, S, (double)N, 0, st->evidence_calc[0]}, SeqSpec{live, N, 0.0, N, disc[S - 1]}, w1,
+                    lds_maps);
   const EvMap A1 = lds_maps[0], A2 = lds_maps[w1];
   // live evaluation counts, new evaluation counts, plateau
   long long le = 0, ne = 0;
