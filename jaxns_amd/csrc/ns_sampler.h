@@ -117,6 +117,12 @@ __host__ __device__ constexpr int grad_rows(int nj, int lpc) {
 // of them; the gradient's product reads whole blocks of output rows
 __host__ __device__ constexpr int mvn_rows(int nj, int lpc, bool grad) { return grad ? grad_rows(nj, lpc) : nj * lpc; }
 
+// Whether an instance's likelihood masks the slots past the run's dimensions at every evaluation, as the
+// regression family's does; the others take them as 1/2 (their parameters are zero there).
+__host__ __device__ constexpr bool lik_masks(int fam, int lpc, int nj) {
+  return fam == HIPNS_FAM_LINREG || (fam == HIPNS_FAM_MVN && lpc == 4 && nj == 8);
+}
+
 // component rows of the mixture kernels' instances: 4, 6 or 8
 __host__ __device__ constexpr int gmm_rows(int K) { return K <= 4 ? 4 : (K <= 6 ? 6 : HIPNS_MAX_GMM_K); }
 

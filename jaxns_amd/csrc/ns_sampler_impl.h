@@ -679,9 +679,10 @@ __device__ __forceinline__ double lik_mvn(const float (&up)[NJ], int nj, int D, 
   const int h = l / CW;
   float z[NJ];
   prior_q<NJ>(up, z, tfm);  // finite on padding slots (u = 1/2), which meet zeros of W
-  if constexpr (LPC == 4 && NJ == 8) {
-    // not needed, but this instance's schedule is the better one with the masks (D=32, 1024 runs: 12.42
-    // against 12.24 G evaluations/s), the others' without (D=10: 19.2 against 18.7; D=20: 8.9 against 8.6)
+  if constexpr (lik_masks(HIPNS_FAM_MVN, LPC, NJ)) {
+    // this instance's schedule is the better one with the masks (D=32, 1024 runs: 12.42 against 12.24 G
+    // evaluations/s; with the seed rows masked instead, 0.6 % longer launches), the others' without (D=10: 19.2
+    // against 18.7; D=20: 8.9 against 8.6)
 #pragma unroll
     for (int j = 0; j < NJ; ++j)
       if (!(j < nj && owned_dim<LPC>(h, j) < D)) z[j] = 0.0f;
@@ -1210,7 +1211,7 @@ __global__ void __launch_bounds__(FAM == HIPNS_FAM_LINREG ? HIPNS_WAVE * lr_max_
   const int D = run.D;
   const int DPr = ((D + 8 * LPC - 1) / (8 * LPC)) * (8 * LPC);
   // (a run has at least 8 slots per lane; not folded where lik_mvn keeps its masks)
-  const int nj = (NJ == 8 && !(FAM == HIPNS_FAM_MVN && LPC == 4)) ? 8 : DPr / LPC;
+  const int nj = (NJ == 8 && !(FAM == HIPNS_FAM_MVN && lik_masks(FAM, LPC, NJ))) ? 8 : DPr / LPC;
 
   MvnLds mv;
   GmmLds gm;
@@ -1277,9 +1278,9 @@ __global__ void __launch_bounds__(FAM == HIPNS_FAM_LINREG ? HIPNS_WAVE * lr_max_
     const float* src = A.B.live_U[cur] + (run.live_off + idx) * (int64_t)dps;
 #pragma unroll
     for (int j = 0; j < NJ; ++j) {
-      // (0.5 past the run's dimensions, whatever the row holds there: the likelihoods do not mask)
+      // (0.5 past the run's dimensions, whatever the row holds there, unless the likelihood masks)
       int d = owned_dim<LPC>(h, j);
-      U0[j] = (alive && j < nj && d < D) ? src[d] : 0.5f;
+      U0[j] = (alive && j < nj && (lik_masks(FAM, LPC, NJ) || d < D)) ? src[d] : 0.5f;
     }
     logL0 = alive ? A.B.live_logL[cur][run.live_off + idx] : 0.0;
   } else {

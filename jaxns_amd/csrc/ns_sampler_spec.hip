@@ -75,9 +75,9 @@ __global__ void __launch_bounds__(FAM == HIPNS_FAM_LINREG ? HIPNS_WAVE * lr_max_
   const float* src = A.B.live_U[cur] + (run.live_off + idx) * (int64_t)dps;
 #pragma unroll
   for (int j = 0; j < NJ; ++j) {
-    // (0.5 past the run's dimensions, whatever the row holds there: the likelihoods do not mask)
+    // (0.5 past the run's dimensions, whatever the row holds there, unless the likelihood masks)
     const int d = owned_dim<LPC>(h, j);
-    U0[j] = (alive && j < nj && d < D) ? src[d] : 0.5f;
+    U0[j] = (alive && j < nj && (lik_masks(FAM, LPC, NJ) || d < D)) ? src[d] : 0.5f;
     nv[j] = 0.0f;
   }
   double logL0 = alive ? A.B.live_logL[cur][run.live_off + idx] : 0.0;
